@@ -687,7 +687,193 @@ __global__ void __launch_bounds__(NTHR) k_fused_step(FusedArgs a) {
     if (a.decode && tid < nb) a.tokens_out[b0 + tid] = sTok[tid];
 }
 
+// ------------------------------------------------------------------------------------------------
+// The decode kernel's GEMM phases as kernels over rows, for compress and forward launches with few tiles: a 64-row
+// workgroup (k_ffn, k_head_xq) keeps one CU busy for its whole K loop (fp32 feed-forward: 162 us) while most of the
+// others idle; 16-row workgroups take a quarter of that on four times as many CUs.  Same arithmetic per row, so the
+// same values (every output accumulates its K steps in ascending order).  BLOCK: 512 threads, one workgroup per CU.
+
+// x <- x + FF2(GELU(FF1(LN2(out_proj(y))))) for 16 rows of tile blockIdx.y.
+template <int NT>
+__global__ void __launch_bounds__(512) k_ffn16(FfnTiles a) {
+    constexpr int NWAVE = 8, RPW = ROWS / NWAVE, FPW_B = NT == 1 ? 8 : 4, D_B = 3, FPW_S = 2, D_S = 6;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[SZ_A + SZ_X];
+    uint16_t* sAh = reinterpret_cast<uint16_t*>(lds);
+    uint16_t* sAl = sAh + ROWS * LA;
+    float* sX = reinterpret_cast<float*>(lds + SZ_A);
+    uint16_t* sHh = reinterpret_cast<uint16_t*>(lds + SZ_A);
+    uint16_t* sHl = sHh + ROWS * LH;
+    const FfnTile& w = a.t[blockIdx.y];
+    const int64_t m0 = (int64_t)blockIdx.x * ROWS;
+    if (m0 >= w.M) return;
+    const int nb = (int)(w.M - m0 < ROWS ? w.M - m0 : ROWS);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = NT == 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
+    const int m_of = 4 * (lane >> 4), n_of = lane & 15;
+    const int rot64 = (int)(blockIdx.x & 7) * 8, rot16 = (int)(blockIdx.x & 15);
+    // y rows (rows past the tile's end read 0)
+    if constexpr (NT == 1) {
+        const __amdgpu_buffer_rsrc_t ry = buf_rsrc(reinterpret_cast<const float*>(w.yh) + m0 * FDI, (uint32_t)nb * FDI * 4);
+#pragma unroll
+        for (int e = 0; e < ROWS * FDI / 4 / 512; ++e) {
+            const int i = e * 512 + tid, r = i / (FDI / 4), k = (i % (FDI / 4)) * 4;
+            *reinterpret_cast<u32x4*>(reinterpret_cast<float*>(sAh) + r * ld32(LA) + k) = buf_ld16(ry, (uint32_t)(r * FDI + k) * 4);
+        }
+    } else {
+        const __amdgpu_buffer_rsrc_t rh = buf_rsrc(w.yh + m0 * FDI, (uint32_t)nb * FDI * 2);
+        const __amdgpu_buffer_rsrc_t rl = buf_rsrc(w.yl + m0 * FDI, (uint32_t)nb * FDI * 2);
+#pragma unroll
+        for (int e = 0; e < ROWS * FDI / 8 / 512; ++e) {
+            const int i = e * 512 + tid, r = i / (FDI / 8), k = (i % (FDI / 8)) * 8;
+            *reinterpret_cast<u32x4*>(sAh + r * LA + k) = buf_ld16(rh, (uint32_t)(r * FDI + k) * 2);
+            *reinterpret_cast<u32x4*>(sAl + r * LA + k) = buf_ld16(rl, (uint32_t)(r * FDI + k) * 2);
+        }
+    }
+    const float4 lnw = ldg_f4(G(w.ln_w) + 4 * lane), lnb = ldg_f4(G(w.ln_b) + 4 * lane);
+    __syncthreads();
+    {
+        floatx4 acc[FPW_S];
+        float bias_j[FPW_S];
+#pragma unroll
+        for (int j = 0; j < FPW_S; ++j) bias_j[j] = G(w.out_b)[16 * frag_of<NWAVE>(0, wave, j, FD / 16, rot16) + n_of];
+        mgemm<NT, NWAVE, FPW_S, FDI, D_S, false>(sAh, sAl, LA, w.out_p, 0, FD / 16, wave, lane, rot16, acc);
+#pragma unroll
+        for (int j = 0; j < FPW_S; ++j) {
+            const int n = 16 * frag_of<NWAVE>(0, wave, j, FD / 16, rot16) + n_of;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sX[(m_of + r) * LRES + n] = epi_value<EPI_BIAS>(acc[j][r], bias_j[j]);
+        }
+    }
+    __syncthreads();
+    ln_rows<NT, RPW>(sX, lnw, lnb, sAh, sAl, wave, lane);
+    __syncthreads();
+#pragma unroll 1
+    for (int f0 = 0; f0 < 4 * FD / 16; f0 += FPW_B * NWAVE) {
+        floatx4 acc[FPW_B];
+        float bias_j[FPW_B];
+#pragma unroll
+        for (int j = 0; j < FPW_B; ++j) bias_j[j] = G(w.ff1_b)[16 * frag_of<NWAVE>(f0, wave, j, 4 * FD / 16, rot64) + n_of];
+        mgemm<NT, NWAVE, FPW_B, FD, D_B, false, 2>(sAh, sAl, LA, w.ff1_p, f0, 4 * FD / 16, wave, lane, rot64, acc);
+#pragma unroll
+        for (int j = 0; j < FPW_B; ++j) {
+            const int n = 16 * frag_of<NWAVE>(f0, wave, j, 4 * FD / 16, rot64) + n_of;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) store_op<NT, LH>(sHh, m_of + r, n, epi_value<EPI_GELU>(acc[j][r], bias_j[j]));
+        }
+    }
+    __syncthreads();
+    {
+        const __amdgpu_buffer_rsrc_t rx = buf_rsrc(w.x + m0 * FD, (uint32_t)nb * FD * 4);
+        floatx4 acc[FPW_S];
+        float bias_j[FPW_S], res[FPW_S][4];
+#pragma unroll
+        for (int j = 0; j < FPW_S; ++j) {
+            const int n = 16 * frag_of<NWAVE>(0, wave, j, FD / 16, rot16) + n_of;
+            bias_j[j] = G(w.ff2_b)[n];
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                res[j][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, (uint32_t)((m_of + r) * FD + n) * 4, 0, 0));
+        }
+        mgemm<NT, NWAVE, FPW_S, 4 * FD, D_S, false>(sHh, sHl, LH, w.ff2_p, 0, FD / 16, wave, lane, rot16, acc);
+#pragma unroll
+        for (int j = 0; j < FPW_S; ++j) {
+            const int n = 16 * frag_of<NWAVE>(0, wave, j, FD / 16, rot16) + n_of;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                __builtin_amdgcn_raw_buffer_store_b32(
+                    __builtin_bit_cast(uint32_t, res[j][r] + epi_value<EPI_RESID>(acc[j][r], bias_j[j])), rx,
+                    (uint32_t)((m_of + r) * FD + n) * 4, 0, 0);
+        }
+    }
+}
+
+// Head of 16 rows, then each row's coder interval (wave w: rows 2 w, 2 w + 1) or its logits.
+template <int NT>
+__global__ void __launch_bounds__(512) k_head16(HeadRows a) {
+    constexpr int NWAVE = 8, RPW = ROWS / NWAVE, FPW_S = 2, D_S = 6;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * SZ_A];
+    uint16_t* sAh = reinterpret_cast<uint16_t*>(lds);
+    uint16_t* sAl = sAh + ROWS * LA;
+    uint16_t* sGh = reinterpret_cast<uint16_t*>(lds + SZ_A);
+    uint16_t* sGl = sGh + ROWS * LH1;
+    float* sLog = reinterpret_cast<float*>(lds);  // after head1, in the operand's place
+    const int64_t m0 = (int64_t)blockIdx.x * ROWS;
+    const int nb = (int)(a.M - m0 < ROWS ? a.M - m0 : ROWS);
+    const int V = a.V;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = NT == 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
+    const int m_of = 4 * (lane >> 4), n_of = lane & 15;
+    const int rot16 = (int)(blockIdx.x & 15);
+#pragma unroll
+    for (int e = 0; e < ROWS * FD / 512; ++e) {
+        const int i = e * 512 + tid, r = i / FD, c = i % FD;
+        store_op<NT, LA>(sAh, r, c, G(a.x)[(m0 + (r < nb ? r : nb - 1)) * FD + c]);
+    }
+    __syncthreads();
+    {
+        floatx4 acc[FPW_S];
+        mgemm<NT, NWAVE, FPW_S, FD, D_S, false>(sAh, sAl, LA, a.h1_p, 0, FD / 16, wave, lane, rot16, acc);
+#pragma unroll
+        for (int j = 0; j < FPW_S; ++j) {
+            const int n = 16 * frag_of<NWAVE>(0, wave, j, FD / 16, rot16) + n_of;
+            const float bias = G(a.h1_b)[n];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) store_op<NT, LH1>(sGh, m_of + r, n, epi_value<EPI_RELU>(acc[j][r], bias));
+        }
+    }
+    __syncthreads();
+    {
+        floatx4 acc[FPW_S];
+        mgemm<NT, NWAVE, FPW_S, FD, D_S>(sGh, sGl, LH1, a.h2_p, 0, V / 16, wave, lane, 0, acc);
+#pragma unroll
+        for (int j = 0; j < FPW_S; ++j) {
+            const int f = wave + NWAVE * j;
+            if (f < V / 16) {
+                const int n = 16 * f + n_of;
+                const float bias = G(a.h2_b)[n];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sLog[(m_of + r) * LRES + n] = epi_value<EPI_BIAS>(acc[j][r], bias);
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < RPW; ++q) {
+        const int r = RPW * wave + q;
+        if (r >= nb) continue;
+        const int64_t m = m0 + r, b = m / a.Tc;
+        const int p = a.t0 + (int)(m - b * a.Tc);
+        if (a.logits) {
+            float* dst = a.logits + (b * a.len + p) * V;
+            for (int c = lane; c < V; c += 64) dst[c] = sLog[r * LRES + c];
+            continue;
+        }
+        uint2 v = make_uint2(LF_SKIP, 0u);
+        if (p + 1 < a.lens[b]) {
+            const int s = a.bytes[b * a.stride + p + 1];
+            if (s < V) v = xq_interval(logits_row4(sLog + r * LRES, V, lane), V, lane, s);
+        }
+        if (lane == 0) a.lf[m] = v;
+    }
+}
+
 }  // namespace
+
+hipError_t launch_ffn16(const FfnTiles& a, int tiles, int64_t max_rows, int nt, hipStream_t s) {
+    const dim3 grid((unsigned)((max_rows + ROWS - 1) / ROWS), (unsigned)tiles);
+    if (nt == 3) hipLaunchKernelGGL((k_ffn16<3>), grid, dim3(512), 0, s, a);
+    else if (nt == 2) hipLaunchKernelGGL((k_ffn16<2>), grid, dim3(512), 0, s, a);
+    else hipLaunchKernelGGL((k_ffn16<1>), grid, dim3(512), 0, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_head16(const HeadRows& a, int nt, hipStream_t s) {
+    const dim3 grid((unsigned)((a.M + ROWS - 1) / ROWS));
+    if (nt == 3) hipLaunchKernelGGL((k_head16<3>), grid, dim3(512), 0, s, a);
+    else if (nt == 2) hipLaunchKernelGGL((k_head16<2>), grid, dim3(512), 0, s, a);
+    else hipLaunchKernelGGL((k_head16<1>), grid, dim3(512), 0, s, a);
+    return hipGetLastError();
+}
 
 bool fused_step_supported(int d_model, int d_state, int dt_rank, int d_conv, int vocab) {
     return d_model == FD && d_state == FNS && dt_rank == FR && d_conv == 4 && vocab % 16 == 0 && vocab <= 256;

@@ -577,10 +577,21 @@ struct EmbedIn {
     const uint8_t* bytes = nullptr;  // the group's bytes [lanes][stride]
     int64_t stride = 0;
     const int32_t* lens = nullptr;   // the group's chunk lengths
+    const int32_t* tokens = nullptr; // or the model inputs themselves [lanes][stride] (general kernels only)
     const float* emb = nullptr;      // [V][d]
     float* xout = nullptr;           // x, where the gathered rows are written for the residual
     int t0 = 0, V = 0;               // the tile's first position; vocab
 };
+
+// The model input of lane b at position t0 + t (t < Tc, else position t0 + Tc - 1 again), from either source.
+__device__ __forceinline__ int embed_token(const EmbedIn& e, int64_t b, int t, int Tc) {
+    t = t < Tc ? t : Tc - 1;
+    if (e.tokens) {
+        const int tok = e.tokens[b * e.stride + e.t0 + t];
+        return tok < 0 ? 0 : (tok >= e.V ? e.V - 1 : tok);
+    }
+    return byte_token(e.bytes, e.stride, e.lens, b, e.t0 + t, e.V);
+}
 
 __global__ void __launch_bounds__(256) k_embed_tokens(const int32_t* __restrict__ tokens, int64_t tok_stride,
                                                      int t0, int Tc, int64_t rows, const float* __restrict__ emb,
@@ -828,12 +839,12 @@ __device__ __forceinline__ int h_off(int r, int k) { return r * HC + (((k >> 3) 
 // stays on chip (fp32 in the operand buffer) for LN2, instead of a round trip through HBM.  Wave w owns
 // out_proj outputs 32 w .. + 31 of all 64 rows; its 32 W_out blocks stream through a 4-slot ring.
 template <int NT, bool OUTP>
-__global__ void __launch_bounds__(512, 4) k_ffn(const float* __restrict__ mm, const float* __restrict__ ln_w,
-                                                const float* __restrict__ ln_b, const uint16_t* __restrict__ W1p,
-                                                const float* __restrict__ b1, const uint16_t* __restrict__ W2p,
-                                                const float* __restrict__ b2, float* __restrict__ x, int64_t M,
-                                                const uint16_t* __restrict__ yh, const uint16_t* __restrict__ yl,
-                                                const uint16_t* __restrict__ Wop, const float* __restrict__ bo) {
+__device__ __forceinline__ void ffn_rows(const float* __restrict__ mm, const float* __restrict__ ln_w,
+                                         const float* __restrict__ ln_b, const uint16_t* __restrict__ W1p,
+                                         const float* __restrict__ b1, const uint16_t* __restrict__ W2p,
+                                         const float* __restrict__ b2, float* __restrict__ x, int64_t M,
+                                         const uint16_t* __restrict__ yh, const uint16_t* __restrict__ yl,
+                                         const uint16_t* __restrict__ Wop, const float* __restrict__ bo) {
     using namespace ffn;
     __shared__ __attribute__((aligned(16))) uint16_t sA[2][BM * D];
     __shared__ __attribute__((aligned(16))) uint16_t sH[2][BM * HC];
@@ -1082,6 +1093,24 @@ __global__ void __launch_bounds__(512, 4) k_ffn(const float* __restrict__ mm, co
     }
 }
 
+template <int NT, bool OUTP>
+__global__ void __launch_bounds__(512, 4) k_ffn(const float* __restrict__ mm, const float* __restrict__ ln_w,
+                                                const float* __restrict__ ln_b, const uint16_t* __restrict__ W1p,
+                                                const float* __restrict__ b1, const uint16_t* __restrict__ W2p,
+                                                const float* __restrict__ b2, float* __restrict__ x, int64_t M,
+                                                const uint16_t* __restrict__ yh, const uint16_t* __restrict__ yl,
+                                                const uint16_t* __restrict__ Wop, const float* __restrict__ bo) {
+    ffn_rows<NT, OUTP>(mm, ln_w, ln_b, W1p, b1, W2p, b2, x, M, yh, yl, Wop, bo);
+}
+
+// The same over several tiles in one launch: blockIdx.y picks the tile (rows past a tile's M read 0, store nothing).
+template <int NT>
+__global__ void __launch_bounds__(512, 4) k_ffn_gen(FfnTiles a) {
+    const FfnTile& t = a.t[blockIdx.y];
+    if ((int64_t)blockIdx.x * ffn::BM >= t.M) return;
+    ffn_rows<NT, true>(nullptr, t.ln_w, t.ln_b, t.ff1_p, t.ff1_b, t.ff2_p, t.ff2_b, t.x, t.M, t.yh, t.yl, t.out_p, t.out_b);
+}
+
 // ================================================================================================
 // The same feed-forward half for d_model 512 (d_ff 2048; configs[4]'s shape):
 //   x <- x + FF2(GELU(FF1(LN2(mm))))
@@ -1123,12 +1152,12 @@ constexpr int ffn_groups() { return NT == 2 ? 2 : 1; }
 // mfma_split_step (as the out_proj GEMM does); mm then stays on chip (fp32 in the operand buffer) for LN2.
 // Wave w owns out_proj outputs 64 w .. + 63 of all 64 rows; its W_out blocks stream through an 8-slot ring.
 template <int NT, bool OUTP>
-__global__ void __launch_bounds__(512, 2) k_ffn512(const float* __restrict__ mm, const float* __restrict__ ln_w,
-                                                   const float* __restrict__ ln_b, const uint16_t* __restrict__ W1p,
-                                                   const float* __restrict__ b1, const uint16_t* __restrict__ W2p,
-                                                   const float* __restrict__ b2, float* __restrict__ x, int64_t M,
-                                                   const uint16_t* __restrict__ yh, const uint16_t* __restrict__ yl,
-                                                   const uint16_t* __restrict__ Wop, const float* __restrict__ bo) {
+__device__ __forceinline__ void ffn512_rows(const float* __restrict__ mm, const float* __restrict__ ln_w,
+                                            const float* __restrict__ ln_b, const uint16_t* __restrict__ W1p,
+                                            const float* __restrict__ b1, const uint16_t* __restrict__ W2p,
+                                            const float* __restrict__ b2, float* __restrict__ x, int64_t M,
+                                            const uint16_t* __restrict__ yh, const uint16_t* __restrict__ yl,
+                                            const uint16_t* __restrict__ Wop, const float* __restrict__ bo) {
     using namespace ffn5;
     __shared__ __attribute__((aligned(16))) uint16_t sA[2][BM * D];
     __shared__ __attribute__((aligned(16))) uint16_t sH[2][BM * HC * ffn_groups<NT>()];
@@ -1392,6 +1421,25 @@ __global__ void __launch_bounds__(512, 2) k_ffn512(const float* __restrict__ mm,
     }
 }
 
+template <int NT, bool OUTP>
+__global__ void __launch_bounds__(512, 2) k_ffn512(const float* __restrict__ mm, const float* __restrict__ ln_w,
+                                                   const float* __restrict__ ln_b, const uint16_t* __restrict__ W1p,
+                                                   const float* __restrict__ b1, const uint16_t* __restrict__ W2p,
+                                                   const float* __restrict__ b2, float* __restrict__ x, int64_t M,
+                                                   const uint16_t* __restrict__ yh, const uint16_t* __restrict__ yl,
+                                                   const uint16_t* __restrict__ Wop, const float* __restrict__ bo) {
+    ffn512_rows<NT, OUTP>(mm, ln_w, ln_b, W1p, b1, W2p, b2, x, M, yh, yl, Wop, bo);
+}
+
+// The same over several tiles in one launch, as k_ffn_gen.
+template <int NT>
+__global__ void __launch_bounds__(512, 2) k_ffn512_gen(FfnTiles a) {
+    const FfnTile& t = a.t[blockIdx.y];
+    if ((int64_t)blockIdx.x * ffn5::BM >= t.M) return;
+    ffn512_rows<NT, true>(nullptr, t.ln_w, t.ln_b, t.ff1_p, t.ff1_b, t.ff2_p, t.ff2_b, t.x, t.M, t.yh, t.yl, t.out_p,
+                          t.out_b);
+}
+
 // ================================================================================================
 // Input half of the mixer in one kernel (split modes, d_model 256, compress tiles of 64 positions):
 //   LN1 -> in_proj (+bias) -> z to HBM; x -> causal conv + SiLU over the 64 positions -> xs to HBM ->
@@ -1412,14 +1460,33 @@ __device__ __forceinline__ int x_off(int r, int k) { return r * CH + (((k >> 3) 
 __device__ __forceinline__ int sx_off(int r, int c) { return r * CH + ((((c >> 2) ^ r) & 15) << 2) + (c & 3); }
 }  // namespace mixin
 
-template <int NT, bool EMB>
-__global__ void __launch_bounds__(256, 2) k_mixin(const float* __restrict__ x, const float* __restrict__ ln_w,
-                                                 const float* __restrict__ ln_b, const uint16_t* __restrict__ Wip,
-                                                 const float* __restrict__ bin, const float* __restrict__ conv_w,
-                                                 const float* __restrict__ conv_b, const uint16_t* __restrict__ Wxp,
-                                                 float* __restrict__ xz, float* __restrict__ xs,
-                                                 float* __restrict__ dbc, float* __restrict__ hist, int p0m3,
-                                                 EmbedIn e) {
+// One tile of the general form (below): its buffers, its layer's weights, its first position mod 3, its positions.
+struct MixinTile {
+    const float *x, *ln_w, *ln_b, *in_b, *conv_w, *conv_b;
+    const uint16_t *in_p, *x_p;
+    float *xz, *xs, *dbc, *hist;
+    int p0m3, Tc;
+};
+struct MixinTiles {
+    MixinTile t[PIPE_MAX];
+    EmbedIn e;       // the embedding source of tile `emb` (its layer is the model's first), if any
+    int emb;         // -1: no tile gathers embedding rows
+    int per;         // in_proj chunks per workgroup (blockIdx.z takes chunks per * z ..)
+};
+
+// GEN: the general form, for tiles of Tc <= 64 positions and for launches with few tiles.  Rows past Tc repeat the
+// tile's last row and are not stored.  A workgroup may own only the in_proj chunks [c0, c1) of its tile: the x
+// chunks' channels are independent of each other up to x_proj, whose partial of each 64-channel K block is then
+// stored (part: [rows][8][48], row stride ldp) for the scan to fold in the same order.  Workgroup `first` also
+// copies the embedding rows out.
+template <int NT, bool EMB, bool GEN>
+__device__ __forceinline__ void mixin_tile(const float* __restrict__ x, const float* __restrict__ ln_w,
+                                           const float* __restrict__ ln_b, const uint16_t* __restrict__ Wip,
+                                           const float* __restrict__ bin, const float* __restrict__ conv_w,
+                                           const float* __restrict__ conv_b, const uint16_t* __restrict__ Wxp,
+                                           float* __restrict__ xz, float* __restrict__ xs,
+                                           float* __restrict__ dbc, float* __restrict__ hist, int p0m3, EmbedIn e,
+                                           bool gather, int tc, int c0, int c1) {
     using namespace mixin;
     constexpr int BLK = two_part_blocks<NT>() ? 1024 : 512;
     __shared__ __attribute__((aligned(16))) uint16_t sA[2][BM * D];  // LN1 output (hi, lo)
@@ -1428,18 +1495,26 @@ __global__ void __launch_bounds__(256, 2) k_mixin(const float* __restrict__ x, c
     uint16_t* sXl = sXh + BM * CH;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t b = blockIdx.x, m0 = b * BM;
+    const int Tc = GEN ? tc : BM;
+    const int64_t b = blockIdx.x, m0 = b * Tc;
+    const bool emb = GEN ? gather : EMB;  // compile-time without GEN
+    const bool split = GEN && c1 - c0 < 2 * DI / CH;
     // ---- LN1 (layer 0 of a compress tile: of the embedding rows, which are also written to x at the end; lane q
     //      of a wave reads the token of its row q, handed to every lane by readlane)
-    const int tokv = EMB ? byte_token(e.bytes, e.stride, e.lens, b, e.t0 + 16 * wave + (lane & 15), e.V) : 0;
+    int tokv = 0;
+    if constexpr (GEN) {
+        if (emb) tokv = embed_token(e, b, 16 * wave + (lane & 15), Tc);
+    } else if constexpr (EMB) {
+        tokv = byte_token(e.bytes, e.stride, e.lens, b, e.t0 + 16 * wave + (lane & 15), e.V);
+    }
     {
         const float4 wv = ldg_f4(G(ln_w) + 4 * lane), bv = ldg_f4(G(ln_b) + 4 * lane);
 #pragma unroll 4
         for (int q = 0; q < BM / 4; ++q) {
             const int r = 16 * wave + q;
             float4 u;
-            if constexpr (EMB) u = ldg_f4(G(e.emb) + (int64_t)__builtin_amdgcn_readlane(tokv, q) * D + 4 * lane);
-            else u = ldg_f4(G(x) + (m0 + r) * D + 4 * lane);
+            if (emb) u = ldg_f4(G(e.emb) + (int64_t)__builtin_amdgcn_readlane(tokv, q) * D + 4 * lane);
+            else u = ldg_f4(G(x) + (m0 + (GEN && r >= Tc ? Tc - 1 : r)) * D + 4 * lane);
             const float v[4] = {u.x, u.y, u.z, u.w};
             float mu, rs;
             ln_stats_row<1>(v, mu, rs);
@@ -1467,6 +1542,7 @@ __global__ void __launch_bounds__(256, 2) k_mixin(const float* __restrict__ x, c
     // stream through 8 register slots, slot s reloaded with K step s of the next chunk right after its use.
     // Chunk order: z first (8..15), then x (0..7).
     constexpr int R1 = 8, NCH = 2 * DI / CH;
+    const int ci0 = GEN ? c0 : 0, ci1 = GEN ? c1 : NCH;
     auto chunk_of = [](int i) { return i < NCH / 2 ? NCH / 2 + i : i - NCH / 2; };  // i-th chunk processed
     u32x4 r1h[R1], r1l[R1];
     auto issue_w = [&](int k, int s) {  // block (fragment 4 k + wave, K step s) into slot s
@@ -1476,16 +1552,16 @@ __global__ void __launch_bounds__(256, 2) k_mixin(const float* __restrict__ x, c
         if constexpr (two_part_blocks<NT>()) r1l[s] = wbuf_ld16(wip, lane * 16, bo + 1024);
     };
 #pragma unroll
-    for (int s = 0; s < R1; ++s) issue_w(chunk_of(0), s);
+    for (int s = 0; s < R1; ++s) issue_w(chunk_of(ci0), s);
     floatx4 dacc[3];  // x_proj (dbc) of rows 16 wave .. + 15, fragments 0..2
 #pragma unroll
     for (int j = 0; j < 3; ++j) dacc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
     const int s1 = p0m3 == 2 ? 0 : p0m3 + 1, s2 = p0m3 == 0 ? 2 : p0m3 - 1;
 
 #pragma unroll 1
-    for (int ci = 0; ci < NCH; ++ci) {
+    for (int ci = ci0; ci < ci1; ++ci) {
         const int k = chunk_of(ci);
-        const int kn = chunk_of(ci + 1 < NCH ? ci + 1 : ci);
+        const int kn = chunk_of(ci + 1 < ci1 ? ci + 1 : ci);
         const int cl0 = 16 * wave + m_of;  // first of this lane's 4 columns within the chunk
         // loaded ahead of the ring's next blocks: its use must not wait for them (in-order wait counter)
         const float4 bias = ldg_f4(G(bin) + CH * k + cl0);
@@ -1511,10 +1587,12 @@ __global__ void __launch_bounds__(256, 2) k_mixin(const float* __restrict__ x, c
         if (k >= NCH / 2) {
             // z chunk: straight to HBM (the scan reads it)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 4; ++i) {
+                if (GEN && 16 * i + ar >= Tc) continue;
                 stg_f4(GM(xz) + (m0 + 16 * i + ar) * (2 * DI) + CH * k + cl0,
                        make_float4(epi_value<EPI_BIAS>(acc[i][0], bias.x), epi_value<EPI_BIAS>(acc[i][1], bias.y),
                                    epi_value<EPI_BIAS>(acc[i][2], bias.z), epi_value<EPI_BIAS>(acc[i][3], bias.w)));
+            }
             continue;
         }
         // x chunk: fp32 to LDS for the conv over time
@@ -1554,6 +1632,11 @@ __global__ void __launch_bounds__(256, 2) k_mixin(const float* __restrict__ x, c
             for (int e = 0; e < 3; ++e) xv[e] = sX[sx_off(g == 0 ? 0 : 16 * g - 3 + e, cl)];
 #pragma unroll
             for (int e = 0; e < 16; ++e) xv[3 + e] = sX[sx_off(16 * g + e, cl)];
+            float tail[3];  // the tile's last 3 inputs (without GEN: xv[16..18] of the last wave)
+            if constexpr (GEN) {
+#pragma unroll
+                for (int e = 0; e < 3; ++e) tail[e] = sX[sx_off(Tc - 3 + e < 0 ? 0 : Tc - 3 + e, cl)];
+            }
             __syncthreads();
             if (g == 0) {
                 xv[0] = h0;
@@ -1564,7 +1647,7 @@ __global__ void __launch_bounds__(256, 2) k_mixin(const float* __restrict__ x, c
             for (int e = 0; e < 16; ++e) {
                 const int r = 16 * g + e;
                 const float y = conv_point(cw, cb, xv[e], xv[e + 1], xv[e + 2], xv[e + 3]);
-                GM(xs)[(m0 + r) * DI + c] = y;
+                if (!GEN || r < Tc) GM(xs)[(m0 + r) * DI + c] = y;
                 if constexpr (NT == 1) {
                     *reinterpret_cast<float*>((f32_lo(cl) ? sXl : sXh) + x_off(r, f32_col(cl))) = y;
                 } else {
@@ -1574,12 +1657,14 @@ __global__ void __launch_bounds__(256, 2) k_mixin(const float* __restrict__ x, c
                     sXl[x_off(r, cl)] = (uint16_t)lo;
                 }
             }
-            // history ring: inputs of positions p0 + 61, 62, 63 in slots (p0 + 64) mod 3, + 1, + 2 (wave 3)
-            const int e0 = (p0m3 + BM) % 3, e1 = (e0 + 1) % 3, e2 = (e0 + 2) % 3;
+            // history ring: inputs of positions p0 + Tc - 3, - 2, - 1 (Tc = 64 without GEN) in slots (p0 + Tc) mod 3,
+            // + 1, + 2 (wave 3); in a tile of fewer than 3 positions the older ones are in their slots already
+            const int e0 = (p0m3 + Tc) % 3, e1 = (e0 + 1) % 3, e2 = (e0 + 2) % 3;
             const __amdgpu_buffer_rsrc_t hw = buf_rsrc(hist + b * 3 * DI, g == BM / 16 - 1 ? 3 * DI * 4 : 0);
-            buf_st1(hw, (uint32_t)(e0 * DI + c) * 4, xv[16]);
-            buf_st1(hw, (uint32_t)(e1 * DI + c) * 4, xv[17]);
-            buf_st1(hw, (uint32_t)(e2 * DI + c) * 4, xv[18]);
+            const uint32_t none = 0xFFFFFFF0u;  // past the range: the store is dropped
+            buf_st1(hw, GEN && Tc < 3 ? none : (uint32_t)(e0 * DI + c) * 4, GEN ? tail[0] : xv[16]);
+            buf_st1(hw, GEN && Tc < 2 ? none : (uint32_t)(e1 * DI + c) * 4, GEN ? tail[1] : xv[17]);
+            buf_st1(hw, (uint32_t)(e2 * DI + c) * 4, GEN ? tail[2] : xv[18]);
         }
         __syncthreads();
         // x_proj partial over this chunk's 64 channels (K block k, from zero): rows 16 wave .. + 15, fragments
@@ -1598,6 +1683,14 @@ __global__ void __launch_bounds__(256, 2) k_mixin(const float* __restrict__ x, c
             }
 #pragma unroll
             for (int j = 0; j < 3; ++j) dacc[j] = k == 0 ? part[j] : dacc[j] + part[j];
+            if (split) {  // the partial itself, in the x half of the row's xz (no one else writes it)
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (16 * wave + m_of + r < Tc)
+                            GM(xz)[(m0 + 16 * wave + m_of + r) * (2 * DI) + k * FW + 16 * j + ar] = part[j][r];
+            }
         }
         __syncthreads();  // the next x chunk rewrites sX
     }
@@ -1605,15 +1698,36 @@ __global__ void __launch_bounds__(256, 2) k_mixin(const float* __restrict__ x, c
 #pragma unroll
     for (int j = 0; j < 3; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) GM(dbc)[(m0 + 16 * wave + m_of + r) * FW + 16 * j + ar] = dacc[j][r];
+        for (int r = 0; r < 4; ++r)
+            if (!GEN || (!split && 16 * wave + m_of + r < Tc)) GM(dbc)[(m0 + 16 * wave + m_of + r) * FW + 16 * j + ar] = dacc[j][r];
     // layer 0 of a compress tile: the embedding rows to x (the residual stream), gathered again from the table
     // (an L2 hit) and stored after the tile's other work (stored in the prologue instead: the same time)
-    if constexpr (EMB) {
+    if (emb && (!GEN || c0 == 0)) {
 #pragma unroll 4
         for (int q = 0; q < BM / 4; ++q)
-            *reinterpret_cast<float4*>(e.xout + (m0 + 16 * wave + q) * D + 4 * lane) =
+            if (!GEN || 16 * wave + q < Tc) *reinterpret_cast<float4*>(e.xout + (m0 + 16 * wave + q) * D + 4 * lane) =
                 ldg_f4(G(e.emb) + (int64_t)__builtin_amdgcn_readlane(tokv, q) * D + 4 * lane);
     }
+}
+
+template <int NT, bool EMB>
+__global__ void __launch_bounds__(256, 2) k_mixin(const float* __restrict__ x, const float* __restrict__ ln_w,
+                                                 const float* __restrict__ ln_b, const uint16_t* __restrict__ Wip,
+                                                 const float* __restrict__ bin, const float* __restrict__ conv_w,
+                                                 const float* __restrict__ conv_b, const uint16_t* __restrict__ Wxp,
+                                                 float* __restrict__ xz, float* __restrict__ xs,
+                                                 float* __restrict__ dbc, float* __restrict__ hist, int p0m3,
+                                                 EmbedIn e) {
+    mixin_tile<NT, EMB, false>(x, ln_w, ln_b, Wip, bin, conv_w, conv_b, Wxp, xz, xs, dbc, hist, p0m3, e, EMB, 0, 0, 0);
+}
+
+// The general form: blockIdx.y picks the tile, blockIdx.z the in_proj chunks.
+template <int NT>
+__global__ void __launch_bounds__(256, 2) k_mixin_gen(MixinTiles a) {
+    const MixinTile& t = a.t[blockIdx.y];
+    const int c0 = (int)blockIdx.z * a.per;
+    mixin_tile<NT, false, true>(t.x, t.ln_w, t.ln_b, t.in_p, t.in_b, t.conv_w, t.conv_b, t.x_p, t.xz, t.xs, t.dbc,
+                                t.hist, t.p0m3, a.e, (int)blockIdx.y == a.emb, t.Tc, c0, c0 + a.per);
 }
 
 // The mixer's input half for d_model 512 (d_inner 1024, dt_rank 32, x_proj width 64; configs[4]'s shape), one
@@ -1632,14 +1746,15 @@ namespace mixin5 {
 constexpr int BM = 64, D = 512, DI = 1024, CH = 64, FW = 64;
 }  // namespace mixin5
 
-template <int NT, bool EMB>
-__global__ void __launch_bounds__(512, 2) k_mixin512(const float* __restrict__ x, const float* __restrict__ ln_w,
-                                                     const float* __restrict__ ln_b, const uint16_t* __restrict__ Wip,
-                                                     const float* __restrict__ bin, const float* __restrict__ conv_w,
-                                                     const float* __restrict__ conv_b, const uint16_t* __restrict__ Wxp,
-                                                     float* __restrict__ xz, float* __restrict__ xs,
-                                                     float* __restrict__ dbc, float* __restrict__ hist, int p0m3,
-                                                     EmbedIn e) {
+// GEN: as in mixin_tile (part: [rows][16][64]).
+template <int NT, bool EMB, bool GEN>
+__device__ __forceinline__ void mixin512_tile(const float* __restrict__ x, const float* __restrict__ ln_w,
+                                              const float* __restrict__ ln_b, const uint16_t* __restrict__ Wip,
+                                              const float* __restrict__ bin, const float* __restrict__ conv_w,
+                                              const float* __restrict__ conv_b, const uint16_t* __restrict__ Wxp,
+                                              float* __restrict__ xz, float* __restrict__ xs,
+                                              float* __restrict__ dbc, float* __restrict__ hist, int p0m3, EmbedIn e,
+                                              bool gather, int tc, int c0, int c1) {
     using namespace mixin5;
     using mixin::sx_off;
     using mixin::x_off;
@@ -1650,10 +1765,18 @@ __global__ void __launch_bounds__(512, 2) k_mixin512(const float* __restrict__ x
     uint16_t* sXl = sXh + BM * CH;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t b = blockIdx.x, m0 = b * BM;
+    const int Tc = GEN ? tc : BM;
+    const int64_t b = blockIdx.x, m0 = b * Tc;
+    const bool emb = GEN ? gather : EMB;  // compile-time without GEN
+    const bool split = GEN && c1 - c0 < 2 * DI / CH;
     // ---- LN1: 8 rows per wave (layer 0 of a compress tile: of the embedding rows, which are also written to x at
     //      the end; lane q of a wave reads the token of its row q, handed to every lane by readlane)
-    const int tokv = EMB ? byte_token(e.bytes, e.stride, e.lens, b, e.t0 + 8 * wave + (lane & 7), e.V) : 0;
+    int tokv = 0;
+    if constexpr (GEN) {
+        if (emb) tokv = embed_token(e, b, 8 * wave + (lane & 7), Tc);
+    } else if constexpr (EMB) {
+        tokv = byte_token(e.bytes, e.stride, e.lens, b, e.t0 + 8 * wave + (lane & 7), e.V);
+    }
     {
         const float4 w0 = ldg_f4(G(ln_w) + 4 * lane), w1 = ldg_f4(G(ln_w) + 256 + 4 * lane);
         const float4 c0 = ldg_f4(G(ln_b) + 4 * lane), c1 = ldg_f4(G(ln_b) + 256 + 4 * lane);
@@ -1663,13 +1786,14 @@ __global__ void __launch_bounds__(512, 2) k_mixin512(const float* __restrict__ x
         for (int q = 0; q < BM / 8; ++q) {
             const int r = 8 * wave + q;
             float4 u0, u1;
-            if constexpr (EMB) {
+            if (emb) {
                 const gptr<float> er = G(e.emb) + (int64_t)__builtin_amdgcn_readlane(tokv, q) * D + 4 * lane;
                 u0 = ldg_f4(er);
                 u1 = ldg_f4(er + 256);
             } else {
-                u0 = ldg_f4(G(x) + (m0 + r) * D + 4 * lane);
-                u1 = ldg_f4(G(x) + (m0 + r) * D + 256 + 4 * lane);
+                const int rr = GEN && r >= Tc ? Tc - 1 : r;
+                u0 = ldg_f4(G(x) + (m0 + rr) * D + 4 * lane);
+                u1 = ldg_f4(G(x) + (m0 + rr) * D + 256 + 4 * lane);
             }
             const float v[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
             float mu, rs;
@@ -1693,6 +1817,7 @@ __global__ void __launch_bounds__(512, 2) k_mixin512(const float* __restrict__ x
     const gptr<uint16_t> wip = G(Wip), wxp = G(Wxp);
     const int rh = wave & 1, cf = wave >> 1;
     constexpr int NS1 = D / 32, R1 = NT == 3 ? 8 : NS1, NCH = 2 * DI / CH;  // K steps per chunk, ring slots
+    const int ci0 = GEN ? c0 : 0, ci1 = GEN ? c1 : NCH;
     auto chunk_of = [](int i) { return i < NCH / 2 ? NCH / 2 + i : i - NCH / 2; };  // z chunks first, then x
     u32x4 r1h[R1], r1l[R1];
     auto issue_w = [&](int k, int s) {  // block (fragment 4 k + cf, K step s) into slot s % R1
@@ -1702,7 +1827,7 @@ __global__ void __launch_bounds__(512, 2) k_mixin512(const float* __restrict__ x
         if constexpr (NT == 3) r1l[s % R1] = ldg16(q + 512);
     };
 #pragma unroll
-    for (int s = 0; s < R1; ++s) issue_w(chunk_of(0), s);
+    for (int s = 0; s < R1; ++s) issue_w(chunk_of(ci0), s);
     const int xr = wave & 3, xf = 2 * (wave >> 2);  // x_proj: row fragment, first output fragment
     floatx4 dacc[2];
 #pragma unroll
@@ -1710,9 +1835,9 @@ __global__ void __launch_bounds__(512, 2) k_mixin512(const float* __restrict__ x
     const int s1 = p0m3 == 2 ? 0 : p0m3 + 1, s2 = p0m3 == 0 ? 2 : p0m3 - 1;
 
 #pragma unroll 1
-    for (int ci = 0; ci < NCH; ++ci) {
+    for (int ci = ci0; ci < ci1; ++ci) {
         const int k = chunk_of(ci);
-        const int kn = chunk_of(ci + 1 < NCH ? ci + 1 : ci);
+        const int kn = chunk_of(ci + 1 < ci1 ? ci + 1 : ci);
         const int cl0 = 16 * cf + m_of;  // first of this lane's 4 columns within the chunk
         const float4 bias = ldg_f4(G(bin) + CH * k + cl0);
         floatx4 acc[2];
@@ -1738,10 +1863,12 @@ __global__ void __launch_bounds__(512, 2) k_mixin512(const float* __restrict__ x
         if (k >= NCH / 2) {
             // z chunk: straight to HBM (the scan reads it)
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < 2; ++i) {
+                if (GEN && 32 * rh + 16 * i + ar >= Tc) continue;
                 stg_f4(GM(xz) + (m0 + 32 * rh + 16 * i + ar) * (2 * DI) + CH * k + cl0,
                        make_float4(epi_value<EPI_BIAS>(acc[i][0], bias.x), epi_value<EPI_BIAS>(acc[i][1], bias.y),
                                    epi_value<EPI_BIAS>(acc[i][2], bias.z), epi_value<EPI_BIAS>(acc[i][3], bias.w)));
+            }
             continue;
         }
         // x chunk: fp32 to LDS for the conv over time
@@ -1775,6 +1902,11 @@ __global__ void __launch_bounds__(512, 2) k_mixin512(const float* __restrict__ x
             for (int e = 0; e < 3; ++e) xv[e] = sX[sx_off(g == 0 ? 0 : 8 * g - 3 + e, cl)];
 #pragma unroll
             for (int e = 0; e < 8; ++e) xv[3 + e] = sX[sx_off(8 * g + e, cl)];
+            float tail[3];  // the tile's last 3 inputs (without GEN: xv[8..10] of the last wave)
+            if constexpr (GEN) {
+#pragma unroll
+                for (int e = 0; e < 3; ++e) tail[e] = sX[sx_off(Tc - 3 + e < 0 ? 0 : Tc - 3 + e, cl)];
+            }
             __syncthreads();
             if (g == 0) {
                 xv[0] = h0;
@@ -1785,18 +1917,20 @@ __global__ void __launch_bounds__(512, 2) k_mixin512(const float* __restrict__ x
             for (int e = 0; e < 8; ++e) {
                 const int r = 8 * g + e;
                 const float y = conv_point(cw, cb, xv[e], xv[e + 1], xv[e + 2], xv[e + 3]);
-                GM(xs)[(m0 + r) * DI + c] = y;
+                if (!GEN || r < Tc) GM(xs)[(m0 + r) * DI + c] = y;
                 uint32_t hi, lo;
                 split2(y, hi, lo);
                 sXh[x_off(r, cl)] = (uint16_t)hi;
                 sXl[x_off(r, cl)] = (uint16_t)lo;
             }
-            // history ring: inputs of positions p0 + 61, 62, 63 in slots (p0 + 64) mod 3, + 1, + 2 (wave 7)
-            const int e0 = (p0m3 + BM) % 3, e1 = (e0 + 1) % 3, e2 = (e0 + 2) % 3;
+            // history ring: inputs of positions p0 + Tc - 3, - 2, - 1 in slots (p0 + Tc) mod 3, + 1, + 2 (wave 7), as
+            // in mixin_tile
+            const int e0 = (p0m3 + Tc) % 3, e1 = (e0 + 1) % 3, e2 = (e0 + 2) % 3;
             const __amdgpu_buffer_rsrc_t hw = buf_rsrc(hist + b * 3 * DI, g == BM / 8 - 1 ? 3 * DI * 4 : 0);
-            buf_st1(hw, (uint32_t)(e0 * DI + c) * 4, xv[8]);
-            buf_st1(hw, (uint32_t)(e1 * DI + c) * 4, xv[9]);
-            buf_st1(hw, (uint32_t)(e2 * DI + c) * 4, xv[10]);
+            const uint32_t none = 0xFFFFFFF0u;
+            buf_st1(hw, GEN && Tc < 3 ? none : (uint32_t)(e0 * DI + c) * 4, GEN ? tail[0] : xv[8]);
+            buf_st1(hw, GEN && Tc < 2 ? none : (uint32_t)(e1 * DI + c) * 4, GEN ? tail[1] : xv[9]);
+            buf_st1(hw, (uint32_t)(e2 * DI + c) * 4, GEN ? tail[2] : xv[10]);
         }
         __syncthreads();
         // x_proj partial over this chunk's 64 channels (K block k)
@@ -1814,23 +1948,53 @@ __global__ void __launch_bounds__(512, 2) k_mixin512(const float* __restrict__ x
             }
 #pragma unroll
             for (int j = 0; j < 2; ++j) dacc[j] = k == 0 ? part[j] : dacc[j] + part[j];
+            if (split) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (16 * xr + m_of + r < Tc)
+                            GM(xz)[(m0 + 16 * xr + m_of + r) * (2 * DI) + k * FW + 16 * (xf + j) + ar] = part[j][r];
+            }
         }
         __syncthreads();  // the next x chunk rewrites sX
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) GM(dbc)[(m0 + 16 * xr + m_of + r) * FW + 16 * (xf + j) + ar] = dacc[j][r];
+        for (int r = 0; r < 4; ++r)
+            if (!GEN || (!split && 16 * xr + m_of + r < Tc)) GM(dbc)[(m0 + 16 * xr + m_of + r) * FW + 16 * (xf + j) + ar] = dacc[j][r];
     // layer 0 of a compress tile: the embedding rows to x, gathered again and stored last (as in k_mixin)
-    if constexpr (EMB) {
+    if (emb && (!GEN || c0 == 0)) {
 #pragma unroll 2
         for (int q = 0; q < BM / 8; ++q) {
+            if (GEN && 8 * wave + q >= Tc) break;
             const gptr<float> er = G(e.emb) + (int64_t)__builtin_amdgcn_readlane(tokv, q) * D + 4 * lane;
             float* xr_ = e.xout + (m0 + 8 * wave + q) * D + 4 * lane;
             *reinterpret_cast<float4*>(xr_) = ldg_f4(er);
             *reinterpret_cast<float4*>(xr_ + 256) = ldg_f4(er + 256);
         }
     }
+}
+
+template <int NT, bool EMB>
+__global__ void __launch_bounds__(512, 2) k_mixin512(const float* __restrict__ x, const float* __restrict__ ln_w,
+                                                     const float* __restrict__ ln_b, const uint16_t* __restrict__ Wip,
+                                                     const float* __restrict__ bin, const float* __restrict__ conv_w,
+                                                     const float* __restrict__ conv_b, const uint16_t* __restrict__ Wxp,
+                                                     float* __restrict__ xz, float* __restrict__ xs,
+                                                     float* __restrict__ dbc, float* __restrict__ hist, int p0m3,
+                                                     EmbedIn e) {
+    mixin512_tile<NT, EMB, false>(x, ln_w, ln_b, Wip, bin, conv_w, conv_b, Wxp, xz, xs, dbc, hist, p0m3, e, EMB, 0, 0, 0);
+}
+
+// The general form: blockIdx.y picks the tile, blockIdx.z the in_proj chunks.
+template <int NT>
+__global__ void __launch_bounds__(512, 2) k_mixin512_gen(MixinTiles a) {
+    const MixinTile& t = a.t[blockIdx.y];
+    const int c0 = (int)blockIdx.z * a.per;
+    mixin512_tile<NT, false, true>(t.x, t.ln_w, t.ln_b, t.in_p, t.in_b, t.conv_w, t.conv_b, t.x_p, t.xz, t.xs, t.dbc,
+                                   t.hist, t.p0m3, a.e, (int)blockIdx.y == a.emb, t.Tc, c0, c0 + a.per);
 }
 
 // fp32 mode: the K-block fold over the fp32 weight matrix (k_xproj_f32)
@@ -1914,12 +2078,12 @@ __device__ __forceinline__ void scan_store_y(float* xs_y, uint16_t* yh, uint16_t
 
 // Tile kernel (compress path): Tc positions per lane, h in registers across them.
 template <int NS, int R, bool OUTS>
-__global__ void __launch_bounds__(256) k_scan(float* __restrict__ xs_y, const float* __restrict__ dbc, int ldd,
-                                             const float* __restrict__ xz, int64_t ldxz,
-                                             const float* __restrict__ dt_w, const float* __restrict__ dt_b,
-                                             const float* __restrict__ Aneg, const float* __restrict__ Dp,
-                                             float* __restrict__ ssm, int di, int Tc, uint16_t* __restrict__ yh,
-                                             uint16_t* __restrict__ yl) {
+__device__ __forceinline__ void scan_tile(float* __restrict__ xs_y, const float* __restrict__ dbc, int ldd,
+                                          const float* __restrict__ xz, int64_t ldxz,
+                                          const float* __restrict__ dt_w, const float* __restrict__ dt_b,
+                                          const float* __restrict__ Aneg, const float* __restrict__ Dp,
+                                          float* __restrict__ ssm, int di, int Tc, uint16_t* __restrict__ yh,
+                                          uint16_t* __restrict__ yl) {
     const int64_t b = blockIdx.y;
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t row0 = b * Tc;
@@ -1952,6 +2116,168 @@ __global__ void __launch_bounds__(256) k_scan(float* __restrict__ xs_y, const fl
         }
     }
     scan_store_channel<NS>(hp, di, h);
+}
+
+template <int NS, int R, bool OUTS>
+__global__ void __launch_bounds__(256) k_scan(float* __restrict__ xs_y, const float* __restrict__ dbc, int ldd,
+                                             const float* __restrict__ xz, int64_t ldxz,
+                                             const float* __restrict__ dt_w, const float* __restrict__ dt_b,
+                                             const float* __restrict__ Aneg, const float* __restrict__ Dp,
+                                             float* __restrict__ ssm, int di, int Tc, uint16_t* __restrict__ yh,
+                                             uint16_t* __restrict__ yl) {
+    scan_tile<NS, R, OUTS>(xs_y, dbc, ldd, xz, ldxz, dt_w, dt_b, Aneg, Dp, ssm, di, Tc, yh, yl);
+}
+
+struct ScanTile {
+    float* xs;           // conv output in; y out in its place (fp32 mode)
+    const float *dbc, *xz, *dt_w, *dt_b, *Aneg, *D;
+    float* ssm;
+    uint16_t *yh, *yl;   // y out, split (split modes)
+    int Tc;
+};
+struct ScanTiles {
+    ScanTile t[PIPE_MAX];
+    int di;
+    int parts;  // x_proj partials per row to fold (in the x half of xz); 0: dbc holds their sum
+};
+
+// The same over several tiles in one launch: blockIdx.z picks the tile.
+template <int NS, int R, bool OUTS>
+__global__ void __launch_bounds__(256) k_scan_gen(ScanTiles a) {
+    const ScanTile& t = a.t[blockIdx.z];
+    scan_tile<NS, R, OUTS>(t.xs, t.dbc, R + 2 * NS, t.xz, 2 * a.di, t.dt_w, t.dt_b, t.Aneg, t.D, t.ssm, a.di, t.Tc, t.yh, t.yl);
+}
+
+// The scan of a tile when there are too few (lane, channel) chains to fill the GPU: four threads per channel, each
+// with 4 of its 16 states, and everything that does not depend on the state done in parallel over the tile's
+// positions.  A workgroup owns 64 channels of one lane's tile of Tc <= 64 positions:
+//   1. [dr | B | C] rows to LDS, folding the x_proj partials where the mixer kernel left them (P_0 + P_1 + ...);
+//   2. dt = softplus(dt_proj) and dt * x of every (position, channel) to LDS, SiLU(z) kept in registers;
+//   3. the recurrence: thread j of a channel updates states 4 j .. 4 j + 3 of position s - j at step s, so that
+//      y = sum_n h_n C_n is accumulated in state order while it moves from thread to thread (DPP), one step each;
+//   4. + D x, the gate, and the store, in parallel over positions.
+// Every value is formed by the operations of scan_position in their order, so y and the state equal k_scan's bit for
+// bit.  One thread per channel (k_scan) is a serial chain of about 80 dependent operations per position and takes
+// 57 us per 64 positions at 1 to 64 lanes; this takes 17 us (1 lane, 8 tiles in flight).
+template <int R, bool OUTS>
+__global__ void __launch_bounds__(256) k_scan_quad(ScanTiles a) {
+    constexpr int NS = 16, FW = R + 2 * NS, BM = 64, LD = 80;  // LD: the four positions in flight hit other banks
+    __shared__ __attribute__((aligned(16))) float sRow[BM * FW];
+    __shared__ float sDt[BM * LD], sDx[BM * LD];  // dt (then y in its place) and dt * x, [position][channel]
+    const ScanTile& tl = a.t[blockIdx.z];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, Tc = tl.Tc, di = a.di;
+    const int64_t b = blockIdx.y, row0 = b * Tc;
+    const int c0 = blockIdx.x * 64;
+    // phases 2 and 4: channel c0 + lane, positions wave, wave + 4, ...
+    const int c = c0 + lane;
+    float xv[16], zv[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int t = 4 * i + wave;
+        const int64_t m = row0 + (t < Tc ? t : Tc - 1);
+        xv[i] = tl.xs[m * di + c];
+        zv[i] = tl.xz[m * 2 * di + di + c];
+    }
+    float wr[R];
+#pragma unroll
+    for (int r = 0; r < R; r += 4) {
+        const float4 q = *reinterpret_cast<const float4*>(tl.dt_w + (int64_t)c * R + r);
+        wr[r] = q.x; wr[r + 1] = q.y; wr[r + 2] = q.z; wr[r + 3] = q.w;
+    }
+    const float bdt = tl.dt_b[c], Dc = tl.D[c];
+    // phase 3: channel c0 + 16 wave + lane / 4, states 4 j .. 4 j + 3
+    const int j = lane & 3, cs = 16 * wave + (lane >> 2);
+    float* hp = tl.ssm + b * di * NS + ((int64_t)j * di + c0 + cs) * 4;
+    const float4 h4 = *reinterpret_cast<const float4*>(hp);
+    const float4 a4 = *reinterpret_cast<const float4*>(tl.Aneg + ((int64_t)j * di + c0 + cs) * 4);
+    if (a.parts == 0) {
+        for (int i = tid; i < Tc * FW; i += 256) sRow[i] = tl.dbc[row0 * FW + i];
+    } else {
+        for (int i = tid; i < Tc * FW; i += 256) {
+            const int t = i / FW;
+            const float* p = tl.xz + (row0 + t) * 2 * di + (i - t * FW);
+            float v = p[0];
+            if constexpr (R == 16) {
+#pragma unroll
+                for (int q = 1; q < 8; ++q) v = v + p[q * FW];
+            } else {
+#pragma unroll
+                for (int q = 1; q < 16; ++q) v = v + p[q * FW];
+            }
+            sRow[i] = v;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int t = 4 * i + wave;
+        if (t < Tc) {
+            const float dt = scan_dt<R>(&sRow[t * FW], wr, bdt);
+            sDt[t * LD + lane] = dt;
+            sDx[t * LD + lane] = dt * xv[i];
+            zv[i] = hw_silu(zv[i]);
+        }
+    }
+    __syncthreads();
+    {
+        float h[4] = {h4.x, h4.y, h4.z, h4.w};
+        const float av[4] = {a4.x, a4.y, a4.z, a4.w};
+        float y = 0.0f;
+        struct In {
+            float dt, dtx;
+            float4 B, C;
+        };
+        // thread j's inputs at step s (position s - j, clamped into the tile outside it), read one step ahead
+        auto read = [&](int s) {
+            int t = s - j;
+            t = t < 0 ? 0 : (t < Tc ? t : Tc - 1);
+            In v;
+            v.dt = sDt[t * LD + cs];
+            v.dtx = sDx[t * LD + cs];
+            v.B = *reinterpret_cast<const float4*>(&sRow[t * FW + R + 4 * j]);
+            v.C = *reinterpret_cast<const float4*>(&sRow[t * FW + R + NS + 4 * j]);
+            return v;
+        };
+        In nx = read(0);
+        auto step = [&](int s, bool all) {
+            const In v = nx;
+            nx = read(s + 1);
+            // y of this position so far, from the thread before (thread 0 starts at 0)
+            const float yin = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, y), 0x111, 0xF, 0xF, true));
+            const int t = s - j;
+            if (all || (t >= 0 && t < Tc)) {
+                const float Bn[4] = {v.B.x, v.B.y, v.B.z, v.B.w}, Cn[4] = {v.C.x, v.C.y, v.C.z, v.C.w};
+                y = j == 0 ? 0.0f : yin;
+#pragma unroll
+                for (int n = 0; n < 4; ++n) {
+                    const float dA = __builtin_amdgcn_exp2f(v.dt * av[n]);
+                    const float dBx = Bn[n] * v.dtx;
+                    h[n] = __builtin_fmaf(dA, h[n], dBx);
+                    y = __builtin_fmaf(h[n], Cn[n], y);
+                }
+                if (j == 3) sDt[t * LD + cs] = y;  // thread 3 is the last to read this position's dt
+            }
+        };
+        int s = 0;
+        for (; s < 3; ++s) step(s, false);
+        for (; s + 4 <= Tc; s += 4) {  // every thread inside the tile
+            step(s, true);
+            step(s + 1, true);
+            step(s + 2, true);
+            step(s + 3, true);
+        }
+        for (; s < Tc + 3; ++s) step(s, false);
+        *reinterpret_cast<float4*>(hp) = make_float4(h[0], h[1], h[2], h[3]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int t = 4 * i + wave;
+        if (t < Tc) {
+            const float y = __builtin_fmaf(Dc, xv[i], sDt[t * LD + lane]);
+            scan_store_y<OUTS>(tl.xs, tl.yh, tl.yl, (row0 + t) * di + c, y * zv[i]);
+        }
+    }
 }
 
 // Step kernel (decompress path, per-layer kernels): one position per lane.  A workgroup owns 256 channels of
@@ -2015,17 +2341,6 @@ __global__ void k_enc_init(EncState* st, int n) {
     if (i < n) enc_init(st[i]);
 }
 
-// cumulative of symbol s and its weight, from the owner lane (s uniform across the wave)
-__device__ __forceinline__ void xq_sym(const XQ& q, int s, uint32_t& c_s, uint32_t& f_s) {
-    const int j = s & 3;
-    uint32_t cl = q.base, fl = q.f[0];
-    if (j >= 1) { cl += q.f[0]; fl = q.f[1]; }
-    if (j >= 2) { cl += q.f[1]; fl = q.f[2]; }
-    if (j >= 3) { cl += q.f[2]; fl = q.f[3]; }
-    c_s = wave_bcast(cl, s >> 2);
-    f_s = wave_bcast(fl, s >> 2);
-}
-
 // Encodes the symbols predicted by the Tc positions of this launch: the logits of position p (absolute
 // t0 + t) code byte p + 1 of the chunk (codec.py:56-76: step(byte t-1) -> probabilities of byte t).
 __global__ void __launch_bounds__(64) k_encode_tile(const float* __restrict__ logits, int V, int Tc, int t0,
@@ -2044,13 +2359,8 @@ __global__ void __launch_bounds__(64) k_encode_tile(const float* __restrict__ lo
         if (p + 1 >= L) break;
         const int s = src[p + 1];
         if (s >= V) continue;  // as gpu_range_coder.py:97: symbols outside [0, K) are skipped
-        XQ q;
-        xq_build(q, logits_row4(logits + (b * Tc + t) * V, V, lane), lane, V, CODER_P);
-        uint32_t c_s, f_s;
-        xq_sym(q, s, c_s, f_s);
-        const uint32_t lo = xq_cdf_at(q, c_s, s);
-        const uint32_t hi = (s + 1 < V) ? xq_cdf_at(q, c_s + f_s, s + 1) : (1u << CODER_P);
-        enc_push(st, CODER_P, lo, hi - lo, sink);
+        const uint2 v = xq_interval(logits_row4(logits + (b * Tc + t) * V, V, lane), V, lane, s);
+        enc_push(st, CODER_P, v.x, v.y, sink);
     }
     if (lane == 0) states[b] = st;
 }
@@ -2076,7 +2386,6 @@ __global__ void __launch_bounds__(64) k_encode_tile(const float* __restrict__ lo
 // D = 256: 80 KB, two workgroups per CU; D = 512: 144 KB, one.
 namespace headq {
 constexpr int BM = 64, V = 256, HC = 64, LLOG = V + 4;
-constexpr uint32_t SKIP = 0xFFFFFFFFu;  // no symbol at this position (past the chunk's end, or byte >= V)
 // 16-byte chunks XOR-swizzled by row (low 4 bits of the chunk index), so 16-row fragment reads spread over banks
 template <int D> __device__ __forceinline__ int a_off(int r, int k) { return r * D + (((k >> 3) ^ (r & 15)) << 3) + (k & 7); }
 __device__ __forceinline__ int h_off(int r, int k) { return r * HC + (((k >> 3) ^ (r >> 1)) & 7) * 8 + (k & 7); }
@@ -2085,7 +2394,9 @@ template <int D> constexpr int lds_bytes() {
 }
 }  // namespace headq
 
-template <int NT, int D>
+// GEN: tiles of Tc <= 64 positions (rows past Tc repeat the last and give no output), and, where `logits` is set, the
+// logits themselves (row t of lane b at logits[(b * len + t0 + t) * V], the teacher-forced forward) instead of intervals.
+template <int NT, int D, bool GEN>
 __global__ void __launch_bounds__(512, (D == 256) ? 4 : 2) k_head_xq(const float* __restrict__ xin,
                                                                    const uint16_t* __restrict__ W1p,
                                                                    const float* __restrict__ b1,
@@ -2093,8 +2404,10 @@ __global__ void __launch_bounds__(512, (D == 256) ? 4 : 2) k_head_xq(const float
                                                                    const float* __restrict__ b2, int t0,
                                                                    const uint8_t* __restrict__ bytes, int64_t stride,
                                                                    const int32_t* __restrict__ lens,
-                                                                   uint2* __restrict__ lf) {
+                                                                   uint2* __restrict__ lf, int tc,
+                                                                   float* __restrict__ logits, int64_t len) {
     using namespace headq;
+    const int Tc = GEN ? tc : BM;
     __shared__ __attribute__((aligned(16))) unsigned char lds[lds_bytes<D>()];
     uint16_t* sAh = reinterpret_cast<uint16_t*>(lds);
     uint16_t* sAl = sAh + BM * D;
@@ -2105,13 +2418,13 @@ __global__ void __launch_bounds__(512, (D == 256) ? 4 : 2) k_head_xq(const float
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t b = blockIdx.x;
     {
-        const gptr<float> xr = G(xin) + b * BM * D;
+        const gptr<float> xr = G(xin) + b * Tc * D;
 #pragma unroll 4
         for (int q = 0; q < BM / 8; ++q) {
             const int r = 8 * wave + q;
 #pragma unroll
             for (int h = 0; h < D / 256; ++h) {
-                const float4 v = ldg_f4(xr + r * D + 256 * h + 4 * lane);
+                const float4 v = ldg_f4(xr + (GEN && r >= Tc ? Tc - 1 : r) * D + 256 * h + 4 * lane);
                 if constexpr (NT == 1) {
                     const int k = 256 * h + 4 * lane;
                     *reinterpret_cast<float4*>((f32_lo(k) ? sAl : sAh) + a_off<D>(r, f32_col(k))) = v;
@@ -2233,6 +2546,14 @@ __global__ void __launch_bounds__(512, (D == 256) ? 4 : 2) k_head_xq(const float
             for (int r = 0; r < 4; ++r) sLog[(16 * i + m_of + r) * LLOG + col] = epi_value<EPI_BIAS>(out[i][j][r], bias);
     }
     __syncthreads();
+    if (GEN && logits) {
+        for (int i = tid; i < Tc * (V / 4); i += 512) {
+            const int t = i / (V / 4), c4 = (i % (V / 4)) * 4;
+            *reinterpret_cast<float4*>(logits + (b * len + t0 + t) * V + c4) =
+                *reinterpret_cast<const float4*>(sLog + t * LLOG + c4);
+        }
+        return;
+    }
     // quantiser and coder interval per position: wave w takes positions 8 w .. 8 w + 7 (uniform per wave)
     const int L = lens[b];
     const uint8_t* src = bytes + b * stride;
@@ -2240,20 +2561,13 @@ __global__ void __launch_bounds__(512, (D == 256) ? 4 : 2) k_head_xq(const float
     for (int q = 0; q < BM / 8; ++q) {
         const int t = 8 * wave + q;
         const int p = t0 + t;
-        uint2 v = make_uint2(SKIP, 0u);
+        if (GEN && t >= Tc) break;
+        uint2 v = make_uint2(LF_SKIP, 0u);
         if (p + 1 < L) {
             const int s = src[p + 1];
-            if (s < V) {
-                XQ xq;
-                xq_build(xq, logits_row4(sLog + t * LLOG, V, lane), lane, V, CODER_P);
-                uint32_t c_s, f_s;
-                xq_sym(xq, s, c_s, f_s);
-                const uint32_t lo = xq_cdf_at(xq, c_s, s);
-                const uint32_t hi = (s + 1 < V) ? xq_cdf_at(xq, c_s + f_s, s + 1) : (1u << CODER_P);
-                v = make_uint2(lo, hi - lo);
-            }
+            if (s < V) v = xq_interval(logits_row4(sLog + t * LLOG, V, lane), V, lane, s);
         }
-        if (lane == 0) lf[b * BM + t] = v;
+        if (lane == 0) lf[b * Tc + t] = v;
     }
 }
 
@@ -2266,12 +2580,33 @@ __global__ void __launch_bounds__(256) k_encode_lf(const uint2* __restrict__ lf,
     EncState st = states[b];
     const WordSink sink{words + b * pitch, pitch, true};
     const uint2* q = lf + b * Tc;
-    for (int t = 0; t < Tc; ++t) {
-        const uint2 v = q[t];
-        if (v.x == headq::SKIP) continue;
-        enc_push(st, CODER_P, v.x, v.y, sink);
+    // the next 8 intervals are in flight while 8 are coded (loads past the tile repeat its last one, unused): with one
+    // load per interval in front of its use every symbol waited for memory
+    constexpr int U = 8;
+    uint2 v[U], nx[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) nx[u] = q[u < Tc ? u : Tc - 1];
+    for (int t0 = 0; t0 < Tc; t0 += U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = nx[u];
+#pragma unroll
+        for (int u = 0; u < U; ++u) nx[u] = q[t0 + U + u < Tc ? t0 + U + u : Tc - 1];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (t0 + u < Tc && v[u].x != LF_SKIP) enc_push(st, CODER_P, v[u].x, v[u].y, sink);
     }
     states[b] = st;
+}
+
+// Zeroes the recurrent state of lanes [0, lanes) of every layer (blockIdx.y: conv history rows of nh floats, state rows
+// of ns floats per lane), in one launch and without memset nodes.
+__global__ void __launch_bounds__(256) k_state_zero(float* __restrict__ hist, int64_t nh, float* __restrict__ ssm,
+                                                   int64_t ns, int lanes, int64_t max_lanes) {
+    const int64_t l = blockIdx.y, stride = (int64_t)gridDim.x * blockDim.x * 4;
+    const int64_t i0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int64_t i = i0; i < lanes * nh; i += stride) *reinterpret_cast<float4*>(hist + l * max_lanes * nh + i) = z;
+    for (int64_t i = i0; i < lanes * ns; i += stride) *reinterpret_cast<float4*>(ssm + l * max_lanes * ns + i) = z;
 }
 
 __global__ void k_enc_finish(EncState* states, uint32_t* words, int64_t pitch, int32_t* nwords, int32_t* overflow,
@@ -2423,6 +2758,10 @@ struct boa_ctx {
     // 2 or 3 groups, default 2)
     bool compress_halves = true;
     int compress_groups = 2;
+    // Launches over several tiles at once for few lanes (run_pipe; BOA_PIPE=0: tile after tile, layer after layer).
+    // ws_rows: rows of x, xz, xs, dbc and the split activations (every tile in flight has its own)
+    bool pipe = true;
+    int64_t ws_rows = 0;
     hipStream_t stream2 = nullptr;
     hipStream_t stream3 = nullptr;     // the third compress group's
     std::vector<hipEvent_t> half_ev;   // [2][L]: state group of layer l done, per half; [2L], [2L + 1]: stream joins
@@ -2552,16 +2891,39 @@ static bool want_fused(const boa_model_cfg& c, int R, int precision) {
     return (d256 || (d512 && precision != BOA_PREC_F32)) && !(fenv && fenv[0] == '0');
 }
 
+// Whether the fused tile kernels (mixer input, scan, feed-forward with out_proj) cover a shape: d_model 256 in every
+// precision mode, d_model 512 in the split modes.
+static bool tile_kernels(const boa_model_cfg& c, int R, int precision) {
+    if (c.d_model == mixin::D) return R + 2 * c.d_state == mixin::FW && fused_step_supported(c.d_model, c.d_state, R, c.d_conv, c.vocab);
+    return c.d_model == mixin5::D && precision != BOA_PREC_F32 && R + 2 * c.d_state == mixin5::FW;
+}
+// Positions per tile of run_pipe, and the workspace rows of a context: max_lanes tiles as every path needs, and for
+// contexts of few lanes room for run_pipe's other tiles in flight: one per layer, but at most PIPE_TILES (lane, tile)
+// pairs in all, which is enough 64-row workgroups for every CU with room to even out the last round.  Sized for the
+// lanes rounded up to a power of two (16 at least).
+constexpr int PIPE_TILES = 2048, PIPE_MIN_TILE = 16, PIPE_LANES = 511;
+static int pipe_tile(int64_t tile_len) { return (int)std::min<int64_t>(tile_len, 64); }
+static int64_t workspace_rows(const boa_model_cfg& c, int R, int precision, int64_t max_lanes, int64_t tile_len) {
+    const int64_t rows = max_lanes * tile_len;
+    const char* env = getenv("BOA_PIPE");
+    if (!tile_kernels(c, R, precision) || pipe_tile(tile_len) < PIPE_MIN_TILE || max_lanes > PIPE_LANES || (env && env[0] == '0'))
+        return rows;
+    int64_t up = 16;
+    while (up < max_lanes) up *= 2;
+    const int64_t p = std::max<int64_t>(1, std::min<int64_t>(PIPE_TILES / up, std::min(c.n_layers, PIPE_MAX)));
+    return rows + (p - 1) * up * pipe_tile(tile_len);
+}
+
 // Device bytes boa_ctx_create allocates for this shape: the same list of buffers, in the same order, each
 // rounded as dmalloc rounds it.  boa_ctx_create checks its own total against this after allocating.
 static int64_t ctx_plan_bytes(const boa_model_cfg& c, int R, int precision, int64_t max_lanes, int64_t tile_len) {
     const int64_t d = c.d_model, di = (int64_t)c.expand * c.d_model, NS = c.d_state, V = c.vocab, L = c.n_layers;
-    const int64_t rows = max_lanes * tile_len;
+    const int64_t rows = max_lanes * tile_len, ws = workspace_rows(c, R, precision, max_lanes, tile_len);
     auto f4 = [](int64_t n) { return 4 * std::max<int64_t>(n, 1); };
     int64_t b = f4(weights_floats(c, R)) + f4(L * di * NS) + f4(L * max_lanes * 3 * di) + f4(L * max_lanes * di * NS) +
-                f4(rows * d) + f4(rows * std::max(2 * di, 4 * d)) + f4(rows * di) + f4(rows * (R + 2 * NS)) +
+                f4(ws * d) + f4(ws * std::max(2 * di, 4 * d)) + f4(ws * di) + f4(ws * (R + 2 * NS)) +
                 f4(rows * d) + f4(rows * V) + 8 * std::max<int64_t>(rows, 1);
-    if (precision != BOA_PREC_F32) b += 2 * 2 * std::max<int64_t>(rows * std::max(d, di), 1);
+    if (precision != BOA_PREC_F32) b += 2 * 2 * std::max<int64_t>(ws * std::max(d, di), 1);
     b += f4(max_lanes) + (int64_t)sizeof(EncState) * max_lanes + (int64_t)sizeof(DecState) * max_lanes + 4;
     const int64_t mats = L * (2 * di * d + (R + 2 * NS) * di + d * di + 4 * d * d + 4 * d * d) + d * d + V * d;
     if (precision != BOA_PREC_F32) {
@@ -2681,6 +3043,9 @@ extern "C" int boa_ctx_create(const boa_model_cfg* cfg, const void* h_weights, i
     x->prec = precision;
     x->max_lanes = max_lanes; x->tile_len = tile_len; x->max_rows = max_rows;
     const int d = x->d, di = x->di, NS = x->NS, V = x->V, L = x->L;
+    x->ws_rows = workspace_rows(c, R, precision, max_lanes, tile_len);
+    if (const char* v = getenv("BOA_PIPE")) x->pipe = v[0] != '0';
+    x->pipe = x->pipe && tile_kernels(c, R, precision);
 
     hipError_t e = hipSuccess;
 #define TRY_ALLOC(p, n) do { if (e == hipSuccess) e = dmalloc(x, &(p), (n)); } while (0)
@@ -2688,16 +3053,16 @@ extern "C" int boa_ctx_create(const boa_model_cfg* cfg, const void* h_weights, i
     TRY_ALLOC(x->aneg, (int64_t)L * di * NS);
     TRY_ALLOC(x->conv_hist, (int64_t)L * max_lanes * 3 * di);
     TRY_ALLOC(x->ssm, (int64_t)L * max_lanes * di * NS);
-    TRY_ALLOC(x->x, max_rows * d);
-    TRY_ALLOC(x->xz, max_rows * std::max(2 * di, 4 * d));
-    TRY_ALLOC(x->xs, max_rows * di);
-    TRY_ALLOC(x->dbc, max_rows * (R + 2 * NS));
+    TRY_ALLOC(x->x, x->ws_rows * d);
+    TRY_ALLOC(x->xz, x->ws_rows * std::max(2 * di, 4 * d));
+    TRY_ALLOC(x->xs, x->ws_rows * di);
+    TRY_ALLOC(x->dbc, x->ws_rows * (R + 2 * NS));
     TRY_ALLOC(x->mm, max_rows * d);
     TRY_ALLOC(x->logits, max_rows * V);
     TRY_ALLOC(x->stats, max_rows);
     if (precision != BOA_PREC_F32) {
-        TRY_ALLOC(x->ah, max_rows * std::max(d, di));
-        TRY_ALLOC(x->al, max_rows * std::max(d, di));
+        TRY_ALLOC(x->ah, x->ws_rows * std::max(d, di));
+        TRY_ALLOC(x->al, x->ws_rows * std::max(d, di));
     }
     TRY_ALLOC(x->tokens, (int64_t)max_lanes);
     TRY_ALLOC(x->enc, (int64_t)max_lanes);
@@ -2877,12 +3242,13 @@ extern "C" int boa_ctx_create(const boa_model_cfg* cfg, const void* h_weights, i
 extern "C" int boa_state_reset(boa_ctx* x, int32_t lanes) {
     if (!x || lanes < 0 || lanes > x->max_lanes) return boa_fail(BOA_ERR_ARG, "boa_state_reset: bad lanes");
     x->pos = 0;
-    for (int l = 0; l < x->L; ++l) {
-        BOA_HIP_TRY(hipMemsetAsync(x->conv_hist + (int64_t)l * x->max_lanes * 3 * x->di, 0,
-                                   sizeof(float) * (size_t)lanes * 3 * x->di, x->stream));
-        BOA_HIP_TRY(hipMemsetAsync(x->ssm + (int64_t)l * x->max_lanes * x->di * x->NS, 0,
-                                   sizeof(float) * (size_t)lanes * x->di * x->NS, x->stream));
-    }
+    if (lanes == 0) return BOA_OK;
+    // one launch for all layers (two memsets per layer took 2 us each plus their gaps: 60 us at 8 layers)
+    const int64_t ns = (int64_t)x->di * x->NS;
+    const unsigned blocks = (unsigned)std::min<int64_t>((lanes * ns / 4 + 255) / 256, 1024);
+    hipLaunchKernelGGL(k_state_zero, dim3(blocks, (unsigned)x->L), dim3(256), 0, x->stream, x->conv_hist,
+                       (int64_t)3 * x->di, x->ssm, ns, lanes, (int64_t)x->max_lanes);
+    BOA_HIP_TRY(hipGetLastError());
     return BOA_OK;
 }
 
@@ -2933,15 +3299,48 @@ static void launch_scan(boa_ctx* x, const LayerW& w, float* ssm, int B, int Tc) 
 }
 
 // Whether a layer of a Tc-position tile runs LN1 through x_proj as one mixer-input kernel: k_mixin512 (d_model
-// 512, split modes) or k_mixin (d_model 256, every mode), on full tiles with fragment-packed weights.
+// 512, split modes) or k_mixin (d_model 256, every mode), with fragment-packed weights, on full tiles, and in their
+// general forms on shorter ones of at least tile_min_rows positions: a lane's tile is one workgroup of 64 rows however
+// few it holds, while the layer-by-layer kernels pack the lanes' rows.  Compress of 2000 lanes (d 256, 4 layers, fp32;
+// 1000 lanes at d 512, 4 layers, bf16w), mixer kernel against layer by layer, by positions of the only tile:
+//   25: 5.96 / 5.52 ms   33: 6.67 / 6.86   41: 7.20 / 7.66   57: 8.41 / 10.27   (d 256)
+//   33: 4.07 / 3.85 ms   41: 4.57 / 4.42   49: 4.93 / 5.22   57: 5.47 / 5.92    (d 512)
+static int tile_min_rows(const boa_ctx* x) { return x->d == 512 ? 48 : 32; }
 static bool mixin512_layer(const boa_ctx* x, const LayerW& w, int Tc) {
     return x->prec != BOA_PREC_F32 && x->d == mixin5::D && x->di == mixin5::DI && x->R + 2 * x->NS == mixin5::FW &&
-           Tc == mixin5::BM && w.in_w.p && w.x_w.p;
+           Tc <= mixin5::BM && Tc >= tile_min_rows(x) && w.in_w.p && w.x_w.p;
 }
 static bool mixin_layer(const boa_ctx* x, const LayerW& w, int Tc) {
     return !mixin512_layer(x, w, Tc) && x->d == mixin::D && x->di == mixin::DI && x->R + 2 * x->NS == mixin::FW &&
-           Tc == mixin::BM && w.in_w.p && w.x_w.p;
+           Tc <= mixin::BM && Tc >= tile_min_rows(x) && w.in_w.p && w.x_w.p;
 }
+// One tile of a general launch: rows from row_off on in the context's buffers, lanes from x->lane0 on.
+static MixinTile mixin_tile_args(const boa_ctx* x, int l, int64_t row_off, int64_t pos, int Tc) {
+    const LayerW& w = x->layers[l];
+    const int64_t d = x->d, di = x->di;
+    MixinTile t;
+    t.x = x->x + row_off * d; t.ln_w = w.ln1_w; t.ln_b = w.ln1_b; t.in_b = w.in_b; t.conv_w = w.conv_w; t.conv_b = w.conv_b;
+    t.in_p = w.in_w.p; t.x_p = w.x_w.p;
+    t.xz = x->xz + row_off * 2 * di; t.xs = x->xs + row_off * di; t.dbc = x->dbc + row_off * (x->R + 2 * x->NS);
+    t.hist = x->conv_hist + ((int64_t)l * x->max_lanes + x->lane0) * 3 * di;
+    t.p0m3 = (int)(pos % 3); t.Tc = Tc;
+    return t;
+}
+// blockIdx.z workgroups per tile, each with an equal share of its in_proj chunks (per chunks)
+static void launch_mixin_gen(const boa_ctx* x, const MixinTiles& a, int lanes, int tiles, int z, hipStream_t s) {
+    const dim3 grid((unsigned)lanes, (unsigned)tiles, (unsigned)z);
+    if (x->d == mixin5::D) {
+        if (x->prec == BOA_PREC_BF16X3) hipLaunchKernelGGL((k_mixin512_gen<3>), grid, dim3(512), 0, s, a);
+        else hipLaunchKernelGGL((k_mixin512_gen<2>), grid, dim3(512), 0, s, a);
+    } else if (x->prec == BOA_PREC_F32) {
+        hipLaunchKernelGGL((k_mixin_gen<1>), grid, dim3(256), 0, s, a);
+    } else if (x->prec == BOA_PREC_BF16X3) {
+        hipLaunchKernelGGL((k_mixin_gen<3>), grid, dim3(256), 0, s, a);
+    } else {
+        hipLaunchKernelGGL((k_mixin_gen<2>), grid, dim3(256), 0, s, a);
+    }
+}
+static int mixin_chunks(const boa_ctx* x) { return 2 * x->di / 64; }
 // Whether a compress tile of Tc positions skips the embedding pass: its layer 0 gathers the rows (EmbedIn).
 static bool embed_in_mixin(const boa_ctx* x, int Tc) {
     return x->embed_ln1 && x->L > 0 && (mixin512_layer(x, x->layers[0], Tc) || mixin_layer(x, x->layers[0], Tc));
@@ -2987,7 +3386,14 @@ static int run_layer(boa_ctx* x, int l, int B, int Tc, int part = 7) {
     int rc = 0;
     float* hist = x->conv_hist + ((int64_t)l * x->max_lanes + x->lane0) * 3 * di;
     const bool mix5 = mixin512_layer(x, w, Tc);
-    if (mix5 && (part & 1)) {
+    const bool shorter = Tc < mixin::BM && (mix5 || mixin_layer(x, w, Tc));
+    if (shorter && (part & 1)) {
+        MixinTiles a;
+        a.t[0] = mixin_tile_args(x, l, 0, x->pos, Tc);
+        a.e = ein; a.emb = emb ? 0 : -1; a.per = mixin_chunks(x);
+        PROF(PC_MIXIN, gemm_flops(M, 2 * di, d) + gemm_flops(M, R + 2 * NS, di) + 8.0 * M * di,
+             4.0 * M * (d + di + di + R + 2 * NS) + 4.0 * 6 * B * di, launch_mixin_gen(x, a, B, 1, 1, s));
+    } else if (mix5 && (part & 1)) {
         // LN1 + in_proj + conv + SiLU + x_proj in one kernel per lane tile, d_model 512
         const double flops = gemm_flops(M, 2 * di, d) + gemm_flops(M, R + 2 * NS, di) + 8.0 * M * di;
         const double bytes = 4.0 * M * (d + di + di + R + 2 * NS) + 4.0 * 6 * B * di;
@@ -3010,7 +3416,9 @@ static int run_layer(boa_ctx* x, int l, int B, int Tc, int part = 7) {
     }
     // (fp32 mode included: its fragment-packed weights exist at d_model 256)
     const bool mix = mixin_layer(x, w, Tc);
-    if (mix && (part & 1)) {
+    if (shorter) {
+        // launched above
+    } else if (mix && (part & 1)) {
         // LN1 + in_proj + conv + SiLU + x_proj in one kernel per lane tile
         const double flops = gemm_flops(M, 2 * di, d) + gemm_flops(M, R + 2 * NS, di) + 8.0 * M * di;
         const double bytes = 4.0 * M * (d + di + di + R + 2 * NS) + 4.0 * 6 * B * di;
@@ -3219,12 +3627,12 @@ static int run_layer(boa_ctx* x, int l, int B, int Tc, int part = 7) {
 
 // Full model over B x Tc rows already embedded in ctx->x; logits to `out` (ld V).
 // Head (Linear -> ReLU -> Linear) over B x Tc rows of ctx->x; logits to `out` (ld V).
-static int run_head(boa_ctx* x, int B, int Tc, float* out) {
+static int run_head(boa_ctx* x, int B, int Tc, float* out, const float* xin = nullptr) {
     const int d = x->d, V = x->V;
     const int64_t M = (int64_t)B * Tc;
     const bool split = x->prec != BOA_PREC_F32;
     int rc = 0;
-    GemmArgs g1 = gemm_args(x->x, d, x->h1_w, x->h1_b, x->mm, d, M, d, d);
+    GemmArgs g1 = gemm_args(xin ? xin : x->x, d, x->h1_w, x->h1_b, x->mm, d, M, d, d);
     GemmArgs g2 = gemm_args(x->mm, d, x->h2_w, x->h2_b, out, V, M, V, d);
     if (split) {
         g1.Ch = x->ah; g1.Cl = x->al;
@@ -3356,10 +3764,233 @@ extern "C" int boa_model_step(boa_ctx* x, const int32_t* d_tokens, int32_t lanes
     return rc;
 }
 
+// ------------------------------------------------------------------------------------------------
+// Tiles in flight at several layers: tile t at layer l needs tile t at layer l - 1 and tile t - 1 at layer l (its
+// state), so at step s every tile can run layer s - start(t), one layer behind the tile before it.  Each step is three
+// launches (mixer input, scan, feed-forward) over all tiles in flight, instead of three per tile and layer: with few
+// lanes those leave most CUs idle and their latencies add up (1 lane, 8 layers, fp32: 2.6 ms per 64 positions).
+// Every tile in flight has its own rows of the workspace (slot t mod P); a tile starts when its slot is free and the
+// tile before it is one layer ahead.  A row's arithmetic does not depend on the launch it is in, so the results equal
+// the layer-by-layer order's bit for bit.
+//
+// Within a step, a kernel with too few workgroups is cut finer: the mixer input over groups of in_proj chunks (its
+// x_proj partials then folded by the scan), the scan over four threads per channel, the feed-forward and the head over
+// 16 rows instead of 64.  finish(t0, Tc, xin) handles a tile that has passed the last layer.
+// Where the lines lie (compress, ms; d 256 x 8 layers over 704 positions, d 512 x 16 layers bf16w over 320):
+//   PIPE_LANES: against tile after tile on two streams, which from 512 lanes on fills the GPU by itself.  fp32 64 lanes
+//     29.0 -> 8.4, 256: 30.6 -> 26.3, 375: 50.2 -> 39.4, 512: 50.1 -> 50.5; bf16x3 375: 23.6 -> 21.1, 512: 26.4 -> 28.4;
+//     d 512 64: 21.3 -> 8.6, 256: 29.5 -> 28.3, 375: 49.7 -> 40.1, 512: 54.0 -> 53.6.
+//   PIPE_SPLIT: (lane, tile) pairs in a step up to which mixer input and scan are cut finer (1 lane fp32: 4.40 -> 1.96;
+//     16 lanes 5.12 -> 3.31; from 256 pairs on no difference), pipe_quad: up to which the scan is (at d 256 faster or
+//     the same up to 512 pairs; at d 512, whose dt_proj rows are twice as long, 10% slower at 512).
+//   PIPE_ROWS16: 64-row groups in a step up to which feed-forward and head run on 16-row workgroups (16 lanes fp32, 128
+//     groups: 4.02 -> 3.31; more 16-row workgroups than CUs stream the weights more often than they gain).
+//   pipe_two: pairs in flight from which the lanes run as two halves on two streams (fp32 100 lanes 13.2 -> 12.7, 180:
+//     22.3 -> 20.1; 8 lanes 2.37 -> 2.85; d 512 8 lanes 4.09 -> 3.88, 64: 10.2 -> 8.6).
+constexpr int PIPE_SPLIT = 128, PIPE_ROWS16 = 128;
+static int pipe_quad(const boa_ctx* x) { return x->d == ffn5::D ? 128 : 512; }
+static int pipe_two(const boa_ctx* x) { return x->d == ffn5::D ? 64 : 640; }
+static int pipe_depth(const boa_ctx* x, int lanes) {
+    const int64_t fit = x->ws_rows / ((int64_t)lanes * pipe_tile(x->tile_len));
+    return (int)std::max<int64_t>(1, std::min<int64_t>(fit, std::min(x->L, PIPE_MAX)));
+}
+static bool pipe_ok(const boa_ctx* x, int lanes) {
+    return x->pipe && x->ffn_outp && pipe_tile(x->tile_len) >= PIPE_MIN_TILE && lanes <= PIPE_LANES;
+}
+
+// One group of the lanes: lanes lane0 .. lane0 + lanes - 1, its slots from workspace row row0 on, on stream s.
+struct PipeRun {
+    boa_ctx* x;
+    int lanes, len;
+    EmbedIn src;
+    int64_t lane0, row0;
+    hipStream_t s;
+    int TL, n, P, step = 0, first = 0;
+    std::vector<int> start;
+    PipeRun(boa_ctx* c, int lanes_, int len_, const EmbedIn& e, int depth, int64_t l0, hipStream_t st)
+        : x(c), lanes(lanes_), len(len_), src(e), lane0(l0), s(st), TL(pipe_tile(c->tile_len)), n((len_ + TL - 1) / TL),
+          P(std::min(depth, n)), start(n) {
+        row0 = lane0 * depth * TL;
+        if (src.bytes) { src.bytes += lane0 * src.stride; src.lens += lane0; }
+        if (src.tokens) src.tokens += lane0 * src.stride;
+        for (int t = 0; t < n; ++t) {
+            start[t] = t ? start[t - 1] + 1 : 0;
+            if (t >= P) start[t] = std::max(start[t], start[t - P] + x->L);
+        }
+    }
+    bool done() const { return first == n; }
+    template <class Finish> int advance(Finish&& finish);  // launches the next step
+};
+
+template <class Finish>
+int PipeRun::advance(Finish&& finish) {
+    const int L = x->L, d = x->d, di = x->di, NS = x->NS, R = x->R;
+    const bool split = x->prec != BOA_PREC_F32;
+    const int nt = x->prec == BOA_PREC_BF16X3 ? 3 : (split ? 2 : 1);
+    const int64_t pos0 = x->pos;
+    LaneView v(x, 0, lane0, s);
+    MixinTiles ma;
+    ScanTiles sa;
+    FfnTiles fa;
+    ma.e = src;
+    sa.di = di;
+    {
+        int ne = 0;
+        int64_t rows = 0, groups64 = 0, max_m = 0;
+        ma.emb = -1;
+        for (int t = first; t < n && start[t] <= step; ++t, ++ne) {
+            const int l = step - start[t], Tc = std::min(TL, len - t * TL);
+            const int64_t ro = row0 + (int64_t)(t % P) * lanes * TL, M = (int64_t)lanes * Tc;
+            const LayerW& w = x->layers[l];
+            ma.t[ne] = mixin_tile_args(x, l, ro, pos0 + (int64_t)t * TL, Tc);
+            if (l == 0) {
+                ma.emb = ne;
+                ma.e.t0 = src.t0 + t * TL;
+                ma.e.xout = x->x + ro * d;
+            }
+            ScanTile& st = sa.t[ne];
+            st.xs = x->xs + ro * di; st.dbc = x->dbc + ro * (R + 2 * NS); st.xz = x->xz + ro * 2 * di;
+            st.dt_w = w.dt_w; st.dt_b = w.dt_b; st.Aneg = w.Aneg; st.D = w.D;
+            st.ssm = x->ssm + ((int64_t)l * x->max_lanes + lane0) * di * NS;
+            st.yh = split ? x->ah + ro * di : nullptr; st.yl = split ? x->al + ro * di : nullptr;
+            st.Tc = Tc;
+            FfnTile& ft = fa.t[ne];
+            ft.out_b = w.out_b; ft.ln_w = w.ln2_w; ft.ln_b = w.ln2_b; ft.ff1_b = w.ff1_b; ft.ff2_b = w.ff2_b;
+            ft.out_p = w.out_w.p; ft.ff1_p = w.ff1_w.p; ft.ff2_p = w.ff2_w.p;
+            ft.x = x->x + ro * d;
+            ft.yh = split ? st.yh : reinterpret_cast<const uint16_t*>(st.xs);
+            ft.yl = st.yl;
+            ft.M = M;
+            rows += M;
+            groups64 += (M + 63) / 64;
+            max_m = std::max(max_m, M);
+        }
+        const int pairs = lanes * ne, chunks = mixin_chunks(x);
+        int z = 1;
+        if (pairs <= PIPE_SPLIT)
+            while (z < chunks && pairs * z * 2 <= 512) z *= 2;
+        ma.per = chunks / z;
+        sa.parts = z > 1 ? di / XPROJ_KB : 0;
+        PROF(PC_MIXIN, gemm_flops(rows, 2 * di, d) + gemm_flops(rows, R + 2 * NS, di) + 8.0 * rows * di,
+             4.0 * rows * (d + di + di + R + 2 * NS) + 4.0 * 6 * pairs * di, launch_mixin_gen(x, ma, lanes, ne, z, s));
+        const double sflops = (double)rows * di * (2.0 * R + 6.0 * NS + 8.0);
+        const double sbytes = 4.0 * ((double)rows * (3.0 * di + R + 2 * NS) + 2.0 * pairs * di * NS);
+        if (pairs <= pipe_quad(x)) {
+            const dim3 grid((unsigned)(di / 64), (unsigned)lanes, (unsigned)ne);
+            if (R == 16) {
+                if (split) PROF(PC_SCAN, sflops, sbytes, hipLaunchKernelGGL((k_scan_quad<16, true>), grid, dim3(256), 0, s, sa));
+                else PROF(PC_SCAN, sflops, sbytes, hipLaunchKernelGGL((k_scan_quad<16, false>), grid, dim3(256), 0, s, sa));
+            } else {
+                PROF(PC_SCAN, sflops, sbytes, hipLaunchKernelGGL((k_scan_quad<32, true>), grid, dim3(256), 0, s, sa));
+            }
+        } else {
+            const dim3 grid((unsigned)(di / 256), (unsigned)lanes, (unsigned)ne);
+            if (R == 16) {
+                if (split) PROF(PC_SCAN, sflops, sbytes, hipLaunchKernelGGL((k_scan_gen<16, 16, true>), grid, dim3(256), 0, s, sa));
+                else PROF(PC_SCAN, sflops, sbytes, hipLaunchKernelGGL((k_scan_gen<16, 16, false>), grid, dim3(256), 0, s, sa));
+            } else {
+                PROF(PC_SCAN, sflops, sbytes, hipLaunchKernelGGL((k_scan_gen<16, 32, true>), grid, dim3(256), 0, s, sa));
+            }
+        }
+        const double fflops = gemm_flops(rows, d, di) + 2.0 * gemm_flops(rows, 4 * d, d);
+        const double fbytes = 4.0 * rows * di + 4.0 * rows * d * 2;
+        const dim3 g64((unsigned)((max_m + 63) / 64), (unsigned)ne);
+        hipError_t e = hipSuccess;
+        if (d == ffn5::D) {
+            PROF(PC_FFN, fflops, fbytes,
+                 if (nt == 3) hipLaunchKernelGGL((k_ffn512_gen<3>), g64, dim3(512), 0, s, fa);
+                 else hipLaunchKernelGGL((k_ffn512_gen<2>), g64, dim3(512), 0, s, fa));
+        } else if (groups64 <= PIPE_ROWS16) {
+            PROF(PC_FFN, fflops, fbytes, e = launch_ffn16(fa, ne, max_m, nt, s));
+        } else {
+            PROF(PC_FFN, fflops, fbytes,
+                 if (nt == 1) hipLaunchKernelGGL((k_ffn_gen<1>), g64, dim3(512), 0, s, fa);
+                 else if (nt == 3) hipLaunchKernelGGL((k_ffn_gen<3>), g64, dim3(512), 0, s, fa);
+                 else hipLaunchKernelGGL((k_ffn_gen<2>), g64, dim3(512), 0, s, fa));
+        }
+        if (e == hipSuccess) e = hipGetLastError();
+        if (e != hipSuccess) return boa_fail_hip(e, "run_pipe", __FILE__, __LINE__);
+        if (step - start[first] == L - 1) {
+            const int rc = finish(*this, first * TL, std::min(TL, len - first * TL),
+                                  x->x + (row0 + (int64_t)(first % P) * lanes * TL) * d);
+            if (rc) return rc;
+            ++first;
+        }
+        ++step;
+    }
+    return BOA_OK;
+}
+
+// All lanes, in one group or in two halves on two streams (as the classic compress tiles run): one half's scan, head and
+// coder then run beside the other's matrix kernels.
+template <class Finish>
+static int run_pipe(boa_ctx* x, int lanes, int len, const EmbedIn& src, Finish&& finish) {
+    const int depth = pipe_depth(x, lanes);
+    const bool own_head = x->head_xq && (x->V == headq::V || x->d == 256);  // no shared buffers behind the head
+    const bool two = x->stream2 && x->compress_halves && own_head && lanes >= 2 && lanes * depth >= pipe_two(x);
+    const int la = two ? lanes / 2 : lanes;
+    int rc = BOA_OK;
+    if (!two) {
+        PipeRun a(x, lanes, len, src, depth, 0, x->stream);
+        while (!a.done() && !rc) rc = a.advance(finish);
+    } else {
+        hipEvent_t join = x->half_ev[2 * x->L];
+        BOA_HIP_TRY(hipEventRecord(join, x->stream));  // the second half starts after what the stream holds
+        BOA_HIP_TRY(hipStreamWaitEvent(x->stream2, join, 0));
+        PipeRun a(x, la, len, src, depth, 0, x->stream), b(x, lanes - la, len, src, depth, la, x->stream2);
+        while (!a.done() && !rc) {  // the same steps on both
+            rc = a.advance(finish);
+            if (!rc) rc = b.advance(finish);
+        }
+        BOA_HIP_TRY(hipEventRecord(join, x->stream2));
+        BOA_HIP_TRY(hipStreamWaitEvent(x->stream, join, 0));
+    }
+    if (rc) return rc;
+    x->pos += len;
+    return BOA_OK;
+}
+
+static int launch_head_rows(boa_ctx* x, HeadRows h) {
+    h.h1_b = x->h1_b; h.h2_b = x->h2_b; h.h1_p = x->h1_w.p; h.h2_p = x->h2_w.p; h.V = x->V;
+    const int nt = x->prec == BOA_PREC_BF16X3 ? 3 : (x->prec == BOA_PREC_BF16W ? 2 : 1);
+    hipError_t e = hipSuccess;
+    PROF(PC_HEADXQ, gemm_flops(h.M, x->d, x->d) + gemm_flops(h.M, x->V, x->d),
+         4.0 * h.M * x->d + (h.logits ? 4.0 * h.M * x->V : 9.0 * h.M), e = launch_head16(h, nt, x->stream));
+    if (e != hipSuccess) return boa_fail_hip(e, "k_head16", __FILE__, __LINE__);
+    return BOA_OK;
+}
+// whether the head of a tile of run_pipe runs as 16-row workgroups
+static bool head16_ok(const boa_ctx* x, int64_t M) {
+    return x->head_xq && x->d == 256 && ((M + 63) / 64 <= PIPE_ROWS16 || x->V != headq::V);
+}
+static bool head_xq_any(const boa_ctx* x);
+static int launch_head_xq(boa_ctx* x, const float* xin, int lanes, int Tc, int t0, const uint8_t* bytes, int64_t stride,
+                          const int32_t* lens, uint2* lf, float* logits, int64_t len);
+
 extern "C" int boa_model_forward(boa_ctx* x, const int32_t* d_tokens, int64_t tok_stride, int32_t lanes, int32_t len,
                                  float* d_logits) {
     if (!x || !d_tokens || !d_logits || lanes < 1 || lanes > x->max_lanes || len < 0 || tok_stride < len)
         return boa_fail(BOA_ERR_ARG, "boa_model_forward: bad arguments");
+    if (len > 0 && pipe_ok(x, lanes)) {
+        EmbedIn src;
+        src.tokens = d_tokens; src.stride = tok_stride; src.emb = x->emb; src.V = x->V;
+        return run_pipe(x, lanes, len, src, [&](const PipeRun& g, int t0, int Tc, const float* xin) {
+            const int64_t M = (int64_t)g.lanes * Tc;
+            float* out = d_logits + g.lane0 * len * x->V;
+            if (head16_ok(x, M)) {
+                HeadRows h{};
+                h.x = xin; h.M = M; h.t0 = t0; h.Tc = Tc; h.logits = out; h.len = len;
+                return launch_head_rows(x, h);
+            }
+            if (head_xq_any(x)) return launch_head_xq(x, xin, g.lanes, Tc, t0, nullptr, 0, nullptr, nullptr, out, len);
+            const int rc = run_head(x, g.lanes, Tc, x->logits, xin);
+            if (rc) return rc;
+            hipLaunchKernelGGL(k_scatter_logits, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, x->stream, x->logits, x->V, Tc,
+                               t0, len, M, out);
+            BOA_HIP_TRY(hipGetLastError());
+            return (int)BOA_OK;
+        });
+    }
     for (int t0 = 0; t0 < len; t0 += x->tile_len) {
         const int Tc = std::min(x->tile_len, len - t0);
         const int64_t rows = (int64_t)lanes * Tc;
@@ -3374,26 +4005,30 @@ extern "C" int boa_model_forward(boa_ctx* x, const int32_t* d_tokens, int64_t to
     return BOA_OK;
 }
 
-// The fused head + quantiser kernel covers full tiles of 64 positions, vocab 256, d_model 256 (every precision
-// mode) or 512 (split modes), from fragment-packed head weights; other tiles take the head GEMMs and
-// k_encode_tile (same values).
-static bool head_xq_ok(const boa_ctx* x, int Tc) {
-    return x->head_xq && Tc == headq::BM && x->V == headq::V && (x->d == 256 || (x->d == 512 && x->prec != BOA_PREC_F32)) &&
-           x->h1_w.p && x->h2_w.p;
+// The fused head + quantiser kernel covers tiles of up to 64 positions (one workgroup per lane, whatever the tile
+// holds: from tile_min_rows on it is the faster form), vocab 256, d_model 256 (every precision mode) or 512 (split
+// modes), from fragment-packed head weights; other tiles take the head GEMMs and k_encode_tile (same values).
+static bool head_xq_any(const boa_ctx* x) {
+    return x->head_xq && x->V == headq::V && (x->d == 256 || (x->d == 512 && x->prec != BOA_PREC_F32)) && x->h1_w.p &&
+           x->h2_w.p;
 }
+static bool head_xq_ok(const boa_ctx* x, int Tc) { return head_xq_any(x) && Tc <= headq::BM && Tc >= tile_min_rows(x); }
 
-static int launch_head_xq(boa_ctx* x, int lanes, int t0, const uint8_t* bytes, int64_t stride, const int32_t* lens,
-                          uint2* lf) {
+static int launch_head_xq(boa_ctx* x, const float* xin, int lanes, int Tc, int t0, const uint8_t* bytes, int64_t stride,
+                          const int32_t* lens, uint2* lf, float* logits, int64_t len) {
     const int d = x->d, V = x->V;
-    const int64_t M = (int64_t)lanes * headq::BM;
+    const int64_t M = (int64_t)lanes * Tc;
+    const bool gen = Tc < headq::BM || logits;
     const double flops = gemm_flops(M, d, d) + gemm_flops(M, V, d);
     const double bytes_ = 4.0 * M * d + 8.0 * M + (double)M + 2.0 * (x->prec == BOA_PREC_BF16W ? 1 : 2) * (double)(x->h1_w.n + x->h2_w.n);
     const bool three = x->prec == BOA_PREC_BF16X3;
     hipStream_t s = x->stream;
 #define HXQ(NT, D)                                                                                                  \
     PROF(PC_HEADXQ, flops, bytes_,                                                                                  \
-         hipLaunchKernelGGL((k_head_xq<NT, D>), dim3((unsigned)lanes), dim3(512), 0, s, x->x, x->h1_w.p, x->h1_b,    \
-                            x->h2_w.p, x->h2_b, t0, bytes, stride, lens, lf))
+         if (gen) hipLaunchKernelGGL((k_head_xq<NT, D, true>), dim3((unsigned)lanes), dim3(512), 0, s, xin, x->h1_w.p, \
+                                     x->h1_b, x->h2_w.p, x->h2_b, t0, bytes, stride, lens, lf, Tc, logits, len);     \
+         else hipLaunchKernelGGL((k_head_xq<NT, D, false>), dim3((unsigned)lanes), dim3(512), 0, s, xin, x->h1_w.p,  \
+                                 x->h1_b, x->h2_w.p, x->h2_b, t0, bytes, stride, lens, lf, Tc, logits, len))
     if (d == 256) {
         if (x->prec == BOA_PREC_F32) HXQ(1, 256); else if (three) HXQ(3, 256); else HXQ(2, 256);
     } else {
@@ -3415,11 +4050,43 @@ extern "C" int boa_compress(boa_ctx* x, const uint8_t* d_bytes, int64_t byte_str
     hipLaunchKernelGGL(k_enc_init, dim3((lanes + 255) / 256), dim3(256), 0, s, x->enc, lanes);
     BOA_HIP_TRY(hipMemsetAsync(x->flag, 0, sizeof(int32_t), s));
     const int positions = max_len - 1;  // model inputs 0..max_len-2 predict bytes 1..max_len-1
+    const bool piped = positions > 0 && pipe_ok(x, lanes);
+    if (piped) {
+        EmbedIn src;
+        src.bytes = d_bytes; src.stride = byte_stride; src.lens = d_lens; src.emb = x->emb; src.V = x->V;
+        rc = run_pipe(x, lanes, positions, src, [&](const PipeRun& g, int t0, int Tc, const float* xin) {
+            const int64_t M = (int64_t)g.lanes * Tc, b0 = g.lane0;
+            const uint8_t* bytes = d_bytes + b0 * byte_stride;
+            // (lo, width) per position: 8 of the row's V * 4 bytes
+            uint2* lf = reinterpret_cast<uint2*>(x->logits + b0 * g.TL * x->V);
+            int r = BOA_OK;
+            if (head16_ok(x, M)) {
+                HeadRows h{};
+                h.x = xin; h.M = M; h.t0 = t0; h.Tc = Tc; h.bytes = bytes; h.stride = byte_stride; h.lens = d_lens + b0; h.lf = lf;
+                r = launch_head_rows(x, h);
+            } else if (head_xq_any(x)) {
+                r = launch_head_xq(x, xin, g.lanes, Tc, t0, bytes, byte_stride, d_lens + b0, lf, nullptr, 0);
+            } else {
+                r = run_head(x, g.lanes, Tc, x->logits, xin);
+                if (r) return r;
+                PROF(PC_ENCODE, 0.0, 4.0 * M * x->V + (double)M,
+                     hipLaunchKernelGGL(k_encode_tile, dim3(g.lanes), dim3(64), 0, g.s, x->logits, x->V, Tc, t0, bytes,
+                                        byte_stride, d_lens + b0, x->enc + b0, d_words + b0 * pitch_words, pitch_words));
+                return r;
+            }
+            if (r) return r;
+            PROF(PC_ENCODE, 0.0, 8.0 * M + 32.0 * g.lanes,
+                 hipLaunchKernelGGL(k_encode_lf, dim3((g.lanes + 255) / 256), dim3(256), 0, g.s, lf, Tc, g.lanes,
+                                    x->enc + b0, d_words + b0 * pitch_words, pitch_words));
+            return r;
+        });
+        if (rc) return rc;
+    }
     // lane groups: group g holds lanes [lo[g], lo[g + 1]), its rows lo[g] * tile_len rows into the workspace
     const int G = x->stream3 ? 3 : 2;
     int lo[4];
     for (int g = 0; g <= G; ++g) lo[g] = (int)((int64_t)lanes * g / G);
-    const bool halves = x->stream2 && x->compress_halves && lanes >= 256 * G;
+    const bool halves = !piped && x->stream2 && x->compress_halves && lanes >= 256 * G;
     if (halves) {
         // Groups of the lanes on their own streams, each running its layers in order (per layer: the mixer input
         // kernel, the scan, the feed-forward kernel), so that the GPU interleaves the groups' kernels: a
@@ -3457,7 +4124,7 @@ extern "C" int boa_compress(boa_ctx* x, const uint8_t* d_bytes, int64_t byte_str
                 const int64_t b0 = x->lane0, rows = (int64_t)nl * Tc;
                 if (head_xq_ok(x, Tc)) {
                     uint2* lf = reinterpret_cast<uint2*>(x->logits);
-                    rc = launch_head_xq(x, nl, t0, d_bytes + b0 * byte_stride, byte_stride, d_lens + b0, lf);
+                    rc = launch_head_xq(x, x->x, nl, Tc, t0, d_bytes + b0 * byte_stride, byte_stride, d_lens + b0, lf, nullptr, 0);
                     if (rc) return rc;
                     PROF(PC_ENCODE, 0.0, 8.0 * rows + 32.0 * nl,
                          hipLaunchKernelGGL(k_encode_lf, dim3((nl + 255) / 256), dim3(256), 0, x->stream, lf, Tc, nl,
@@ -3479,7 +4146,7 @@ extern "C" int boa_compress(boa_ctx* x, const uint8_t* d_bytes, int64_t byte_str
             BOA_HIP_TRY(hipStreamWaitEvent(s, join[g - 1], 0));
         }
     }
-    for (int t0 = 0; !halves && t0 < positions; t0 += x->tile_len) {
+    for (int t0 = 0; !halves && !piped && t0 < positions; t0 += x->tile_len) {
         const int Tc = std::min(x->tile_len, positions - t0);
         const int64_t rows = (int64_t)lanes * Tc;
         const bool fuse_emb = embed_in_mixin(x, Tc);
@@ -3496,7 +4163,7 @@ extern "C" int boa_compress(boa_ctx* x, const uint8_t* d_bytes, int64_t byte_str
             x->pos += Tc;
             if (rc) return rc;
             uint2* lf = reinterpret_cast<uint2*>(x->logits);  // (lo, width) per position: 8 of the row's V * 4 bytes
-            rc = launch_head_xq(x, lanes, t0, d_bytes, byte_stride, d_lens, lf);
+            rc = launch_head_xq(x, x->x, lanes, Tc, t0, d_bytes, byte_stride, d_lens, lf, nullptr, 0);
             if (rc) return rc;
             PROF(PC_ENCODE, 0.0, 8.0 * rows + 32.0 * lanes,
                  hipLaunchKernelGGL(k_encode_lf, dim3((lanes + 255) / 256), dim3(256), 0, s, lf, Tc, lanes, x->enc,

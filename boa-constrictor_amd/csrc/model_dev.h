@@ -311,6 +311,29 @@ __device__ __forceinline__ float4 logits_row4(const float* row, int V, int lane)
     return l4;
 }
 
+// cumulative of symbol s and its weight, from the owner lane (s uniform across the wave)
+__device__ __forceinline__ void xq_sym(const XQ& q, int s, uint32_t& c_s, uint32_t& f_s) {
+    const int j = s & 3;
+    uint32_t cl = q.base, fl = q.f[0];
+    if (j >= 1) { cl += q.f[0]; fl = q.f[1]; }
+    if (j >= 2) { cl += q.f[1]; fl = q.f[2]; }
+    if (j >= 3) { cl += q.f[2]; fl = q.f[3]; }
+    c_s = wave_bcast(cl, s >> 2);
+    f_s = wave_bcast(fl, s >> 2);
+}
+
+// The coder interval (lo, width) of symbol s under one row of logits held as logits_row4 gives them (whole wavefront).
+__device__ __forceinline__ uint2 xq_interval(const float4 l4, int V, int lane, int s) {
+    XQ q;
+    xq_build(q, l4, lane, V, CODER_P);
+    uint32_t c_s, f_s;
+    xq_sym(q, s, c_s, f_s);
+    const uint32_t lo = xq_cdf_at(q, c_s, s);
+    const uint32_t hi = (s + 1 < V) ? xq_cdf_at(q, c_s + f_s, s + 1) : (1u << CODER_P);
+    return make_uint2(lo, hi - lo);
+}
+constexpr uint32_t LF_SKIP = 0xFFFFFFFFu;  // lo of a position that codes no symbol (past the chunk's end, or byte >= V)
+
 // Chunk b's stream inside a payload of `total` words: words [off[b], off[b] + nwords[b]) clamped to
 // [0, total).  Offsets or counts that do not fit the payload then read zeros, as the decoder reads zeros
 // past the end of any stream, and no word outside the payload is read (the file reader's bound,

@@ -64,6 +64,40 @@ struct FusedArgs {
     float* scr;
 };
 
+// Launches over several tiles at once (a tile: all lanes of a group at Tc consecutive positions, at one layer).
+constexpr int PIPE_MAX = 16;  // tiles per launch at most
+
+// out_proj + LN2 + feed-forward + residual of one tile's M rows.
+struct FfnTile {
+    const float *out_b, *ln_w, *ln_b, *ff1_b, *ff2_b;
+    const uint16_t *out_p, *ff1_p, *ff2_p;
+    float* x;
+    const uint16_t *yh, *yl;  // the scan's output: split parts, or fp32 at yh (fp32 mode)
+    int64_t M;
+};
+struct FfnTiles {
+    FfnTile t[PIPE_MAX];
+};
+// d_model 256, 16 rows per workgroup (fused_step.hip): for launches whose tiles are too few for k_ffn's 64-row workgroups
+hipError_t launch_ffn16(const FfnTiles& a, int tiles, int64_t max_rows, int nt, hipStream_t s);
+
+// Head (Linear -> ReLU -> Linear) of M rows of x, 16 per workgroup (d_model 256): row m is position t0 + m % Tc of lane
+// m / Tc.  Either the coder interval of the byte the position predicts (lf[m]), or the logits (logits[(lane * len + t0 +
+// m % Tc) * V]).
+struct HeadRows {
+    const float *x, *h1_b, *h2_b;
+    const uint16_t *h1_p, *h2_p;
+    int64_t M;
+    int V, t0, Tc;
+    const uint8_t* bytes;
+    int64_t stride;
+    const int32_t* lens;
+    uint2* lf;
+    float* logits;
+    int64_t len;
+};
+hipError_t launch_head16(const HeadRows& a, int nt, hipStream_t s);
+
 // Supported shape of the fused kernel: d_model 256, d_state 16, dt_rank 16, d_conv 4, vocab % 16 == 0.
 bool fused_step_supported(int d_model, int d_state, int dt_rank, int d_conv, int vocab);
 

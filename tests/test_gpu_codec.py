@@ -480,3 +480,64 @@ def test_compress_in_two_halves(gpu, precision):
     out = codec.decompress_payload(m, p0, n0, L0, f0)
     for i, c in enumerate(chunks):
         assert (out[i, :lens[i]] == c).all(), i
+
+
+@pytest.mark.parametrize("d_model,n_layers,precision", [(256, 3, "f32"), (256, 2, "bf16x3"), (256, 17, "bf16w"),
+                                                        (512, 3, "bf16w"), (512, 2, "bf16x3")])
+def test_tiles_in_flight_match_tile_after_tile(gpu, monkeypatch, d_model, n_layers, precision):
+    """Few lanes: launches over several tiles at several layers give the words and logits of one tile and layer at a
+    time, bit for bit: one lane, short and 1-position last tiles, ragged lanes, one and two streams, more layers than
+    tiles in flight, and the finer cuts of each kernel and their limits."""
+    import codec
+    import model as M
+    from boa_amd import weights as W
+
+    blob = W.seeded_blob(W.Cfg(d_model=d_model, n_layers=n_layers), 3)
+    shapes = [(1, 17), (2, 65), (3, 66), (1, 67), (5, 130), (9, 331), (70, 200), (200, 131)]
+    got = {}
+    for pipe in ("0", "1"):
+        monkeypatch.setenv("BOA_PIPE", pipe)
+        rng = np.random.default_rng(4)
+        for n, length in shapes:
+            m = M.BoaConstrictor(d_model, n_layers, 256).load_blob(blob)
+            m.precision = precision
+            chunks = [rng.integers(0, 256, length if i % 4 == 0 else int(rng.integers(1, length + 1))).astype(np.uint8)
+                      for i in range(n)]
+            payload, nw, fb, Ls = codec.compress_payload(m, chunks)
+            tok = torch.from_numpy(rng.integers(0, 256, (n, length))).cuda()
+            got[pipe, n, length] = (payload, nw, m.forward(tok).cpu())
+            if pipe == "1":
+                out = codec.decompress_payload(m, payload, nw, Ls, fb)
+                assert all((out[i, :Ls[i]] == c).all() for i, c in enumerate(chunks)), (n, length)
+    for n, length in shapes:
+        a, b = got["0", n, length], got["1", n, length]
+        assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]), (n, length)
+        assert torch.equal(a[2], b[2]), (n, length)
+
+
+@pytest.mark.parametrize("d_model,precision", [(256, "f32"), (256, "bf16x3"), (512, "bf16w")])
+@pytest.mark.parametrize("split", [1, 2, 3, 64, 65, 130])
+def test_forward_in_pieces_and_steps(gpu, d_model, precision, split):
+    """The state that the tiles in flight leave (conv history ring, SSM state, position) continues: a forward over
+    `split` positions, one over the rest, then single steps equal one forward over everything, bit for bit."""
+    from boa_amd import weights as W
+    from model import _Engine
+
+    cfg = W.Cfg(d_model=d_model, n_layers=3)
+    B, T = 3, 150
+    eng = _Engine(W.seeded_blob(cfg, 5), cfg, B, 64, precision)
+    tok = torch.from_numpy(np.random.default_rng(6).integers(0, 256, (B, T)).astype(np.int32)).cuda()
+    whole = torch.empty((B, T, 256), device="cuda")
+    eng.reset(B)
+    eng.forward(tok, whole)
+    eng.reset(B)
+    parts = []
+    for lo, hi in ((0, split), (split, T - 4)):
+        out = torch.empty((B, hi - lo, 256), device="cuda")
+        eng.forward(tok[:, lo:hi].contiguous(), out)
+        parts.append(out)
+    for t in range(T - 4, T):
+        out = torch.empty((B, 256), device="cuda")
+        eng.step(tok[:, t].contiguous(), out)
+        parts.append(out[:, None])
+    assert torch.equal(torch.cat(parts, 1), whole)
