@@ -2762,6 +2762,11 @@ struct boa_ctx {
     // ws_rows: rows of x, xz, xs, dbc and the split activations (every tile in flight has its own)
     bool pipe = true;
     int64_t ws_rows = 0;
+    // decode steps with several workgroups per 16 lanes (BOA_GROUP_STEP=0: the fused kernels only)
+    uint64_t* xch = nullptr;
+    int32_t* xbad = nullptr;
+    uint32_t xseq = 1;                 // the next sequence number of an exchange packet
+    int cus = 0;
     hipStream_t stream2 = nullptr;
     hipStream_t stream3 = nullptr;     // the third compress group's
     std::vector<hipEvent_t> half_ev;   // [2][L]: state group of layer l done, per half; [2L], [2L + 1]: stream joins
@@ -2884,6 +2889,13 @@ static bool f32_packed(const boa_model_cfg& c, int R, int precision) {
     return precision == BOA_PREC_F32 && fused_step_supported(c.d_model, c.d_state, R, c.d_conv, c.vocab);
 }
 
+static bool want_fused(const boa_model_cfg& c, int R, int precision);
+// Whether a context of this shape gets the exchange buffer of group_step.hip.
+static bool want_group(const boa_model_cfg& c, int R, int precision) {
+    const char* env = getenv("BOA_GROUP_STEP");
+    return want_fused(c, R, precision) && c.vocab == 256 && !(env && env[0] == '0');
+}
+
 static bool want_fused(const boa_model_cfg& c, int R, int precision) {
     const char* fenv = getenv("BOA_FUSED_STEP");
     const bool d256 = fused_step_supported(c.d_model, c.d_state, R, c.d_conv, c.vocab);
@@ -2933,6 +2945,7 @@ static int64_t ctx_plan_bytes(const boa_model_cfg& c, int R, int precision, int6
         b += 2 * std::max<int64_t>(2 * mats, 1);  // fp32 fragment-packed weights, in 16-bit units
     }
     if (want_fused(c, R, precision)) b += (int64_t)sizeof(FusedLayer) * L;
+    if (want_group(c, R, precision)) b += group_step_bytes(c.d_model, max_lanes) + (int64_t)sizeof(int32_t);
     return b;
 }
 
@@ -2955,7 +2968,7 @@ extern "C" int boa_ctx_destroy(boa_ctx* ctx) {
     else (void)hipDeviceSynchronize();
     void* ptrs[] = {ctx->wblob, ctx->aneg, ctx->conv_hist, ctx->ssm, ctx->x, ctx->xz, ctx->xs, ctx->dbc,
                     ctx->mm, ctx->logits, ctx->stats, ctx->tokens, ctx->enc, ctx->dec, ctx->flag, ctx->wsplit,
-                    ctx->ah, ctx->al, ctx->wfrag, ctx->d_layers};
+                    ctx->ah, ctx->al, ctx->wfrag, ctx->d_layers, ctx->xch, ctx->xbad};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& p : ctx->prof)
@@ -3179,6 +3192,16 @@ extern "C" int boa_ctx_create(const boa_model_cfg* cfg, const void* h_weights, i
         }
     }
     if (e == hipSuccess && x->fused) e = dmalloc(x, &x->d_layers, (int64_t)L);
+    if (e == hipSuccess && want_group(c, R, x->prec)) {
+        const int64_t n = group_step_bytes(c.d_model, max_lanes) / 8;
+        int dev = 0;
+        e = dmalloc(x, &x->xch, n);
+        if (e == hipSuccess) e = dmalloc(x, &x->xbad, 1);
+        if (e == hipSuccess) e = hipMemsetAsync(x->xch, 0, (size_t)n * 8, x->stream);  // sequence number 0: none
+        if (e == hipSuccess) e = hipMemsetAsync(x->xbad, 0, sizeof(int32_t), x->stream);
+        if (e == hipSuccess) e = hipGetDevice(&dev);
+        if (e == hipSuccess) e = hipDeviceGetAttribute(&x->cus, hipDeviceAttributeMultiprocessorCount, dev);
+    }
     if (e != hipSuccess) {
         boa_ctx_destroy(x);
         return boa_fail_hip(e, "boa_ctx_create allocation", __FILE__, __LINE__);
@@ -3718,8 +3741,22 @@ static FusedArgs fused_args(boa_ctx* x, int32_t lanes, const int32_t* tokens_in)
     return a;
 }
 
-static hipError_t launch_fused(const boa_ctx* x, const FusedArgs& a, hipStream_t s) {
+static hipError_t launch_fused(boa_ctx* x, FusedArgs& a, hipStream_t s) {
     const int nt = x->prec == BOA_PREC_BF16X3 ? 3 : (x->prec == BOA_PREC_BF16W ? 2 : 1);
+    const int g = x->xch ? group_step_width(x->d, a.B, x->cus) : 1;
+    if (g > 1) {
+        // a stream that is being captured takes the fused kernel: replays would repeat the sequence numbers
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+            (void)hipGetLastError();
+            cap = hipStreamCaptureStatusActive;
+        }
+        if (cap == hipStreamCaptureStatusNone) {
+            a.xch = x->xch; a.bad = x->xbad; a.seq0 = x->xseq;
+            x->xseq += 1u + (uint32_t)a.nsteps * (uint32_t)(x->L + 1);
+            return launch_group_step(a, x->d, nt, g, s);
+        }
+    }
     return x->d == 512 ? launch_fused_step512(a, nt, s) : launch_fused_step(a, nt, s);
 }
 
@@ -4215,7 +4252,10 @@ extern "C" int boa_decompress(boa_ctx* x, const uint32_t* d_payload, int64_t pay
             if (e != hipSuccess) return boa_fail_hip(e, "k_fused_step", __FILE__, __LINE__);
             x->pos += a.nsteps;
         }
+        int32_t bad = 0;
+        if (x->xbad) BOA_HIP_TRY(hipMemcpyAsync(&bad, x->xbad, sizeof(int32_t), hipMemcpyDeviceToHost, s));
         BOA_HIP_TRY(hipStreamSynchronize(s));
+        if (bad) return boa_fail(BOA_ERR_HIP, "boa_decompress: a wait between workgroups expired");
         return BOA_OK;
     }
     if (x->stream2 && lanes >= 512) {

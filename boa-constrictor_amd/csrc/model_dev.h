@@ -351,12 +351,13 @@ __device__ __forceinline__ LaneWords lane_words(const uint32_t* payload, int64_t
     return {payload + o, (int32_t)n};
 }
 
-// One decode step of one lane (whole wavefront): quantise the logits (XQ), find the symbol the coder state
+// One decode step of one lane (whole wavefront), its logits held as logits_row4 gives them (decode_row: in memory):
+// quantise the logits (XQ), find the symbol the coder state
 // points into, advance the state.  Returns the symbol (uniform across the wave).
-__device__ __forceinline__ int decode_row(const float* row, int V, int lane, DecState& st, const uint32_t* in,
-                                          int32_t nw) {
+__device__ __forceinline__ int decode_l4(const float4 l4, int V, int lane, DecState& st, const uint32_t* in,
+                                         int32_t nw) {
     XQ q;
-    xq_build(q, logits_row4(row, V, lane), lane, V, CODER_P);
+    xq_build(q, l4, lane, V, CODER_P);
     uint32_t e[4];
     uint32_t c = q.base;
 #pragma unroll
@@ -370,6 +371,10 @@ __device__ __forceinline__ int decode_row(const float* row, int V, int lane, Dec
     const int s = wave_find_symbol<CODER_P>(e, V, qv, lane, lo, hi);
     dec_advance(st, CODER_P, lo, hi - lo, in, nw);
     return s;
+}
+__device__ __forceinline__ int decode_row(const float* row, int V, int lane, DecState& st, const uint32_t* in,
+                                          int32_t nw) {
+    return decode_l4(logits_row4(row, V, lane), V, lane, st, in, nw);
 }
 
 }  // namespace boa

@@ -62,6 +62,11 @@ struct FusedArgs {
     // d_model 512 kernel only: per-lane scratch in device memory (the context's workspace rows, row = lane): the
     // mixer's z | conv output [lanes][2 d_inner]
     float* scr;
+    // group_step.hip only: the exchange packets, the first sequence number of this launch, and where an expired wait is
+    // reported
+    uint64_t* xch;
+    uint32_t seq0;
+    int32_t* bad;
 };
 
 // Launches over several tiles at once (a tile: all lanes of a group at Tc consecutive positions, at one layer).
@@ -108,5 +113,12 @@ hipError_t launch_fused_step(const FusedArgs& a, int nt, hipStream_t s);
 // workgroup of 32 lanes, one workgroup per CU (256 VGPRs per thread, 145 KB of LDS with the residual stream).
 bool fused_step512_supported(int d_model, int d_state, int dt_rank, int d_conv, int vocab);
 hipError_t launch_fused_step512(const FusedArgs& a, int nt, hipStream_t s);
+
+// Decode steps with several workgroups per 16 lanes (group_step.hip): vocab 256, otherwise the fused kernels' shapes.
+constexpr int GROUP_MAX = 128;  // groups of 16 lanes at most
+int64_t group_step_bytes(int d_model, int64_t max_lanes);     // exchange packets, in bytes
+int group_step_width(int d_model, int lanes, int cus);         // workgroups per group on a GPU of that many CUs; 1: none
+// takes 1 + nsteps (L + 1) sequence numbers from a.seq0 on; a cooperative launch
+hipError_t launch_group_step(const FusedArgs& a, int d_model, int nt, int g, hipStream_t s);
 
 }  // namespace boa

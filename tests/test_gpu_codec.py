@@ -541,3 +541,60 @@ def test_forward_in_pieces_and_steps(gpu, d_model, precision, split):
         eng.step(tok[:, t].contiguous(), out)
         parts.append(out[:, None])
     assert torch.equal(torch.cat(parts, 1), whole)
+
+
+@pytest.mark.parametrize("d_model,precision,lanes", [
+    (256, "f32", (1, 15, 17, 130, 513, 1100)), (256, "bf16x3", (3, 512, 1024, 1025)), (256, "bf16w", (33, 600, 2048)),
+    (512, "bf16w", (1, 20, 129, 300, 1000, 1500)), (512, "bf16x3", (16, 257, 513, 1025))])
+def test_group_step_matches_fused_kernels(gpu, monkeypatch, d_model, precision, lanes):
+    """Decode steps with several workgroups per 16 lanes (every group width, partly filled and single groups) give the
+    fused kernels' logits and decoded bytes, bit for bit; ragged lanes, and a payload that ends early (zeros)."""
+    import codec
+    import model as M
+    from boa_amd import weights as W
+
+    blob = W.seeded_blob(W.Cfg(d_model=d_model, n_layers=2), 7)
+    for n in lanes:
+        got = {}
+        for group in ("0", "1"):
+            monkeypatch.setenv("BOA_GROUP_STEP", group)
+            rng = np.random.default_rng(n)
+            m = M.BoaConstrictor(d_model, 2, 256).load_blob(blob)
+            m.precision = precision
+            inf = m.init_stream(max_len=8, batch_size=n)
+            logits = [m.step(torch.from_numpy(rng.integers(0, 256, n).astype(np.int32)).cuda(), inf).cpu() for _ in range(4)]
+            lens = [int(v) for v in rng.integers(1, 20, n)]
+            nw = rng.integers(0, 9, n)
+            payload = rng.integers(0, 1 << 32, int(nw.sum()), dtype=np.uint64).astype(np.uint32)
+            out = codec.decompress_payload(m, payload, nw, lens, rng.integers(0, 256, n).tolist())
+            got[group] = (logits, np.concatenate([out[i, :L] for i, L in enumerate(lens)]))
+        assert all(torch.equal(a, b) for a, b in zip(got["0"][0], got["1"][0])), n
+        assert np.array_equal(got["0"][1], got["1"][1]), n
+
+
+def test_step_under_capture(gpu):
+    """A step recorded into a graph (which cannot hold the group kernel's sequence numbers) replays as the eager step
+    from the same state."""
+    from boa_amd import weights as W
+    from model import _Engine
+
+    cfg = W.Cfg(n_layers=2)
+    tok = torch.tensor([3, 200, 7], dtype=torch.int32, device="cuda")
+    out, ref = (torch.zeros((3, 256), device="cuda") for _ in range(2))
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        eng = _Engine(W.seeded_blob(cfg, 1), cfg, 3, 1, "f32")
+        eng.reset(3)
+        eng.step(tok, ref)
+        eng.reset(3)
+        s.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            eng.step(tok, out)
+        for _ in range(3):
+            eng.reset(3)
+            out.zero_()
+            g.replay()
+            s.synchronize()
+            assert torch.equal(out, ref)
