@@ -245,6 +245,7 @@ typedef __attribute__((address_space(4))) const FusedArgs KArgs;
 // is x_proj's K block w (XPROJ_KB).
 template <int NT, int NTHR>
 __global__ void __launch_bounds__(NTHR) k_fused_step(FusedArgs a) {
+    if (left_out(a)) return;
     constexpr int NWAVE = NTHR / 64;
     constexpr int RPW = ROWS / NWAVE;               // rows per wave (LN, decode)
     // fragments per wave and pass, N = 1024 GEMMs (in_proj, FF1): 4 in the split forms (two passes); 8 in the fp32

@@ -140,6 +140,7 @@ __global__ void __launch_bounds__(NTHR, 1) k_fused_step512(FusedArgs a0) {
     float* sF = reinterpret_cast<float*>(lds);  // fp32 view of the operand buffer
     float* sRes = reinterpret_cast<float*>(lds + SZ_A + SZ_C);  // residual stream [ROWS][LRS]
 
+    if (left_out(a0)) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t b0 = (int64_t)blockIdx.x * ROWS;

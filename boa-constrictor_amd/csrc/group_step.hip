@@ -28,10 +28,13 @@
 // between): no packet is overwritten before all have read it.  Sequence numbers grow over the context's life, so what
 // earlier launches left never matches.
 //
-// All members of a group have to be resident at once: the launch is cooperative, with at most one workgroup per CU.  With
-// more groups than CUs / 2 the fused kernels, one workgroup per group, fill the GPU and have no exchange.
-// Waits are bounded (WAIT_TICKS): if one expires, the workgroup stops waiting for good, reports it in *bad, and gives
-// NaN logits.
+// All workgroups have to be resident at once (at most one per CU).  They meet at a gate first, before anything is read or
+// written: the last to arrive opens it; the first to find its time up (another kernel holds the CUs) closes it for this
+// launch, all of them leave, and the fused launch that follows does the work (left_out).  Beyond the gate every wait ends
+// because its partners run.  (A cooperative launch gives the same guarantee but took 80 us longer per launch, of a step's
+// 187.)  The waits are bounded all the same (WAIT_TICKS): if one expires, the workgroup stops waiting for good, reports it
+// in *bad, and gives NaN logits.  With more groups than CUs / 2 the fused kernels, one workgroup per group, fill the GPU
+// and have no exchange.
 //
 // Arithmetic: every GEMM output accumulates its K steps in ascending order through mfma_split_step_t, x_proj is the left
 // fold of 64-channel partials, and every elementwise step is the shared function of model_dev.h, as in the fused and
@@ -335,7 +338,7 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
     __shared__ __attribute__((aligned(16))) float sDbc[ROWS * FW];
     __shared__ floatx4 sAcc[NWAVE * 64 / 2];
     __shared__ int sTok[ROWS];
-    __shared__ int sDead, sMaxLen;
+    __shared__ int sDead, sMaxLen, sGo;
     float* sXZ = reinterpret_cast<float*>(op + OFF_XZ);
     unsigned char* sCv = op + OFF_CV;
 
@@ -346,6 +349,29 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
     if (b0 >= a0.B) return;
     const int nb = (int)((a0.B - b0) < ROWS ? (a0.B - b0) : ROWS);
     volatile int* dead = &sDead;
+    // ---- the gate
+    if (threadIdx.x == 0) {
+        const uint64_t open = 2ull * a0.seq0, shut = open + 1ull;
+        const uint64_t total = (uint64_t)((a0.B + ROWS - 1) / ROWS) * G;
+        uint64_t* const gate = a0.gate;
+        auto state = [&]() { return __hip_atomic_load(gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+        // the first to decide for this launch: `was` holds an earlier launch's decision
+        auto decide = [&](uint64_t was, uint64_t how) {
+            if (was != open && was != shut)
+                __hip_atomic_compare_exchange_strong(gate, &was, how, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        const uint64_t n = __hip_atomic_fetch_add(gate + 1, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        uint64_t st = state();
+        if (n - a0.arrived == total - 1) decide(st, open);
+        const uint64_t t0 = wall_clock64();
+        while (st != open && st != shut) {
+            st = state();
+            if (wall_clock64() - t0 > a0.gate_ticks) decide(st, shut);
+        }
+        sGo = st == open ? 1 : 0;
+    }
+    __syncthreads();
+    if (!sGo) return;
     {
         const int tid = (int)threadIdx.x;
         if (tid < ROWS) sTok[tid] = tid < nb ? a0.tokens_in[b0 + tid] : 0;
@@ -821,10 +847,8 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
 
 template <int NT, int D, int G>
 hipError_t launch(const FusedArgs& a, hipStream_t s) {
-    FusedArgs args = a;
-    void* p[] = {&args};
-    return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&k_group_step<NT, D, G>),
-                                      dim3((unsigned)((a.B + 8 * ROWS - 1) / (8 * ROWS) * 8 * G)), dim3(NTHR), p, 0, s);
+    hipLaunchKernelGGL((k_group_step<NT, D, G>), dim3((unsigned)((a.B + 8 * ROWS - 1) / (8 * ROWS) * 8 * G)), dim3(NTHR), 0, s, a);
+    return hipGetLastError();
 }
 template <int NT, int D>
 hipError_t launch_g(const FusedArgs& a, int g, hipStream_t s) {
@@ -850,6 +874,8 @@ int group_step_width(int d_model, int lanes, int cus) {
         if ((groups + 7) / 8 * 8 * g <= cus) return g;
     return 1;
 }
+
+int64_t group_step_blocks(int lanes, int g) { return (int64_t)((lanes + ROWS - 1) / ROWS) * g; }
 
 hipError_t launch_group_step(const FusedArgs& a, int d_model, int nt, int g, hipStream_t s) {
     if (d_model == 512) return nt == 3 ? launch_g<3, 512>(a, g, s) : launch_g<2, 512>(a, g, s);

@@ -2765,6 +2765,9 @@ struct boa_ctx {
     // decode steps with several workgroups per 16 lanes (BOA_GROUP_STEP=0: the fused kernels only)
     uint64_t* xch = nullptr;
     int32_t* xbad = nullptr;
+    uint64_t* xgate = nullptr;         // where a group launch's workgroups meet: [decisions, arrivals]
+    uint64_t xarrived = 0;             // arrivals so far
+    bool group_shut = false;           // BOA_GROUP_STEP=shut: the gate never opens (tests of the launch that then follows)
     uint32_t xseq = 1;                 // the next sequence number of an exchange packet
     int cus = 0;
     hipStream_t stream2 = nullptr;
@@ -2945,7 +2948,7 @@ static int64_t ctx_plan_bytes(const boa_model_cfg& c, int R, int precision, int6
         b += 2 * std::max<int64_t>(2 * mats, 1);  // fp32 fragment-packed weights, in 16-bit units
     }
     if (want_fused(c, R, precision)) b += (int64_t)sizeof(FusedLayer) * L;
-    if (want_group(c, R, precision)) b += group_step_bytes(c.d_model, max_lanes) + (int64_t)sizeof(int32_t);
+    if (want_group(c, R, precision)) b += group_step_bytes(c.d_model, max_lanes) + (int64_t)sizeof(int32_t) + 8 * GROUP_GATE_WORDS;
     return b;
 }
 
@@ -2968,7 +2971,7 @@ extern "C" int boa_ctx_destroy(boa_ctx* ctx) {
     else (void)hipDeviceSynchronize();
     void* ptrs[] = {ctx->wblob, ctx->aneg, ctx->conv_hist, ctx->ssm, ctx->x, ctx->xz, ctx->xs, ctx->dbc,
                     ctx->mm, ctx->logits, ctx->stats, ctx->tokens, ctx->enc, ctx->dec, ctx->flag, ctx->wsplit,
-                    ctx->ah, ctx->al, ctx->wfrag, ctx->d_layers, ctx->xch, ctx->xbad};
+                    ctx->ah, ctx->al, ctx->wfrag, ctx->d_layers, ctx->xch, ctx->xbad, ctx->xgate};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& p : ctx->prof)
@@ -3197,6 +3200,8 @@ extern "C" int boa_ctx_create(const boa_model_cfg* cfg, const void* h_weights, i
         int dev = 0;
         e = dmalloc(x, &x->xch, n);
         if (e == hipSuccess) e = dmalloc(x, &x->xbad, 1);
+        if (e == hipSuccess) e = dmalloc(x, &x->xgate, GROUP_GATE_WORDS);
+        if (e == hipSuccess) e = hipMemsetAsync(x->xgate, 0, 8 * GROUP_GATE_WORDS, x->stream);
         if (e == hipSuccess) e = hipMemsetAsync(x->xch, 0, (size_t)n * 8, x->stream);  // sequence number 0: none
         if (e == hipSuccess) e = hipMemsetAsync(x->xbad, 0, sizeof(int32_t), x->stream);
         if (e == hipSuccess) e = hipGetDevice(&dev);
@@ -3232,6 +3237,7 @@ extern "C" int boa_ctx_create(const boa_model_cfg* cfg, const void* h_weights, i
         boa_ctx_destroy(x);
         return boa_fail_hip(e, "boa_ctx_create upload", __FILE__, __LINE__);
     }
+    if (const char* v = getenv("BOA_GROUP_STEP")) x->group_shut = strcmp(v, "shut") == 0;
     if (const char* v = getenv("BOA_DECODE_HALVES")) x->decode_halves = atoi(v) == 1 ? 1 : 2;
     if (const char* v = getenv("BOA_FFN_OUTP")) x->ffn_outp = atoi(v) != 0;
     if (const char* v = getenv("BOA_HEAD_XQ")) x->head_xq = atoi(v) != 0;
@@ -3744,6 +3750,7 @@ static FusedArgs fused_args(boa_ctx* x, int32_t lanes, const int32_t* tokens_in)
 static hipError_t launch_fused(boa_ctx* x, FusedArgs& a, hipStream_t s) {
     const int nt = x->prec == BOA_PREC_BF16X3 ? 3 : (x->prec == BOA_PREC_BF16W ? 2 : 1);
     const int g = x->xch ? group_step_width(x->d, a.B, x->cus) : 1;
+    a.only_if = 0;
     if (g > 1) {
         // a stream that is being captured takes the fused kernel: replays would repeat the sequence numbers
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -3752,9 +3759,13 @@ static hipError_t launch_fused(boa_ctx* x, FusedArgs& a, hipStream_t s) {
             cap = hipStreamCaptureStatusActive;
         }
         if (cap == hipStreamCaptureStatusNone) {
-            a.xch = x->xch; a.bad = x->xbad; a.seq0 = x->xseq;
+            a.xch = x->xch; a.bad = x->xbad; a.seq0 = x->xseq; a.gate = x->xgate; a.arrived = x->group_shut ? ~0ull : x->xarrived;
+            a.gate_ticks = 50000u + 5000u * (uint32_t)a.nsteps;  // 0.5 ms and 50 us per step
+            const hipError_t e = launch_group_step(a, x->d, nt, g, s);
+            if (e != hipSuccess) return e;
             x->xseq += 1u + (uint32_t)a.nsteps * (uint32_t)(x->L + 1);
-            return launch_group_step(a, x->d, nt, g, s);
+            x->xarrived += (uint64_t)group_step_blocks(a.B, g);
+            a.only_if = 2ull * a.seq0 + 1ull;  // then the fused launch, which leaves if the group launch ran
         }
     }
     return x->d == 512 ? launch_fused_step512(a, nt, s) : launch_fused_step(a, nt, s);
