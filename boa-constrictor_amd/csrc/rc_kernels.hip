@@ -97,9 +97,9 @@ constexpr int DPP_HALF_MIRROR = 0x141; // row_half_mirror: lane i <- lane 7 - i 
 constexpr int DPP_SHR1 = 0x111;        // row_shr:1: lane i <- lane i - 1 within each 16 lanes
 constexpr int DPP_MIRROR = 0x140;      // row_mirror: lane i <- lane 15 - i within each 16 lanes
 
-// The same coder for full tables (K = 256) in any table format, lengths divisible by D: four streams per
-// wavefront, 16 lanes per stream, lane j holding entries 16 j .. 16 j + 15 of each row (a row of one stream is
-// one contiguous 512 B (2-byte entries) or 1 KiB (4-byte entries) read by its 16 lanes).  The scaffolding is
+// The same coder for full tables (K = 256) in any table format and of any length: four streams per wavefront, 16 lanes
+// per stream, lane j holding entries 16 j .. 16 j + 15 of each row (a row of one stream is one contiguous 512 B
+// (2-byte entries) or 1 KiB (4-byte entries) read by its 16 lanes).  The scaffolding is
 // k_rc_decode_tables8's (below): rows through a non-temporal register ring D - 1 steps ahead, code words from a
 // three-block register window moved once per pass, symbols stored once per pass, no memory access under a
 // branch.  The coder arithmetic is the reference's (rc_core.h: dec_target, and dec_advance's update with its
@@ -225,12 +225,17 @@ __global__ void __launch_bounds__(256) k_rc_decode_tables4(const TC* __restrict_
             st.point = sh ? (st.point << 32) | (uint64_t)wa : st.point;
             st.read_idx += (sh && st.read_idx < nw) ? 1 : 0;
         }
-        __builtin_amdgcn_raw_buffer_store_b32(packed, rs, sbase + (uint32_t)t0, 0, 0);
+        // lane u < D stores the pass's symbol u; the steps of a last pass past the stream's end (they decode its last
+        // row again) take an offset past the array's end, which drops the store
+        const int tj = t0 + j;
+        const bool put = j < D && tj < len;
+        __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(packed >> (8 * (j & (D - 1)))), rs,
+                                             put ? sbase + (uint32_t)tj : 0xFFFFFFF0u, 0, 0);
     }
 }
 
 
-// The table decoder for 2-byte tables at P = 16 (configs[1]'s coder), K = 256, lengths divisible by D: eight
+// The table decoder for 2-byte tables at P = 16, K = 256, any length: eight
 // lanes per stream, so eight streams per wavefront and half the instructions per decoded symbol of the
 // four-streams form above.  Lane j of a stream holds entries 64 v + 8 j .. + 7 (v = 0..3) of each row, so each
 // of its four 16-byte loads is, over the stream's eight lanes, one contiguous 128-byte line of the row; rows
@@ -244,15 +249,17 @@ __global__ void __launch_bounds__(256) k_rc_decode_tables4(const TC* __restrict_
 //  - the symbol is that index minus one (the reference's linear search, gpu_range_coder.py:195-199), and the
 //    coder update is dec_advance's (rc_core.h), its renormalisation word read from the register window before
 //    the search (the window's first half always holds it: the read position stays within S words of its base).
-// The D symbols of a pass are stored as one D-byte word.
-template <int D>
+// WHOLE (lengths divisible by 8, 8-byte aligned symbols): the symbols of a pass are stored as one word; otherwise by the
+// stream's eight lanes, a byte each, and a last pass of fewer symbols decodes its last row again for the steps past the
+// end and stores nothing for them (one wavefront per stream took 4583 us for 16384 x 1023, this 1406: 4.3 GB of table
+// rows at 3.1 TB/s).
+template <int D, bool WHOLE>
 __global__ void __launch_bounds__(256) k_rc_decode_tables8(const uint16_t* __restrict__ cdf,
                                                          const uint32_t* __restrict__ words, int64_t pitch,
                                                          const int32_t* __restrict__ nwords, int streams, int len,
                                                          uint8_t* __restrict__ syms, uint32_t words_bytes) {
     constexpr int P = 16, K = 256, S = 8, NV = 4, E = 32;  // lanes per stream, 16-byte loads and entries per lane
-    static_assert(D == 4 || D == 8, "symbols of a pass are stored as one 4- or 8-byte word");
-    using SymWord = typename std::conditional<D == 8, uint64_t, uint32_t>::type;
+    static_assert(D == S, "a lane per symbol of a pass; at most S words are read per pass");
     const int lane = threadIdx.x & 63;
     const int j = lane & (S - 1), gbase = lane & ~(S - 1);
     const int64_t n = ((int64_t)blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6)) * (64 / S) + lane / S;
@@ -312,7 +319,7 @@ __global__ void __launch_bounds__(256) k_rc_decode_tables8(const uint16_t* __res
         w1 = rot ? w2 : w1;
         base += rot ? S : 0;
         w2 = word(base + 2 * S + j);
-        SymWord packed = 0;
+        uint64_t packed = 0;
 #pragma unroll
         for (int u = 0; u < D; ++u) {
             load_row(t0 + u + D - 1, rows[(u + D - 1) % D]);
@@ -352,7 +359,7 @@ __global__ void __launch_bounds__(256) k_rc_decode_tables8(const uint16_t* __res
             vv |= dpp<DPP_HALF_MIRROR>(vv);
             const uint32_t lo = vv & 0xFFFFu;
             const uint32_t hi = kl < K ? vv >> 16 : (1u << P);
-            packed |= (SymWord)(uint8_t)(kl - 1) << (8 * u);
+            packed |= (uint64_t)(uint8_t)(kl - 1) << (8 * u);
             // dec_advance (rc_core.h), one renormalisation at most (the range is >= 2^32 before every step)
             uint32_t prob = hi - lo;
             if (prob == 0u) prob = 1u;
@@ -365,67 +372,105 @@ __global__ void __launch_bounds__(256) k_rc_decode_tables8(const uint16_t* __res
             st.point = sh ? (st.point << 32) | (uint64_t)wa : st.point;
             st.read_idx += (sh && st.read_idx < nw) ? 1 : 0;
         }
-        // the stream's eight lanes store the same word (one write)
-        if constexpr (D == 8)
+        if constexpr (WHOLE) {
             __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2v, packed), rs, sbase + (uint32_t)t0, 0, 0);
-        else
-            __builtin_amdgcn_raw_buffer_store_b32(packed, rs, sbase + (uint32_t)t0, 0, 0);
+        } else {
+            const int tj = t0 + j;
+            __builtin_amdgcn_raw_buffer_store_b8((uint8_t)((j < 4 ? (uint32_t)packed : (uint32_t)(packed >> 32)) >> (8 * (j & 3))),
+                                                 rs, tj < len ? sbase + (uint32_t)tj : 0xFFFFFFF0u, 0, 0);
+        }
     }
+}
+
+// DPP row_newbcast within halves of a row: every lane <- lane U of its own 8 lanes.
+template <int U>
+__device__ __forceinline__ uint32_t bcast8(uint32_t v) {
+    const int low = __builtin_amdgcn_update_dpp((int)v, (int)v, 0x150 + U, 0xF, 0x3, false);
+    return (uint32_t)__builtin_amdgcn_update_dpp(low, (int)v, 0x158 + U, 0xF, 0xC, false);
 }
 
 constexpr int ENC_LANES_PER_STREAM = 8;
 
-// Encoder on full tables (K = 256), streams of a length divisible by 16: R lanes per stream, all computing the
-// stream's coder state and the first of them writing its words, so that there are R times as many wavefronts
-// as with one lane per stream (a wavefront's symbols are a sequential chain of dependent steps; more wavefronts
-// per SIMD hide more of its latency; 8 lanes measured 12% faster than 1).  The table entries of 16 symbols
-// (independent of the coder state) are loaded one block ahead, non-temporal (6% faster: each is read once), the
-// symbols two blocks ahead, so enc_push (rc_core.h) runs without waiting on memory.
-template <int P, typename TC, int R>
-__global__ void __launch_bounds__(64) k_rc_encode_tables16(const TC* __restrict__ cdf,
-                                                         const uint8_t* __restrict__ syms, int streams, int len,
-                                                         uint32_t* __restrict__ words, int64_t pitch,
-                                                         int32_t* __restrict__ nwords) {
-    constexpr int K = 256, B = 16;
+// Encoder on full tables (K = 256), any length: eight lanes per stream, all computing the stream's coder state and the
+// first of them writing its words, so that there are eight times as many wavefronts as with one lane per stream (a
+// wavefront's symbols are a sequential chain of dependent steps; more wavefronts per SIMD hide more of its latency).
+// The lanes share the loads: of each block of 16 symbols lane j reads the 8th-spaced two, j and j + 8, and their table
+// entries (6 loads a lane for 16 symbols), the entries one block and the symbols two blocks before they are coded,
+// non-temporal (each is read once); a symbol's entries reach the other lanes by DPP broadcasts when it is coded.
+// Positions past the end of the stream load its last symbol again and are not coded.
+// Bound by the chain of dependent steps (about 120 ns each with one stream).  Every lane loading all 32 entries of a
+// block, whole blocks only, before / now in us (2-byte tables): 16384 x 1024 541 / 544, 4096 x 1024 239 / 213,
+// 64 x 1504 322 / 300; lengths not divisible by 16, one lane per stream before: 16384 x 1023 1476 / 492,
+// 64 x 1500 1071 / 299, 1 x 1000 276 / 121.
+template <int P, typename TC>
+__global__ void __launch_bounds__(64) k_rc_encode_tables8(const TC* __restrict__ cdf, const uint8_t* __restrict__ syms,
+                                                        int streams, int len, uint32_t* __restrict__ words,
+                                                        int64_t pitch, int32_t* __restrict__ nwords) {
+    constexpr int K = 256, R = ENC_LANES_PER_STREAM, B = 2 * R;
+    const int j = threadIdx.x % R;
     const int64_t n = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / R;
     const bool live = n < streams;
-    const bool writer = live && threadIdx.x % R == 0;
+    const bool writer = live && j == 0;
     const int64_t nn = live ? n : 0;
     EncState st;
     enc_init(st);
     const WordSink sink{words + nn * pitch, pitch, writer};
     const TC* c = cdf + nn * (int64_t)len * K;
     const uint8_t* sp = syms + nn * (int64_t)len;
-    const int nb = len / B;
-    auto load_syms = [&](int b) { return *reinterpret_cast<const uint4*>(sp + (int64_t)(b < nb ? b : nb - 1) * B); };
-    auto issue = [&](int b, uint4 sv, uint32_t (&lo)[B], uint32_t (&hi)[B]) {
-        const int bb = b < nb ? b : nb - 1;
-        const uint32_t w[4] = {sv.x, sv.y, sv.z, sv.w};
+    struct Block {
+        int s[2];
+        uint32_t lo[2], hi[2];
+    };
+    auto at = [&](int b, int i) {
+        const int t = b * B + i * R + j;
+        return t < len ? t : len - 1;
+    };
+    auto load_syms = [&](int b, Block& k) {
 #pragma unroll
-        for (int u = 0; u < B; ++u) {
-            const int s = (w[u / 4] >> (8 * (u % 4))) & 0xFF;
-            const TC* r = c + ((int64_t)bb * B + u) * K;
-            lo[u] = (uint32_t)__builtin_nontemporal_load(r + s);
-            hi[u] = (uint32_t)__builtin_nontemporal_load(r + (s + 1 < K ? s + 1 : s));
-            if (s + 1 >= K) hi[u] = 1u << P;
+        for (int i = 0; i < 2; ++i) k.s[i] = sp[at(b, i)];
+    };
+    auto load_entries = [&](int b, Block& k) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const TC* r = c + (int64_t)at(b, i) * K;
+            k.lo[i] = (uint32_t)__builtin_nontemporal_load(r + k.s[i]);
+            k.hi[i] = (uint32_t)__builtin_nontemporal_load(r + (k.s[i] + 1 < K ? k.s[i] + 1 : k.s[i]));
         }
     };
-    auto code = [&](const uint32_t (&lo)[B], const uint32_t (&hi)[B]) {
+    auto code = [&](int b, const Block& k) {
+        auto one = [&](int t, uint32_t lo, uint32_t hi) {
+            if (t < len) enc_push(st, P, lo, hi - lo, sink);
+        };
 #pragma unroll
-        for (int u = 0; u < B; ++u) enc_push(st, P, lo[u], hi[u] - lo[u], sink);
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t lo = k.lo[i], hi = k.s[i] + 1 < K ? k.hi[i] : 1u << P;
+            const int t = b * B + i * R;
+            one(t, bcast8<0>(lo), bcast8<0>(hi));
+            one(t + 1, bcast8<1>(lo), bcast8<1>(hi));
+            one(t + 2, bcast8<2>(lo), bcast8<2>(hi));
+            one(t + 3, bcast8<3>(lo), bcast8<3>(hi));
+            one(t + 4, bcast8<4>(lo), bcast8<4>(hi));
+            one(t + 5, bcast8<5>(lo), bcast8<5>(hi));
+            one(t + 6, bcast8<6>(lo), bcast8<6>(hi));
+            one(t + 7, bcast8<7>(lo), bcast8<7>(hi));
+        }
     };
-    uint32_t loA[B], hiA[B], loB[B], hiB[B];
-    uint4 sv1 = load_syms(1), sv2;
-    issue(0, load_syms(0), loA, hiA);
+    const int nb = (len + B - 1) / B;
+    Block k0, k1, k2;
+    load_syms(0, k0);
+    load_syms(1, k1);
+    load_entries(0, k0);
 #pragma unroll 1
-    for (int b = 0; b < nb; b += 2) {
-        sv2 = load_syms(b + 2);
-        issue(b + 1, sv1, loB, hiB);
-        code(loA, hiA);
-        if (b + 1 >= nb) break;
-        sv1 = load_syms(b + 3);
-        issue(b + 2, sv2, loA, hiA);
-        code(loB, hiB);
+    for (int b = 0; b < nb; b += 3) {
+        load_syms(b + 2, k2);
+        load_entries(b + 1, k1);
+        code(b, k0);
+        load_syms(b + 3, k0);
+        load_entries(b + 2, k2);
+        code(b + 1, k1);
+        load_syms(b + 4, k1);
+        load_entries(b + 3, k0);
+        code(b + 2, k2);
     }
     enc_finish(st, sink);
     if (writer) nwords[n] = st.nwords;
@@ -661,18 +706,17 @@ extern "C" int rc_encode_tables(int32_t precision, int32_t cdf_bytes, const void
     if (streams == 0) return BOA_OK;
     const dim3 grid((streams + 255) / 256), block(256);
     hipStream_t s = as_stream(stream);
-    // full tables, whole 16-symbol blocks, 16-byte aligned symbol rows: the pipelined encoder
-    if (K == 256 && len >= 16 && len % 16 == 0 && ((uintptr_t)d_syms & 15) == 0 && (precision == 16 || cdf_bytes == 4)) {
-        constexpr int R = ENC_LANES_PER_STREAM;
-        const dim3 g16((unsigned)(((int64_t)streams * R + 63) / 64)), b16(64);
+    // full tables: the pipelined encoder
+    if (K == 256 && len >= 1 && (precision == 16 || cdf_bytes == 4)) {
+        const dim3 g8((unsigned)(((int64_t)streams * ENC_LANES_PER_STREAM + 63) / 64)), b8(64);
         if (cdf_bytes == 2 && precision == 16)
-            hipLaunchKernelGGL((k_rc_encode_tables16<16, uint16_t, R>), g16, b16, 0, s, (const uint16_t*)d_cdf, d_syms,
+            hipLaunchKernelGGL((k_rc_encode_tables8<16, uint16_t>), g8, b8, 0, s, (const uint16_t*)d_cdf, d_syms,
                                streams, len, d_words, pitch_words, d_nwords);
         else if (cdf_bytes == 4 && precision == 16)
-            hipLaunchKernelGGL((k_rc_encode_tables16<16, uint32_t, R>), g16, b16, 0, s, (const uint32_t*)d_cdf, d_syms,
+            hipLaunchKernelGGL((k_rc_encode_tables8<16, uint32_t>), g8, b8, 0, s, (const uint32_t*)d_cdf, d_syms,
                                streams, len, d_words, pitch_words, d_nwords);
         else if (cdf_bytes == 4 && precision == 24)
-            hipLaunchKernelGGL((k_rc_encode_tables16<24, uint32_t, R>), g16, b16, 0, s, (const uint32_t*)d_cdf, d_syms,
+            hipLaunchKernelGGL((k_rc_encode_tables8<24, uint32_t>), g8, b8, 0, s, (const uint32_t*)d_cdf, d_syms,
                                streams, len, d_words, pitch_words, d_nwords);
         else
             return boa_fail(BOA_ERR_ARG, "rc_encode_tables: precision %d with %d-byte tables unsupported",
@@ -705,19 +749,26 @@ extern "C" int rc_decode_tables(int32_t precision, int32_t cdf_bytes, const void
     if (streams == 0) return BOA_OK;
     const dim3 grid(streams), block(64);
     hipStream_t s = as_stream(stream);
-    // Full tables, lengths in whole groups of 4 steps, 16-byte aligned tables and 4-byte aligned symbol rows, and
-    // sizes whose byte offsets fit the kernels' 32-bit buffer offsets: the throughput decoders (eight streams
-    // per wavefront for 2-byte tables at P = 16 and lengths in whole groups of 8 steps, four otherwise).
+    // Full tables, 16-byte aligned (and the symbols 4-byte aligned), and sizes whose byte offsets fit the kernels'
+    // 32-bit buffer offsets: the throughput decoders.  2-byte tables at P = 16 take eight streams per wavefront once
+    // wavefronts of four streams would be more than one on each SIMD (4 streams x 4 SIMDs x 256 CUs): below, a step's
+    // latency is the time and the four-streams step is the shorter, above, its twice the instructions.  Decode in us,
+    // eight / four: 1000 x 1023 532 / 447, 4096 x 1023 531 / 472, 6000 x 1023 530 / 730, 16384 x 1023 1406 / 1642.
+    constexpr int DEC4_STREAMS = 4096;
     const int64_t words_bytes = (int64_t)streams * pitch_words * 4;
     const bool fits = words_bytes < (1ll << 32) - 16 && (int64_t)(streams + 1) * len < (1ll << 32) - 16 &&
                       (int64_t)len * K * cdf_bytes * 4 < (1ll << 31);
-    if (K == 256 && len >= 4 && len % 4 == 0 && ((uintptr_t)d_cdf & 15) == 0 && ((uintptr_t)d_syms & 3) == 0 &&
-        fits) {
+    if (K == 256 && len >= 1 && ((uintptr_t)d_cdf & 15) == 0 && ((uintptr_t)d_syms & 3) == 0 && fits) {
         const dim3 g4((unsigned)((streams + 15) / 16)), b4(256);
         const uint32_t wb = (uint32_t)words_bytes;
-        if (cdf_bytes == 2 && precision == 16 && len % 8 == 0 && ((uintptr_t)d_syms & 7) == 0)
-            hipLaunchKernelGGL((k_rc_decode_tables8<8>), dim3((unsigned)((streams + 31) / 32)), b4, 0, s,
-                               (const uint16_t*)d_cdf, d_words, pitch_words, d_nwords, streams, len, d_syms, wb);
+        const dim3 g8((unsigned)((streams + 31) / 32));
+        const bool wide = cdf_bytes == 2 && precision == 16 && streams > DEC4_STREAMS;
+        if (wide && len % 8 == 0 && ((uintptr_t)d_syms & 7) == 0)
+            hipLaunchKernelGGL((k_rc_decode_tables8<8, true>), g8, b4, 0, s, (const uint16_t*)d_cdf, d_words, pitch_words,
+                               d_nwords, streams, len, d_syms, wb);
+        else if (wide)
+            hipLaunchKernelGGL((k_rc_decode_tables8<8, false>), g8, b4, 0, s, (const uint16_t*)d_cdf, d_words, pitch_words,
+                               d_nwords, streams, len, d_syms, wb);
         else if (cdf_bytes == 2 && precision == 16)
             hipLaunchKernelGGL((k_rc_decode_tables4<16, uint16_t>), g4, b4, 0, s, (const uint16_t*)d_cdf, d_words,
                                pitch_words, d_nwords, streams, len, d_syms, wb);

@@ -34,9 +34,9 @@ def _encode_gpu(lib, P, cb, tables, syms, pitch):
     return d_cdf, d_words, d_n
 
 
-# T = 256 with K = 256 takes the throughput kernels (the block-pipelined encoder; the decoder with eight streams
-# per wave for 2-byte tables at P = 16 and T divisible by 8, four streams per wave otherwise, as T = 260);
-# T = 257 and K < 256 the one-stream-per-wave ones.  S = 45 leaves part of the last wave without a stream.
+# K = 256 takes the throughput kernels (the encoder with eight lanes per stream, the decoder with four streams per wave;
+# past 4096 streams of 2-byte tables, below, eight), K < 256 the one-stream-per-wave ones.
+# S = 45 leaves part of the last wave without a stream.
 @pytest.mark.parametrize("P,cb,K,T", [(16, 2, 256, 257), (16, 4, 256, 257), (24, 4, 256, 257), (16, 2, 100, 257),
                                       (24, 4, 7, 257), (16, 2, 256, 256), (16, 4, 256, 256), (24, 4, 256, 256),
                                       (16, 2, 256, 260)])
@@ -107,11 +107,71 @@ def test_decode_tables_arbitrary_words(gpu, ora, P, cb, T, zero):
         assert (out[s] == ref).all(), s
 
 
+@pytest.mark.parametrize("P,cb", [(16, 2), (16, 4), (24, 4)])
+@pytest.mark.parametrize("S,T", [(1, 1), (9, 2), (5, 3), (9, 5), (33, 7), (8, 9), (9, 15), (17, 17), (3, 31), (9, 49),
+                                 (4097, 1), (4101, 7), (4100, 8), (4097, 17)])
+def test_tables_any_length(gpu, ora, P, cb, S, T):
+    """The throughput coders at lengths around their blocks of 16 symbols and passes of 8 and 4: words equal the oracle's,
+    symbols come back, nothing is stored past a stream's row (guard bytes behind the last), and the encoder on symbols
+    at an odd address, as well as the one-stream decoder (tables not 16-byte aligned), give the same."""
+    from boa_amd import _native as N
+
+    rng = np.random.default_rng(P * 1000 + cb * 100 + S * 10 + T)
+    K = 256
+    cdf = ora.xq_cdf(rng.normal(0, 3, (S, T, K)).astype(np.float32), P)
+    syms = _sample(cdf, rng, P)
+    syms[:, -1] = 255  # the top entry of a row, whose upper bound is not in the table
+    tables = cdf[..., :K].astype(np.uint16 if cb == 2 else np.uint32)
+    pitch = T + 8
+    d_cdf, d_words, d_n = _encode_gpu(gpu, P, cb, tables, syms, pitch)
+    words, nw = d_words.cpu().numpy().view(np.uint32), d_n.cpu().numpy()
+    for s in range(S):
+        ref = ora.encode_tables(P, cdf[s], syms[s])
+        assert nw[s] == len(ref) and (words[s, :nw[s]] == ref).all(), s
+    odd = torch.empty(S * T + 1, dtype=torch.uint8, device="cuda")
+    odd[1:] = _dev(syms.astype(np.uint8)).reshape(-1)
+    d_w2, d_n2 = torch.zeros_like(d_words), torch.zeros_like(d_n)
+    N.check(gpu.rc_encode_tables(P, cb, N.ptr(d_cdf), K, odd.data_ptr() + 1, S, T, N.ptr(d_w2), pitch, N.ptr(d_n2),
+                                 N.stream_ptr()))
+    assert torch.equal(d_w2, d_words) and torch.equal(d_n2, d_n)
+    shifted = torch.empty(tables.nbytes + cb, dtype=torch.uint8, device="cuda")
+    shifted[cb:] = torch.from_numpy(tables.view(np.uint8).reshape(-1)).cuda()
+    for ptr in (N.ptr(d_cdf), shifted.data_ptr() + cb):
+        d_out = torch.full((S * T + 16,), 171, dtype=torch.uint8, device="cuda")
+        N.check(gpu.rc_decode_tables(P, cb, ptr, K, N.ptr(d_words), pitch, N.ptr(d_n), S, T, N.ptr(d_out),
+                                     N.stream_ptr()))
+        out = d_out.cpu().numpy()
+        assert (out[:S * T].reshape(S, T) == syms).all() and (out[S * T:] == 171).all()
+
+
+@pytest.mark.parametrize("T,zero", [(1, False), (6, False), (8, True), (13, True), (16, False)])
+def test_decode_tables_arbitrary_words_many_streams(gpu, ora, T, zero):
+    """Words that no encoder wrote through the eight-streams decoder (more than 4096 streams), whole passes of 8 and
+    not, against the oracle decoder."""
+    from boa_amd import _native as N
+
+    rng = np.random.default_rng(50 + 2 * T + zero)
+    S, K, P = 4099, 256, 16
+    cdf = ora.xq_cdf(rng.normal(0, 3, (S, T, K)).astype(np.float32), P)
+    if zero:
+        cdf = _zero_runs(cdf, rng, P)
+    pitch = 2 * T + 8
+    words = rng.integers(0, 1 << 32, (S, pitch), dtype=np.uint64).astype(np.uint32)
+    nw = rng.integers(0, 2 * T + 3, S).astype(np.int32)
+    d_cdf, d_w, d_n = _dev(cdf[..., :K].astype(np.uint16)), _dev(words.view(np.int32)), _dev(nw)
+    d_out = torch.zeros((S, T), dtype=torch.uint8, device="cuda")
+    N.check(gpu.rc_decode_tables(P, 2, N.ptr(d_cdf), K, N.ptr(d_w), pitch, N.ptr(d_n), S, T, N.ptr(d_out),
+                                 N.stream_ptr()))
+    out = d_out.cpu().numpy()
+    for s in range(S):
+        assert (out[s] == ora.decode_tables(P, cdf[s], words[s, :nw[s]])).all(), s
+
+
 @pytest.mark.parametrize("S,T", [(1, 8), (7, 16), (33, 8), (1, 4), (9, 12), (65, 4)])
 def test_decode_tables_short_streams(gpu, ora, S, T):
-    """The throughput decoders at their smallest shapes: one stream, fewer streams than a wavefront holds, and the
-    shortest lengths each takes (8 and 16 steps for eight streams per wave; 4 and 12 for four), on encoder
-    words and on arbitrary words (stream lengths 0 .. 2 T + 2), against the oracle decoder."""
+    """The throughput decoder at its smallest shapes: one stream, fewer streams than a wavefront holds, and lengths of
+    one pass and a few, on encoder words and on arbitrary words (stream lengths 0 .. 2 T + 2), against the
+    oracle decoder."""
     from boa_amd import _native as N
 
     rng = np.random.default_rng(S * 100 + T)
