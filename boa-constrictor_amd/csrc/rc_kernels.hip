@@ -108,7 +108,7 @@ constexpr int DPP_MIRROR = 0x140;      // row_mirror: lane i <- lane 15 - i with
 // cdf[i] and cdf[i - 1]; the stream's smallest index, then that entry's two values, are reduced over its 16
 // lanes with DPP moves (no entry > q gives index K, with cdf[K - 1] from the last lane and hi = 2^P).
 template <int P, typename TC, int D = 4>
-__global__ void __launch_bounds__(256) k_rc_decode_tables4(const TC* __restrict__ cdf,
+__global__ void __launch_bounds__(64) k_rc_decode_tables4(const TC* __restrict__ cdf,
                                                          const uint32_t* __restrict__ words, int64_t pitch,
                                                          const int32_t* __restrict__ nwords, int streams, int len,
                                                          uint8_t* __restrict__ syms, uint32_t words_bytes) {
@@ -116,9 +116,9 @@ __global__ void __launch_bounds__(256) k_rc_decode_tables4(const TC* __restrict_
     constexpr int NV = E * (int)sizeof(TC) / 16;  // 16-byte loads per lane per row
     constexpr uint32_t ROWB = K * sizeof(TC);      // bytes per row
     static_assert(D <= S, "at most S words are read per pass of D steps");
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x;
     const int j = lane & (S - 1), gbase = lane & ~(S - 1);
-    const int64_t n = ((int64_t)blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6)) * G + lane / S;
+    const int64_t n = (int64_t)blockIdx.x * G + lane / S;
     const bool live = n < streams;
     const int64_t nn = live ? n : 0;  // streams past the last shadow stream 0 with no words and write nothing
     int32_t nw = live ? nwords[nn] : 0;
@@ -136,8 +136,7 @@ __global__ void __launch_bounds__(256) k_rc_decode_tables4(const TC* __restrict_
     const uint32_t sbase = (uint32_t)((live ? nn : (int64_t)streams) * len);
     int32_t base = 0;
     uint32_t w0 = word(j), w1 = word(S + j), w2 = word(2 * S + j);
-    const int64_t wfirst =
-        ((int64_t)blockIdx.x * (blockDim.x / 64) + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) * G;
+    const int64_t wfirst = (int64_t)blockIdx.x * G;
     const int nlive = (int)(streams - wfirst < 0 ? 0 : (streams - wfirst > G ? G : streams - wfirst));
     const __amdgpu_buffer_rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<TC*>(cdf + (nlive > 0 ? wfirst : 0) * (int64_t)len * K), (short)0,
@@ -759,15 +758,17 @@ extern "C" int rc_decode_tables(int32_t precision, int32_t cdf_bytes, const void
     const bool fits = words_bytes < (1ll << 32) - 16 && (int64_t)(streams + 1) * len < (1ll << 32) - 16 &&
                       (int64_t)len * K * cdf_bytes * 4 < (1ll << 31);
     if (K == 256 && len >= 1 && ((uintptr_t)d_cdf & 15) == 0 && ((uintptr_t)d_syms & 3) == 0 && fits) {
-        const dim3 g4((unsigned)((streams + 15) / 16)), b4(256);
+        // a wavefront is a block: a few streams then spread over the CUs, whose address units the rows of 4-byte tables
+        // (64 B a lane) keep busy: 64 x 1500 1390 -> 633 us, 1000 x 1020 925 -> 434, 4096 x 1024 1105 -> 1101
+        const dim3 g4((unsigned)((streams + 3) / 4)), b4(64), b8(256);
         const uint32_t wb = (uint32_t)words_bytes;
         const dim3 g8((unsigned)((streams + 31) / 32));
         const bool wide = cdf_bytes == 2 && precision == 16 && streams > DEC4_STREAMS;
         if (wide && len % 8 == 0 && ((uintptr_t)d_syms & 7) == 0)
-            hipLaunchKernelGGL((k_rc_decode_tables8<8, true>), g8, b4, 0, s, (const uint16_t*)d_cdf, d_words, pitch_words,
+            hipLaunchKernelGGL((k_rc_decode_tables8<8, true>), g8, b8, 0, s, (const uint16_t*)d_cdf, d_words, pitch_words,
                                d_nwords, streams, len, d_syms, wb);
         else if (wide)
-            hipLaunchKernelGGL((k_rc_decode_tables8<8, false>), g8, b4, 0, s, (const uint16_t*)d_cdf, d_words, pitch_words,
+            hipLaunchKernelGGL((k_rc_decode_tables8<8, false>), g8, b8, 0, s, (const uint16_t*)d_cdf, d_words, pitch_words,
                                d_nwords, streams, len, d_syms, wb);
         else if (cdf_bytes == 2 && precision == 16)
             hipLaunchKernelGGL((k_rc_decode_tables4<16, uint16_t>), g4, b4, 0, s, (const uint16_t*)d_cdf, d_words,
