@@ -96,6 +96,7 @@ constexpr int DPP_XOR2 = 0x4E;         // quad_perm [2, 3, 0, 1]: lane i <- lane
 constexpr int DPP_HALF_MIRROR = 0x141; // row_half_mirror: lane i <- lane 7 - i within each 8 lanes
 constexpr int DPP_SHR1 = 0x111;        // row_shr:1: lane i <- lane i - 1 within each 16 lanes
 constexpr int DPP_MIRROR = 0x140;      // row_mirror: lane i <- lane 15 - i within each 16 lanes
+constexpr int DPP_LAST = 0x15F;        // row_newbcast:15: lane i <- lane 15 within each 16 lanes
 
 // The same coder for full tables (K = 256) in any table format and of any length: four streams per wavefront, 16 lanes
 // per stream, lane j holding entries 16 j .. 16 j + 15 of each row (a row of one stream is one contiguous 512 B
@@ -539,47 +540,120 @@ __global__ void k_rcb_init(EncState* st, int n) {
     if (i < n) enc_init(st[i]);
 }
 
-// gpu_range_coder.py:88-141, one wavefront per lane: the probabilities are staged through LDS with
-// coalesced loads, then lane 0 runs the sequential double accumulation of build_cdf_fast (the same
-// additions in the same order, so the prefix values equal the reference's cumulative_float).
+// A step's quantiser (build_cdf_fast) for four coder lanes per wavefront, 16 of its lanes to each: lane j holds the e =
+// ceil(K / 16) probabilities from j e on, the rest of its E zeros (which add nothing).  The reference adds the
+// probabilities in double one after the other, and so does this: in 16 rounds every lane takes the running sum of the
+// lane before it (0 in the first) and adds its own probabilities in order; lane j's is the reference's sum from round j
+// on.  The chain of K dependent additions is the time, and nothing else is on it but 16 moves between lanes.  One
+// wavefront per coder lane, adding in one of its lanes from LDS, before / now, encode and decode step in us: 1 x 256
+// 9.7 / 2.8 and 6.5 / 3.9, 1000 x 256 14.0 / 3.5 and 9.1 / 4.5, 4096 x 256 23.5 / 4.2 and 21.8 / 5.3, 4096 x 1000
+// 84 / 25 and 79 / 29.  (Adding from LDS without the compares, the prefixes written back, took 10.8 and 10.0 for
+// 1000 x 256: the LDS instructions of the four wavefronts on a CU, one lane active in each, were the time.)
+template <int E>
+struct RcbRow {
+    float p[E];
+    double start, norm, scale;  // the sum before this lane's entries, the sum of all
+    bool uniform;
+    uint32_t step;
+    int K, e, j;
+
+    __device__ __forceinline__ void load(const float* __restrict__ row, int k) {
+        K = k;
+        e = (k + 15) / 16;
+        j = threadIdx.x & 15;
+        if (E % 4 == 0 && e == E && K == 16 * E && ((uintptr_t)row & 15) == 0) {
+#pragma unroll
+            for (int i = 0; i < E; i += 4) {
+                const float4 v = *reinterpret_cast<const float4*>(row + j * E + i);
+                p[i] = v.x, p[i + 1] = v.y, p[i + 2] = v.z, p[i + 3] = v.w;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < E; ++i) {
+                const int t = j * e + i;
+                p[i] = i < e && t < K ? row[t] : 0.0f;
+            }
+        }
+    }
+    __device__ __forceinline__ void sum() {
+        double d[E];
+#pragma unroll
+        for (int i = 0; i < E; ++i) d[i] = (double)p[i];
+        double run = 0.0;
+#pragma unroll 1
+        for (int r = 0; r < 16; ++r) {
+            const uint64_t u = __builtin_bit_cast(uint64_t, run);
+            const uint64_t v = (uint64_t)dpp<DPP_SHR1>((uint32_t)(u >> 32)) << 32 | dpp<DPP_SHR1>((uint32_t)u);
+            run = start = __builtin_bit_cast(double, v);
+#pragma unroll
+            for (int i = 0; i < E; ++i) run += d[i];
+        }
+        const uint64_t u = __builtin_bit_cast(uint64_t, run);
+        norm = __builtin_bit_cast(double, (uint64_t)dpp<DPP_LAST>((uint32_t)(u >> 32)) << 32 | dpp<DPP_LAST>((uint32_t)u));
+        const uint32_t free_weight = (1u << RCB_P) - (uint32_t)K;
+        uniform = !(norm > 0.0) || !__builtin_isfinite(norm);
+        scale = uniform ? 0.0 : (double)free_weight / norm;
+        step = free_weight / (uint32_t)K + 1u;
+    }
+    // cdf[i], cum the sum before entry i
+    __device__ __forceinline__ uint32_t at(double cum, int i) const {
+        if (i >= K) return 1u << RCB_P;
+        if (uniform) return (uint32_t)i * step;
+        return (uint32_t)(cum * scale) + (uint32_t)i;
+    }
+    // does this lane hold entry s?  Then lo = cdf[s] and hi = cdf[s + 1].
+    __device__ __forceinline__ bool interval(int s, uint32_t& lo, uint32_t& hi) const {
+        const int own = s - j * e;
+        double run = start, c0 = 0.0, c1 = 0.0;
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            c0 = i == own ? run : c0;
+            run += (double)p[i];
+            c1 = i == own ? run : c1;
+        }
+        lo = at(c0, s);
+        hi = at(c1, s + 1);
+        return own >= 0 && own < e && s < K;
+    }
+    // the stream's smallest i in [1, K) with cdf[i] > q, K if there is none
+    __device__ __forceinline__ int above(uint32_t q) const {
+        double run = start;
+        int first = K;
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            const int t = j * e + i;
+            const bool hit = i < e && t >= 1 && t < K && at(run, t) > q;
+            first = hit && t < first ? t : first;
+            run += (double)p[i];
+        }
+        first = min(first, (int)dpp<DPP_XOR1>((uint32_t)first));
+        first = min(first, (int)dpp<DPP_XOR2>((uint32_t)first));
+        first = min(first, (int)dpp<DPP_HALF_MIRROR>((uint32_t)first));
+        return min(first, (int)dpp<DPP_MIRROR>((uint32_t)first));
+    }
+};
+
+// gpu_range_coder.py:88-141
+template <int E>
 __global__ void __launch_bounds__(64) k_rcb_encode_step(const int32_t* __restrict__ syms,
                                                        const float* __restrict__ probs,
                                                        const uint8_t* __restrict__ mask, int n, int K,
                                                        EncState* __restrict__ states,
                                                        uint32_t* __restrict__ words, int64_t pitch) {
-    __shared__ float sp[RCB_KMAX];
-    const int b = blockIdx.x;
-    const int lane = threadIdx.x;
-    if (b >= n) return;
-    if (mask && mask[b] == 0) return;
-    const int s = syms[b];
-    if (s < 0 || s >= K) return;
-    const float* row = probs + (int64_t)b * K;
-    for (int i = lane; i < K; i += 64) sp[i] = row[i];
-    __syncthreads();
-    if (lane != 0) return;
-    const uint32_t TOTAL = 1u << RCB_P;
-    const uint32_t free_weight = TOTAL - (uint32_t)K;
-    double norm = 0.0, cum_s = 0.0, cum_s1 = 0.0;
-    for (int i = 0; i < K; ++i) {
-        if (i == s) cum_s = norm;
-        if (i == s + 1) cum_s1 = norm;
-        norm += (double)sp[i];
-    }
+    const int b = blockIdx.x * 4 + threadIdx.x / 16;
+    const int bb = b < n ? b : n - 1;  // lanes past the last read the last's row and write nothing
+    RcbRow<E> row;
+    row.load(probs + (int64_t)bb * K, K);
+    const int s = syms[bb];
+    const bool codes = b < n && !(mask && mask[bb] == 0) && s >= 0 && s < K;
+    EncState st = states[bb];
+    row.sum();
     uint32_t lo, hi;
-    if (!(norm > 0.0) || !__builtin_isfinite(norm)) {
-        const uint32_t step = free_weight / (uint32_t)K + 1u;
-        lo = (uint32_t)s * step;
-        hi = (s + 1 < K) ? (uint32_t)(s + 1) * step : TOTAL;
-    } else {
-        const double scale = (double)free_weight / norm;
-        lo = (uint32_t)(cum_s * scale) + (uint32_t)s;
-        hi = (s + 1 < K) ? (uint32_t)(cum_s1 * scale) + (uint32_t)(s + 1) : TOTAL;
+    if (row.interval(codes ? s : 0, lo, hi) && codes) {
+        const WordSink sink{words + (int64_t)b * pitch, pitch, true};
+        enc_push(st, RCB_P, lo, hi - lo, sink);
+        states[b] = st;
     }
-    EncState st = states[b];
-    const WordSink sink{words + (int64_t)b * pitch, pitch, true};
-    enc_push(st, RCB_P, lo, hi - lo, sink);
-    states[b] = st;
 }
 
 __global__ void k_rcb_finalize(EncState* states, uint32_t* words, int64_t pitch, int32_t* sizes, int n) {
@@ -601,65 +675,28 @@ __global__ void k_rcb_init_dec(DecState* states, const uint32_t* words, int64_t 
     states[b] = st;
 }
 
-// gpu_range_coder.py:182-210.  Lane 0 writes the sequential Q2 prefix sums to LDS; the wave then
-// evaluates every cdf entry in parallel and finds the reference's linear-search answer with ballots.
+// gpu_range_coder.py:182-210: the symbol is the reference's linear-search answer, the smallest i in [1, K] with cdf[i] >
+// target, minus one; the lane that holds it moves the state on.
+template <int E>
 __global__ void __launch_bounds__(64) k_rcb_decode_step(const float* __restrict__ probs,
                                                        const uint8_t* __restrict__ mask, int n, int K,
                                                        DecState* __restrict__ states,
                                                        const uint32_t* __restrict__ words, int64_t pitch,
                                                        const int32_t* __restrict__ sizes,
                                                        int32_t* __restrict__ out_syms) {
-    __shared__ float sp[RCB_KMAX];
-    __shared__ double scum[RCB_KMAX + 1];
-    __shared__ double s_scale;
-    __shared__ int s_uniform;
-    const int b = blockIdx.x;
-    const int lane = threadIdx.x;
-    if (b >= n) return;
-    if (mask && mask[b] == 0) return;
-    const float* row = probs + (int64_t)b * K;
-    for (int i = lane; i < K; i += 64) sp[i] = row[i];
-    __syncthreads();
-    const uint32_t TOTAL = 1u << RCB_P;
-    const uint32_t free_weight = TOTAL - (uint32_t)K;
-    if (lane == 0) {
-        double norm = 0.0;
-        for (int i = 0; i < K; ++i) {
-            scum[i] = norm;
-            norm += (double)sp[i];
-        }
-        scum[K] = norm;
-        const int uni = (!(norm > 0.0) || !__builtin_isfinite(norm)) ? 1 : 0;
-        s_uniform = uni;
-        s_scale = uni ? 0.0 : (double)free_weight / norm;
-    }
-    __syncthreads();
-    const uint32_t* in = words + (int64_t)b * pitch;
-    const int32_t nw = sizes[b];
-    DecState st = states[b];
+    const int b = blockIdx.x * 4 + threadIdx.x / 16;
+    const int bb = b < n ? b : n - 1;
+    RcbRow<E> row;
+    row.load(probs + (int64_t)bb * K, K);
+    const bool codes = b < n && !(mask && mask[bb] == 0);
+    DecState st = states[bb];
+    const int32_t nw = sizes[bb];
     const uint32_t q = dec_target(st, RCB_P);
-    const bool uni = s_uniform != 0;
-    const double scale = s_scale;
-    const uint32_t ustep = free_weight / (uint32_t)K + 1u;
-    auto cdf_at = [&](int i) -> uint32_t {
-        if (i >= K) return TOTAL;
-        if (uni) return (uint32_t)i * ustep;
-        return (uint32_t)(scum[i] * scale) + (uint32_t)i;
-    };
-    // smallest i in [1, K] with cdf[i] > q
-    int first = K;
-    for (int base = 0; base < K; base += 64) {
-        const int i = base + lane;
-        const bool pred = (i >= 1) && (i < K) && (cdf_at(i) > q);
-        const uint64_t m = __ballot(pred);
-        if (m) { first = base + __builtin_ctzll(m); break; }
-    }
-    int s = first - 1;
-    if (s < 0) s = 0;
-    if (s >= K) s = K - 1;
-    const uint32_t lo = cdf_at(s), hi = cdf_at(s + 1);
-    dec_advance(st, RCB_P, lo, hi - lo, in, nw);
-    if (lane == 0) {
+    row.sum();
+    const int s = row.above(q) - 1;
+    uint32_t lo, hi;
+    if (row.interval(s, lo, hi) && codes) {
+        dec_advance(st, RCB_P, lo, hi - lo, words + (int64_t)b * pitch, nw);
         out_syms[b] = s;
         states[b] = st;
     }
@@ -895,11 +932,19 @@ extern "C" int rcb_create(int32_t n, int32_t k, int64_t pitch_words, void* strea
     return BOA_OK;
 }
 
+// E entries a lane hold up to 16 E symbols; a step costs the additions of 16 E, so the smallest that holds K
+#define RCB_LAUNCH(kernel, ...)                                                                                          \
+    do {                                                                                                                \
+        const dim3 grid((unsigned)((b->n + 3) / 4)), block(64);                                                          \
+        if (b->k <= 256) hipLaunchKernelGGL(kernel<16>, grid, block, 0, b->stream, __VA_ARGS__);                         \
+        else if (b->k <= 512) hipLaunchKernelGGL(kernel<32>, grid, block, 0, b->stream, __VA_ARGS__);                    \
+        else hipLaunchKernelGGL(kernel<64>, grid, block, 0, b->stream, __VA_ARGS__);                                     \
+    } while (0)
+
 extern "C" int rcb_encode_step(rcb* b, const int32_t* d_syms, const float* d_probs, const uint8_t* d_mask) {
     if (!b || !d_syms || !d_probs) return boa_fail(BOA_ERR_ARG, "rcb_encode_step: null argument");
     if (b->finalized) return boa_fail(BOA_ERR_STATE, "rcb_encode_step: batch already finalized");
-    hipLaunchKernelGGL(k_rcb_encode_step, dim3(b->n), dim3(64), 0, b->stream, d_syms, d_probs, d_mask, b->n, b->k,
-                       b->enc, b->words, b->pitch);
+    RCB_LAUNCH(k_rcb_encode_step, d_syms, d_probs, d_mask, b->n, b->k, b->enc, b->words, b->pitch);
     BOA_HIP_TRY(hipGetLastError());
     return BOA_OK;
 }
@@ -975,8 +1020,7 @@ extern "C" int rcb_init_decoder(rcb* b) {
 extern "C" int rcb_decode_step(rcb* b, const float* d_probs, int32_t* d_out_syms, const uint8_t* d_mask) {
     if (!b || !d_probs || !d_out_syms) return boa_fail(BOA_ERR_ARG, "rcb_decode_step: null argument");
     if (!b->dec_ready) return boa_fail(BOA_ERR_STATE, "rcb_decode_step: call init_decoder first");
-    hipLaunchKernelGGL(k_rcb_decode_step, dim3(b->n), dim3(64), 0, b->stream, d_probs, d_mask, b->n, b->k, b->dec,
-                       b->words, b->pitch, b->sizes, d_out_syms);
+    RCB_LAUNCH(k_rcb_decode_step, d_probs, d_mask, b->n, b->k, b->dec, b->words, b->pitch, b->sizes, d_out_syms);
     BOA_HIP_TRY(hipGetLastError());
     return BOA_OK;
 }

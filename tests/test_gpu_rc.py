@@ -426,3 +426,47 @@ def test_compaction(gpu, lanes, pitch):
     with pytest.raises(N.BoaError):
         N.check(gpu.boa_compact(N.ptr(d_words), pitch, N.ptr(d_nw), lanes, N.ptr(d_off), N.ptr(small), total - 1,
                                 ctypes.byref(got), N.stream_ptr()))
+
+
+@pytest.mark.parametrize("N,K", [(1, 1), (3, 2), (5, 15), (4, 16), (6, 17), (9, 255), (7, 256), (2, 257), (5, 511),
+                                 (3, 512), (6, 513), (5, 1023), (4, 1024)])
+def test_batch_coder_alphabets(gpu, ora, N, K):
+    """Alphabets around the 16 lanes and the 256, 512 and 1024 entries that a coder lane's wavefront part holds, streams
+    that do not fill a wavefront, rows with zero runs, masked lanes and symbols out of range (skipped): the words are the
+    oracle's and the symbols come back; rows off 16-byte alignment give the same."""
+    import gpu_range_coder as gr
+
+    rng = np.random.default_rng(N * 10000 + K)
+    T = 6
+    probs = rng.random((T, N, K)).astype(np.float32)
+    probs[rng.random(probs.shape) < 0.3] = 0.0
+    probs[0] = np.exp(rng.normal(0, 6, (N, K))).astype(np.float32)  # sums that round differently in another order
+    syms = rng.integers(0, K, (T, N)).astype(np.int32)
+    syms[1] = K - 1
+    syms[2] = 0
+    mask = rng.random((T, N)) < 0.7
+    mask[0] = True
+    sent = syms.copy()
+    sent[3, 0] = K  # out of range: skipped
+    mask_dec = mask.copy()
+    mask_dec[3, 0] = False
+    flat = torch.zeros(T * N * K + 1, dtype=torch.float32, device="cuda")
+    flat[1:] = _dev(probs).reshape(-1)
+    got = []
+    for view in (_dev(probs), flat[1:].view(T, N, K)):
+        b = gr.gpu.queue.RangeCoderBatch(N, K, T + 8)
+        for t in range(T):
+            b.encode_step(_dev(sent[t]), view[t], torch.from_numpy(mask[t]).cuda())
+        b.finalize()
+        got.append(b.get_compressed_list())
+    for i in range(N):
+        keep = [t for t in range(T) if mask_dec[t, i]]
+        ref = ora.encode_probs_q2(24, probs[keep, i], syms[keep, i])
+        assert (got[0][i] == ref).all() and len(got[0][i]) == len(ref) and (got[1][i] == ref).all(), i
+    d = gr.gpu.queue.RangeCoderBatch(N, K, T + 8)
+    d.load_compressed_list(got[0])
+    d.init_decoder()
+    for t in range(T):
+        out = torch.full((N,), -1, dtype=torch.int32, device="cuda")
+        d.decode_step(_dev(probs[t]), out, torch.from_numpy(mask_dec[t]).cuda())
+        assert (out.cpu().numpy() == np.where(mask_dec[t], syms[t], -1)).all(), t
