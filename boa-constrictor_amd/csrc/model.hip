@@ -2925,7 +2925,8 @@ static int64_t workspace_rows(const boa_model_cfg& c, int R, int precision, int6
         return rows;
     int64_t up = 16;
     while (up < max_lanes) up *= 2;
-    const int64_t p = std::max<int64_t>(1, std::min<int64_t>(PIPE_TILES / up, std::min(c.n_layers, PIPE_MAX)));
+    int64_t p = std::max<int64_t>(1, std::min<int64_t>(PIPE_TILES / up, std::min(c.n_layers, PIPE_MAX)));
+    if (up == 16) ++p;  // for the tile whose head runs beside the next step (run_pipe)
     return rows + (p - 1) * up * pipe_tile(tile_len);
 }
 
@@ -3838,9 +3839,10 @@ extern "C" int boa_model_step(boa_ctx* x, const int32_t* d_tokens, int32_t lanes
 constexpr int PIPE_SPLIT = 128, PIPE_ROWS16 = 128;
 static int pipe_quad(const boa_ctx* x) { return x->d == ffn5::D ? 128 : 512; }
 static int pipe_two(const boa_ctx* x) { return x->d == ffn5::D ? 64 : 640; }
-static int pipe_depth(const boa_ctx* x, int lanes) {
+// tiles that the workspace holds, of up to one more than are in flight at once
+static int pipe_slots(const boa_ctx* x, int lanes) {
     const int64_t fit = x->ws_rows / ((int64_t)lanes * pipe_tile(x->tile_len));
-    return (int)std::max<int64_t>(1, std::min<int64_t>(fit, std::min(x->L, PIPE_MAX)));
+    return (int)std::max<int64_t>(1, std::min<int64_t>(fit, std::min(x->L, PIPE_MAX) + 1));
 }
 static bool pipe_ok(const boa_ctx* x, int lanes) {
     return x->pipe && x->ffn_outp && pipe_tile(x->tile_len) >= PIPE_MIN_TILE && lanes <= PIPE_LANES;
@@ -3853,12 +3855,13 @@ struct PipeRun {
     EmbedIn src;
     int64_t lane0, row0;
     hipStream_t s;
-    int TL, n, P, step = 0, first = 0;
+    hipStream_t side = nullptr;  // where finish() runs, if not on s
+    int TL, n, P, slots, step = 0, first = 0;
     std::vector<int> start;
-    PipeRun(boa_ctx* c, int lanes_, int len_, const EmbedIn& e, int depth, int64_t l0, hipStream_t st)
+    PipeRun(boa_ctx* c, int lanes_, int len_, const EmbedIn& e, int depth, int slots_, int64_t l0, hipStream_t st)
         : x(c), lanes(lanes_), len(len_), src(e), lane0(l0), s(st), TL(pipe_tile(c->tile_len)), n((len_ + TL - 1) / TL),
-          P(std::min(depth, n)), start(n) {
-        row0 = lane0 * depth * TL;
+          P(std::min(depth, n)), slots(slots_), start(n) {
+        row0 = lane0 * slots * TL;
         if (src.bytes) { src.bytes += lane0 * src.stride; src.lens += lane0; }
         if (src.tokens) src.tokens += lane0 * src.stride;
         for (int t = 0; t < n; ++t) {
@@ -3888,10 +3891,11 @@ int PipeRun::advance(Finish&& finish) {
         ma.emb = -1;
         for (int t = first; t < n && start[t] <= step; ++t, ++ne) {
             const int l = step - start[t], Tc = std::min(TL, len - t * TL);
-            const int64_t ro = row0 + (int64_t)(t % P) * lanes * TL, M = (int64_t)lanes * Tc;
+            const int64_t ro = row0 + (int64_t)(t % slots) * lanes * TL, M = (int64_t)lanes * Tc;
             const LayerW& w = x->layers[l];
             ma.t[ne] = mixin_tile_args(x, l, ro, pos0 + (int64_t)t * TL, Tc);
             if (l == 0) {
+                if (side && t >= slots) BOA_HIP_TRY(hipStreamWaitEvent(s, x->half_ev[t % slots], 0));  // the slot's last head
                 ma.emb = ne;
                 ma.e.t0 = src.t0 + t * TL;
                 ma.e.xout = x->x + ro * d;
@@ -3959,9 +3963,16 @@ int PipeRun::advance(Finish&& finish) {
         if (e == hipSuccess) e = hipGetLastError();
         if (e != hipSuccess) return boa_fail_hip(e, "run_pipe", __FILE__, __LINE__);
         if (step - start[first] == L - 1) {
+            if (side) {
+                BOA_HIP_TRY(hipEventRecord(x->half_ev[2 * L + 1], s));
+                BOA_HIP_TRY(hipStreamWaitEvent(side, x->half_ev[2 * L + 1], 0));
+                x->stream = side;
+            }
             const int rc = finish(*this, first * TL, std::min(TL, len - first * TL),
-                                  x->x + (row0 + (int64_t)(first % P) * lanes * TL) * d);
+                                  x->x + (row0 + (int64_t)(first % slots) * lanes * TL) * d);
+            x->stream = s;
             if (rc) return rc;
+            if (side) BOA_HIP_TRY(hipEventRecord(x->half_ev[first % slots], side));
             ++first;
         }
         ++step;
@@ -3971,21 +3982,32 @@ int PipeRun::advance(Finish&& finish) {
 
 // All lanes, in one group or in two halves on two streams (as the classic compress tiles run): one half's scan, head and
 // coder then run beside the other's matrix kernels.
+// In one group whose 16-row workgroups leave CUs for it, a finished tile's head and coder, which nothing in the next step
+// waits for, run on the second stream beside that step, in tile order (a tile's head and 64 coder steps take 34 us of a
+// step's 120); the tile's slot is taken again by the tile that starts a step later, behind an event.  Compress in us, one
+// stream / two: 1 x 1000 2842 / 2498.  Where the step fills the GPU the head only holds up its last workgroups: 64 x 1500
+// 17202 / 18130, forward 8 x 500 1274 / 1286.
 template <class Finish>
 static int run_pipe(boa_ctx* x, int lanes, int len, const EmbedIn& src, Finish&& finish) {
-    const int depth = pipe_depth(x, lanes);
+    const int slots = pipe_slots(x, lanes), depth = std::min(slots, std::min(x->L, PIPE_MAX));
     const bool own_head = x->head_xq && (x->V == headq::V || x->d == 256);  // no shared buffers behind the head
     const bool two = x->stream2 && x->compress_halves && own_head && lanes >= 2 && lanes * depth >= pipe_two(x);
     const int la = two ? lanes / 2 : lanes;
     int rc = BOA_OK;
     if (!two) {
-        PipeRun a(x, lanes, len, src, depth, 0, x->stream);
+        PipeRun a(x, lanes, len, src, depth, slots, 0, x->stream);
+        const bool room = (int64_t)lanes * (depth + 1) * ((a.TL + 15) / 16) <= x->cus;
+        if (room && x->stream2 && x->compress_halves && own_head && a.n > 1 && (slots > depth || a.n <= slots)) a.side = x->stream2;
         while (!a.done() && !rc) rc = a.advance(finish);
+        if (a.side) {
+            BOA_HIP_TRY(hipEventRecord(x->half_ev[2 * x->L], a.side));
+            BOA_HIP_TRY(hipStreamWaitEvent(x->stream, x->half_ev[2 * x->L], 0));
+        }
     } else {
         hipEvent_t join = x->half_ev[2 * x->L];
         BOA_HIP_TRY(hipEventRecord(join, x->stream));  // the second half starts after what the stream holds
         BOA_HIP_TRY(hipStreamWaitEvent(x->stream2, join, 0));
-        PipeRun a(x, la, len, src, depth, 0, x->stream), b(x, lanes - la, len, src, depth, la, x->stream2);
+        PipeRun a(x, la, len, src, depth, depth, 0, x->stream), b(x, lanes - la, len, src, depth, depth, la, x->stream2);
         while (!a.done() && !rc) {  // the same steps on both
             rc = a.advance(finish);
             if (!rc) rc = b.advance(finish);
@@ -4118,13 +4140,13 @@ extern "C" int boa_compress(boa_ctx* x, const uint8_t* d_bytes, int64_t byte_str
                 r = run_head(x, g.lanes, Tc, x->logits, xin);
                 if (r) return r;
                 PROF(PC_ENCODE, 0.0, 4.0 * M * x->V + (double)M,
-                     hipLaunchKernelGGL(k_encode_tile, dim3(g.lanes), dim3(64), 0, g.s, x->logits, x->V, Tc, t0, bytes,
+                     hipLaunchKernelGGL(k_encode_tile, dim3(g.lanes), dim3(64), 0, x->stream, x->logits, x->V, Tc, t0, bytes,
                                         byte_stride, d_lens + b0, x->enc + b0, d_words + b0 * pitch_words, pitch_words));
                 return r;
             }
             if (r) return r;
             PROF(PC_ENCODE, 0.0, 8.0 * M + 32.0 * g.lanes,
-                 hipLaunchKernelGGL(k_encode_lf, dim3((g.lanes + 255) / 256), dim3(256), 0, g.s, lf, Tc, g.lanes,
+                 hipLaunchKernelGGL(k_encode_lf, dim3((g.lanes + 255) / 256), dim3(256), 0, x->stream, lf, Tc, g.lanes,
                                     x->enc + b0, d_words + b0 * pitch_words, pitch_words));
             return r;
         });

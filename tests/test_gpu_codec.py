@@ -515,6 +515,30 @@ def test_tiles_in_flight_match_tile_after_tile(gpu, monkeypatch, d_model, n_laye
         assert torch.equal(a[2], b[2]), (n, length)
 
 
+@pytest.mark.parametrize("d_model,n_layers,precision", [(256, 1, "f32"), (256, 3, "bf16x3"), (512, 2, "bf16w")])
+@pytest.mark.parametrize("n,length", [(1, 65), (1, 1300), (3, 200), (6, 700)])
+def test_heads_beside_the_next_step_match_one_stream(gpu, monkeypatch, d_model, n_layers, precision, n, length):
+    """One group of lanes: heads and coder of finished tiles on the second stream (fewer tiles than slots, every slot
+    taken many times) give the words and logits of one stream, bit for bit, on each of several calls in a row."""
+    import codec
+    import model as M
+    from boa_amd import weights as W
+
+    blob = W.seeded_blob(W.Cfg(d_model=d_model, n_layers=n_layers), 7)
+    rng = np.random.default_rng(length)
+    calls = [([rng.integers(0, 256, length - 5 * i).astype(np.uint8) for i in range(n)],
+              torch.from_numpy(rng.integers(0, 256, (n, length)))) for _ in range(3)]
+    got = {}
+    for halves in ("0", "1"):
+        monkeypatch.setenv("BOA_COMPRESS_HALVES", halves)
+        m = M.BoaConstrictor(d_model, n_layers, 256).load_blob(blob)
+        m.precision = precision
+        got[halves] = [(codec.compress_payload(m, chunks), m.forward(tok.cuda()).cpu()) for chunks, tok in calls]
+    for (pa, fa), (pb, fb) in zip(got["0"], got["1"]):
+        assert np.array_equal(pa[0], pb[0]) and np.array_equal(pa[1], pb[1])
+        assert torch.equal(fa, fb)
+
+
 @pytest.mark.parametrize("d_model,precision", [(256, "f32"), (256, "bf16x3"), (512, "bf16w")])
 @pytest.mark.parametrize("split", [1, 2, 3, 64, 65, 130])
 def test_forward_in_pieces_and_steps(gpu, d_model, precision, split):
