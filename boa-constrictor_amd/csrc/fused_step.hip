@@ -694,10 +694,24 @@ __global__ void __launch_bounds__(NTHR) k_fused_step(FusedArgs a) {
 // others idle; 16-row workgroups take a quarter of that on four times as many CUs.  Same arithmetic per row, so the
 // same values (every output accumulates its K steps in ascending order).  BLOCK: 512 threads, one workgroup per CU.
 
-// x <- x + FF2(GELU(FF1(LN2(out_proj(y))))) for 16 rows of tile blockIdx.y.
-template <int NT>
+// x <- x + FF2(GELU(FF1(LN2(out_proj(y))))) for 16 rows of tile blockIdx.y: by one workgroup (FFN_ALL), or by S that share
+// the rows, in two launches: FFN_UP, out_proj and LN2 by each, FF1 + GELU of hidden units (1024 / S) blockIdx.z .., which
+// go to the tile's hid rows; FFN_DOWN, FF2 and the residual of outputs (256 / S) blockIdx.z .. from them.
+// One workgroup multiplies for 34 us at a CU's fp32 rate (45 us in all; bf16x3: 32 us, its 2.6 MB of weights through one
+// CU), so with 32 of them (1 lane, 8 tiles in flight) 7/8 of the CUs idle.  A share of 4 does 2/5 of the MFMAs (out_proj
+// 1/5 whole, the rest a quarter), for one more launch.  Splitting K instead would change the order of FF2's sums.
+// Whole passes in us, one workgroup / S = 4 (fp32, 64 to 128 groups of rows: / S = 2 at full steps), d 256 x 8 layers:
+//   compress 1 x 1000 fp32 2511 / 2169, 2 x 1000 2584 / 2330, 4 x 700 2104 / 1911, 12 x 60 1004 / 880;
+//   bf16x3 1 x 1000 2093 / 1945; forward 1 x 1000 fp32 2180 / 1836, bf16x3 1790 / 1651.
+// bf16x3 with S = 2 (1 x 1000 2220, 4 x 700 1980 against 1830) loses to one workgroup and is not built.
+enum { FFN_ALL, FFN_UP, FFN_DOWN };
+template <int NT, int PART, int S>
 __global__ void __launch_bounds__(512) k_ffn16(FfnTiles a) {
-    constexpr int NWAVE = 8, RPW = ROWS / NWAVE, FPW_B = NT == 1 ? 8 : 4, D_B = 3, FPW_S = 2, D_S = 6;
+    constexpr int NWAVE = 8, RPW = ROWS / NWAVE, FPW_S = 2, D_S = 6, HID = 4 * FD;
+    constexpr int FPW_B = PART == FFN_UP ? HID / 16 / S / NWAVE : (NT == 1 ? 8 : 4), D_B = PART == FFN_UP ? 6 : 3;
+    constexpr int FPW_D = PART == FFN_DOWN ? 1 : FPW_S, NFD = FD / 16 / S;  // FF2: fragments per wave, per workgroup
+    static_assert(PART == FFN_ALL ? S == 1 : (NFD <= NWAVE && NFD * S * 16 == FD), "shares");
+    static_assert(PART != FFN_UP || FPW_B * NWAVE * S * 16 == HID, "shares");
     __shared__ __attribute__((aligned(16))) unsigned char lds[SZ_A + SZ_X];
     uint16_t* sAh = reinterpret_cast<uint16_t*>(lds);
     uint16_t* sAl = sAh + ROWS * LA;
@@ -711,74 +725,102 @@ __global__ void __launch_bounds__(512) k_ffn16(FfnTiles a) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = NT == 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
     const int m_of = 4 * (lane >> 4), n_of = lane & 15;
-    const int rot64 = (int)(blockIdx.x & 7) * 8, rot16 = (int)(blockIdx.x & 15);
-    // y rows (rows past the tile's end read 0)
-    if constexpr (NT == 1) {
-        const __amdgpu_buffer_rsrc_t ry = buf_rsrc(reinterpret_cast<const float*>(w.yh) + m0 * FDI, (uint32_t)nb * FDI * 4);
+    const int part = PART == FFN_ALL ? 0 : (int)blockIdx.z;
+    const int rot64 = PART == FFN_ALL ? (int)(blockIdx.x & 7) * 8 : 0, rot16 = PART == FFN_DOWN ? 0 : (int)(blockIdx.x & 15);
+    // hidden rows: fp32, or hi and lo parts one after the other
+    const __amdgpu_buffer_rsrc_t rhid = buf_rsrc(w.hid + m0 * HID, (uint32_t)nb * HID * 4);
+    if constexpr (PART == FFN_DOWN) {
 #pragma unroll
-        for (int e = 0; e < ROWS * FDI / 4 / 512; ++e) {
-            const int i = e * 512 + tid, r = i / (FDI / 4), k = (i % (FDI / 4)) * 4;
-            *reinterpret_cast<u32x4*>(reinterpret_cast<float*>(sAh) + r * ld32(LA) + k) = buf_ld16(ry, (uint32_t)(r * FDI + k) * 4);
-        }
-    } else {
-        const __amdgpu_buffer_rsrc_t rh = buf_rsrc(w.yh + m0 * FDI, (uint32_t)nb * FDI * 2);
-        const __amdgpu_buffer_rsrc_t rl = buf_rsrc(w.yl + m0 * FDI, (uint32_t)nb * FDI * 2);
-#pragma unroll
-        for (int e = 0; e < ROWS * FDI / 8 / 512; ++e) {
-            const int i = e * 512 + tid, r = i / (FDI / 8), k = (i % (FDI / 8)) * 8;
-            *reinterpret_cast<u32x4*>(sAh + r * LA + k) = buf_ld16(rh, (uint32_t)(r * FDI + k) * 2);
-            *reinterpret_cast<u32x4*>(sAl + r * LA + k) = buf_ld16(rl, (uint32_t)(r * FDI + k) * 2);
+        for (int e = 0; e < ROWS * HID / 4 / 512; ++e) {
+            const int i = e * 512 + tid, r = i / (HID / 4), q = i % (HID / 4);  // 16 bytes q of row r
+            const u32x4 v = buf_ld16(rhid, (uint32_t)i * 16);
+            if constexpr (NT == 1) *reinterpret_cast<u32x4*>(reinterpret_cast<float*>(sHh) + r * ld32(LH) + q * 4) = v;
+            else *reinterpret_cast<u32x4*>((q < HID / 8 ? sHh : sHl - HID) + r * LH + q * 8) = v;
         }
     }
-    const float4 lnw = ldg_f4(G(w.ln_w) + 4 * lane), lnb = ldg_f4(G(w.ln_b) + 4 * lane);
-    __syncthreads();
-    {
-        floatx4 acc[FPW_S];
-        float bias_j[FPW_S];
+    if constexpr (PART != FFN_DOWN) {
+        // y rows (rows past the tile's end read 0)
+        if constexpr (NT == 1) {
+            const __amdgpu_buffer_rsrc_t ry = buf_rsrc(reinterpret_cast<const float*>(w.yh) + m0 * FDI, (uint32_t)nb * FDI * 4);
 #pragma unroll
-        for (int j = 0; j < FPW_S; ++j) bias_j[j] = G(w.out_b)[16 * frag_of<NWAVE>(0, wave, j, FD / 16, rot16) + n_of];
-        mgemm<NT, NWAVE, FPW_S, FDI, D_S, false>(sAh, sAl, LA, w.out_p, 0, FD / 16, wave, lane, rot16, acc);
+            for (int e = 0; e < ROWS * FDI / 4 / 512; ++e) {
+                const int i = e * 512 + tid, r = i / (FDI / 4), k = (i % (FDI / 4)) * 4;
+                *reinterpret_cast<u32x4*>(reinterpret_cast<float*>(sAh) + r * ld32(LA) + k) = buf_ld16(ry, (uint32_t)(r * FDI + k) * 4);
+            }
+        } else {
+            const __amdgpu_buffer_rsrc_t rh = buf_rsrc(w.yh + m0 * FDI, (uint32_t)nb * FDI * 2);
+            const __amdgpu_buffer_rsrc_t rl = buf_rsrc(w.yl + m0 * FDI, (uint32_t)nb * FDI * 2);
 #pragma unroll
-        for (int j = 0; j < FPW_S; ++j) {
-            const int n = 16 * frag_of<NWAVE>(0, wave, j, FD / 16, rot16) + n_of;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sX[(m_of + r) * LRES + n] = epi_value<EPI_BIAS>(acc[j][r], bias_j[j]);
+            for (int e = 0; e < ROWS * FDI / 8 / 512; ++e) {
+                const int i = e * 512 + tid, r = i / (FDI / 8), k = (i % (FDI / 8)) * 8;
+                *reinterpret_cast<u32x4*>(sAh + r * LA + k) = buf_ld16(rh, (uint32_t)(r * FDI + k) * 2);
+                *reinterpret_cast<u32x4*>(sAl + r * LA + k) = buf_ld16(rl, (uint32_t)(r * FDI + k) * 2);
+            }
         }
-    }
-    __syncthreads();
-    ln_rows<NT, RPW>(sX, lnw, lnb, sAh, sAl, wave, lane);
-    __syncthreads();
+        const float4 lnw = ldg_f4(G(w.ln_w) + 4 * lane), lnb = ldg_f4(G(w.ln_b) + 4 * lane);
+        __syncthreads();
+        {
+            floatx4 acc[FPW_S];
+            float bias_j[FPW_S];
+#pragma unroll
+            for (int j = 0; j < FPW_S; ++j) bias_j[j] = G(w.out_b)[16 * frag_of<NWAVE>(0, wave, j, FD / 16, rot16) + n_of];
+            mgemm<NT, NWAVE, FPW_S, FDI, D_S, false>(sAh, sAl, LA, w.out_p, 0, FD / 16, wave, lane, rot16, acc);
+#pragma unroll
+            for (int j = 0; j < FPW_S; ++j) {
+                const int n = 16 * frag_of<NWAVE>(0, wave, j, FD / 16, rot16) + n_of;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sX[(m_of + r) * LRES + n] = epi_value<EPI_BIAS>(acc[j][r], bias_j[j]);
+            }
+        }
+        __syncthreads();
+        ln_rows<NT, RPW>(sX, lnw, lnb, sAh, sAl, wave, lane);
+        __syncthreads();
 #pragma unroll 1
-    for (int f0 = 0; f0 < 4 * FD / 16; f0 += FPW_B * NWAVE) {
-        floatx4 acc[FPW_B];
-        float bias_j[FPW_B];
+        for (int f0 = part * (HID / 16 / S); f0 < (part + 1) * (HID / 16 / S); f0 += FPW_B * NWAVE) {
+            floatx4 acc[FPW_B];
+            float bias_j[FPW_B];
 #pragma unroll
-        for (int j = 0; j < FPW_B; ++j) bias_j[j] = G(w.ff1_b)[16 * frag_of<NWAVE>(f0, wave, j, 4 * FD / 16, rot64) + n_of];
-        mgemm<NT, NWAVE, FPW_B, FD, D_B, false, 2>(sAh, sAl, LA, w.ff1_p, f0, 4 * FD / 16, wave, lane, rot64, acc);
+            for (int j = 0; j < FPW_B; ++j) bias_j[j] = G(w.ff1_b)[16 * frag_of<NWAVE>(f0, wave, j, 4 * FD / 16, rot64) + n_of];
+            mgemm<NT, NWAVE, FPW_B, FD, D_B, false, 2>(sAh, sAl, LA, w.ff1_p, f0, 4 * FD / 16, wave, lane, rot64, acc);
 #pragma unroll
-        for (int j = 0; j < FPW_B; ++j) {
-            const int n = 16 * frag_of<NWAVE>(f0, wave, j, 4 * FD / 16, rot64) + n_of;
+            for (int j = 0; j < FPW_B; ++j) {
+                const int n = 16 * frag_of<NWAVE>(f0, wave, j, 4 * FD / 16, rot64) + n_of;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) store_op<NT, LH>(sHh, m_of + r, n, epi_value<EPI_GELU>(acc[j][r], bias_j[j]));
+                for (int r = 0; r < 4; ++r) {
+                    const float y = epi_value<EPI_GELU>(acc[j][r], bias_j[j]);
+                    if constexpr (PART == FFN_ALL) {
+                        store_op<NT, LH>(sHh, m_of + r, n, y);
+                    } else if constexpr (NT == 1) {
+                        buf_st1(rhid, (uint32_t)((m_of + r) * HID + n) * 4, y);
+                    } else {
+                        uint32_t hi, lo;
+                        split2(y, hi, lo);
+                        __builtin_amdgcn_raw_buffer_store_b16((uint16_t)hi, rhid, (uint32_t)((m_of + r) * 2 * HID + n) * 2, 0, 0);
+                        __builtin_amdgcn_raw_buffer_store_b16((uint16_t)lo, rhid, (uint32_t)((m_of + r) * 2 * HID + HID + n) * 2, 0, 0);
+                    }
+                }
+            }
         }
     }
+    if constexpr (PART == FFN_UP) return;
     __syncthreads();
-    {
+    if (PART == FFN_ALL || wave < NFD) {
+        const int f0 = part * NFD;
         const __amdgpu_buffer_rsrc_t rx = buf_rsrc(w.x + m0 * FD, (uint32_t)nb * FD * 4);
-        floatx4 acc[FPW_S];
-        float bias_j[FPW_S], res[FPW_S][4];
+        floatx4 acc[FPW_D];
+        float bias_j[FPW_D], res[FPW_D][4];
 #pragma unroll
-        for (int j = 0; j < FPW_S; ++j) {
-            const int n = 16 * frag_of<NWAVE>(0, wave, j, FD / 16, rot16) + n_of;
+        for (int j = 0; j < FPW_D; ++j) {
+            const int n = 16 * frag_of<NWAVE>(f0, wave, j, FD / 16, rot16) + n_of;
             bias_j[j] = G(w.ff2_b)[n];
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 res[j][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, (uint32_t)((m_of + r) * FD + n) * 4, 0, 0));
         }
-        mgemm<NT, NWAVE, FPW_S, 4 * FD, D_S, false>(sHh, sHl, LH, w.ff2_p, 0, FD / 16, wave, lane, rot16, acc);
+        mgemm<NT, NWAVE, FPW_D, 4 * FD, D_S, false>(sHh, sHl, LH, w.ff2_p, f0, FD / 16, wave, lane, rot16, acc);
 #pragma unroll
-        for (int j = 0; j < FPW_S; ++j) {
-            const int n = 16 * frag_of<NWAVE>(0, wave, j, FD / 16, rot16) + n_of;
+        for (int j = 0; j < FPW_D; ++j) {
+            const int n = 16 * frag_of<NWAVE>(f0, wave, j, FD / 16, rot16) + n_of;
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 __builtin_amdgcn_raw_buffer_store_b32(
@@ -860,11 +902,30 @@ __global__ void __launch_bounds__(512) k_head16(HeadRows a) {
 
 }  // namespace
 
-hipError_t launch_ffn16(const FfnTiles& a, int tiles, int64_t max_rows, int nt, hipStream_t s) {
+template <int NT>
+static void ffn16(const FfnTiles& a, dim3 grid, int split, hipStream_t s) {
+    grid.z = (unsigned)split;
+    if (split == 4) {
+        hipLaunchKernelGGL((k_ffn16<NT, FFN_UP, 4>), grid, dim3(512), 0, s, a);
+        hipLaunchKernelGGL((k_ffn16<NT, FFN_DOWN, 4>), grid, dim3(512), 0, s, a);
+        return;
+    }
+    if constexpr (NT == 1) {
+        if (split == 2) {
+            hipLaunchKernelGGL((k_ffn16<NT, FFN_UP, 2>), grid, dim3(512), 0, s, a);
+            hipLaunchKernelGGL((k_ffn16<NT, FFN_DOWN, 2>), grid, dim3(512), 0, s, a);
+            return;
+        }
+    }
+    grid.z = 1;
+    hipLaunchKernelGGL((k_ffn16<NT, FFN_ALL, 1>), grid, dim3(512), 0, s, a);
+}
+
+hipError_t launch_ffn16(const FfnTiles& a, int tiles, int64_t max_rows, int split, int nt, hipStream_t s) {
     const dim3 grid((unsigned)((max_rows + ROWS - 1) / ROWS), (unsigned)tiles);
-    if (nt == 3) hipLaunchKernelGGL((k_ffn16<3>), grid, dim3(512), 0, s, a);
-    else if (nt == 2) hipLaunchKernelGGL((k_ffn16<2>), grid, dim3(512), 0, s, a);
-    else hipLaunchKernelGGL((k_ffn16<1>), grid, dim3(512), 0, s, a);
+    if (nt == 3) ffn16<3>(a, grid, split, s);
+    else if (nt == 2) ffn16<2>(a, grid, split, s);
+    else ffn16<1>(a, grid, split, s);
     return hipGetLastError();
 }
 

@@ -3912,6 +3912,7 @@ int PipeRun::advance(Finish&& finish) {
             ft.x = x->x + ro * d;
             ft.yh = split ? st.yh : reinterpret_cast<const uint16_t*>(st.xs);
             ft.yl = st.yl;
+            ft.hid = x->xz + ro * 2 * di;  // the scan has read z; a row holds the 4 d hidden units
             ft.M = M;
             rows += M;
             groups64 += (M + 63) / 64;
@@ -3953,7 +3954,9 @@ int PipeRun::advance(Finish&& finish) {
                  if (nt == 3) hipLaunchKernelGGL((k_ffn512_gen<3>), g64, dim3(512), 0, s, fa);
                  else hipLaunchKernelGGL((k_ffn512_gen<2>), g64, dim3(512), 0, s, fa));
         } else if (groups64 <= PIPE_ROWS16) {
-            PROF(PC_FFN, fflops, fbytes, e = launch_ffn16(fa, ne, max_m, nt, s));
+            const int64_t groups16 = (int64_t)ne * ((max_m + 15) / 16);
+            const int fsplit = groups16 * 4 <= x->cus ? 4 : (nt == 1 && groups16 * 2 <= x->cus ? 2 : 1);  // while CUs idle
+            PROF(PC_FFN, fflops, fbytes, e = launch_ffn16(fa, ne, max_m, fsplit, nt, s));
         } else {
             PROF(PC_FFN, fflops, fbytes,
                  if (nt == 1) hipLaunchKernelGGL((k_ffn_gen<1>), g64, dim3(512), 0, s, fa);

@@ -86,13 +86,15 @@ struct FfnTile {
     const uint16_t *out_p, *ff1_p, *ff2_p;
     float* x;
     const uint16_t *yh, *yl;  // the scan's output: split parts, or fp32 at yh (fp32 mode)
+    float* hid;               // [M][4 d], for k_ffn16 in two launches
     int64_t M;
 };
 struct FfnTiles {
     FfnTile t[PIPE_MAX];
 };
 // d_model 256, 16 rows per workgroup (fused_step.hip): for launches whose tiles are too few for k_ffn's 64-row workgroups
-hipError_t launch_ffn16(const FfnTiles& a, int tiles, int64_t max_rows, int nt, hipStream_t s);
+// split: workgroups per 16 rows (1, 4, in the fp32 mode also 2).
+hipError_t launch_ffn16(const FfnTiles& a, int tiles, int64_t max_rows, int split, int nt, hipStream_t s);
 
 // Head (Linear -> ReLU -> Linear) of M rows of x, 16 per workgroup (d_model 256): row m is position t0 + m % Tc of lane
 // m / Tc.  Either the coder interval of the byte the position predicts (lf[m]), or the logits (logits[(lane * len + t0 +

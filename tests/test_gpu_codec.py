@@ -539,6 +539,30 @@ def test_heads_beside_the_next_step_match_one_stream(gpu, monkeypatch, d_model, 
         assert torch.equal(fa, fb)
 
 
+@pytest.mark.parametrize("precision", ["f32", "bf16x3", "bf16w"])
+@pytest.mark.parametrize("n,length", [(1, 18), (1, 80), (3, 34), (15, 66), (16, 130), (17, 129), (33, 64)])
+def test_feed_forward_in_shares(gpu, monkeypatch, precision, n, length):
+    """Feed-forward of 16 rows by four, two (fp32) and one workgroup, on both sides of each limit and with remainders of
+    16 rows: words and logits of 64-row workgroups, tile after tile, bit for bit."""
+    import codec
+    import model as M
+    from boa_amd import weights as W
+
+    blob = W.seeded_blob(W.Cfg(d_model=256, n_layers=2), 11)
+    rng = np.random.default_rng(n)
+    chunks = [rng.integers(0, 256, length).astype(np.uint8) for _ in range(n)]
+    tok = torch.from_numpy(rng.integers(0, 256, (n, length))).cuda()
+    got = []
+    for pipe in ("0", "1"):
+        monkeypatch.setenv("BOA_PIPE", pipe)
+        m = M.BoaConstrictor(256, 2, 256).load_blob(blob)
+        m.precision = precision
+        payload, nw, _, _ = codec.compress_payload(m, chunks)
+        got.append((payload, nw, m.forward(tok).cpu()))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+    assert torch.equal(got[0][2], got[1][2])
+
+
 @pytest.mark.parametrize("d_model,precision", [(256, "f32"), (256, "bf16x3"), (512, "bf16w")])
 @pytest.mark.parametrize("split", [1, 2, 3, 64, 65, 130])
 def test_forward_in_pieces_and_steps(gpu, d_model, precision, split):
