@@ -535,9 +535,11 @@ __global__ void __launch_bounds__(256) k_rc_synth_tables(uint64_t seed, float si
 static constexpr int RCB_P = 24;
 static constexpr int RCB_KMAX = 1024;  // the reference's per-thread table holds K+1 <= 1025 entries
 
-__global__ void k_rcb_init(EncState* st, int n) {
+__global__ void k_rcb_init(EncState* st, int32_t* sizes, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) enc_init(st[i]);
+    if (i >= n) return;
+    enc_init(st[i]);
+    sizes[i] = 0;
 }
 
 // A step's quantiser (build_cdf_fast) for four coder lanes per wavefront, 16 of its lanes to each: lane j holds the e =
@@ -881,6 +883,7 @@ struct rcb {
     int32_t n = 0, k = 0;
     int64_t pitch = 0;
     hipStream_t stream = nullptr;
+    unsigned char* mem = nullptr;  // one allocation for the five arrays below (each of its own cost a malloc and a free)
     EncState* enc = nullptr;
     DecState* dec = nullptr;
     uint32_t* words = nullptr;
@@ -895,7 +898,7 @@ extern "C" int rcb_destroy(rcb* b) {
     if (!b) return BOA_OK;
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     else (void)hipDeviceSynchronize();
-    void* ptrs[] = {b->enc, b->dec, b->words, b->sizes, b->off, b->payload};
+    void* ptrs[] = {b->mem, b->payload};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     delete b;
@@ -913,14 +916,19 @@ extern "C" int rcb_create(int32_t n, int32_t k, int64_t pitch_words, void* strea
     b->pitch = pitch_words;
     b->stream = as_stream(stream);
     hipError_t e = hipSuccess;
-    if (e == hipSuccess) e = hipMalloc((void**)&b->enc, sizeof(EncState) * n);
-    if (e == hipSuccess) e = hipMalloc((void**)&b->dec, sizeof(DecState) * n);
-    if (e == hipSuccess) e = hipMalloc((void**)&b->words, sizeof(uint32_t) * (size_t)n * (size_t)pitch_words);
-    if (e == hipSuccess) e = hipMalloc((void**)&b->sizes, sizeof(int32_t) * n);
-    if (e == hipSuccess) e = hipMalloc((void**)&b->off, sizeof(int64_t) * n);
-    if (e == hipSuccess) e = hipMemsetAsync(b->sizes, 0, sizeof(int32_t) * n, b->stream);
+    auto up = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+    const size_t s_enc = up(sizeof(EncState) * (size_t)n), s_dec = up(sizeof(DecState) * (size_t)n),
+                 s_sizes = up(sizeof(int32_t) * (size_t)n), s_off = up(sizeof(int64_t) * (size_t)n);
+    if (e == hipSuccess)
+        e = hipMalloc((void**)&b->mem, s_enc + s_dec + s_sizes + s_off + sizeof(uint32_t) * (size_t)n * (size_t)pitch_words);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_rcb_init, dim3((n + 255) / 256), dim3(256), 0, b->stream, b->enc, n);
+        unsigned char* p = b->mem;
+        b->enc = reinterpret_cast<EncState*>(p); p += s_enc;
+        b->dec = reinterpret_cast<DecState*>(p); p += s_dec;
+        b->sizes = reinterpret_cast<int32_t*>(p); p += s_sizes;
+        b->off = reinterpret_cast<int64_t*>(p); p += s_off;
+        b->words = reinterpret_cast<uint32_t*>(p);
+        hipLaunchKernelGGL(k_rcb_init, dim3((n + 255) / 256), dim3(256), 0, b->stream, b->enc, b->sizes, n);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipStreamSynchronize(b->stream);

@@ -25,6 +25,8 @@ from boa_amd import _native as _nat
 
 __all__ = ["gpu"]
 
+_U32 = np.dtype(np.uint32)
+
 
 class _RangeCoderBatch:
     def __init__(self, N: int, K: int, maxL: int, pitch_bytes: int | None = None):
@@ -47,16 +49,14 @@ class _RangeCoderBatch:
     def load_compressed_list(self, compressed_list):
         if len(compressed_list) != self.N:
             raise RuntimeError("compressed_list length must equal N")
-        arrs, sizes = [], np.zeros(self.N, dtype=np.int32)
-        for i, c in enumerate(compressed_list):
-            a = np.asarray(c)
-            if a.ndim != 1 or a.itemsize != 4 or a.dtype.kind != "u":
+        arrs = list(map(np.asarray, compressed_list))
+        for a in arrs:
+            if a.ndim != 1 or (a.dtype != _U32 and (a.itemsize != 4 or a.dtype.kind != "u")):
                 raise RuntimeError("Each compressed item must be uint32[?]")
-            if a.shape[0] > self.pitch_words:
+            if len(a) > self.pitch_words:
                 raise RuntimeError("Compressed stream exceeds pitch; increase pitch")
-            arrs.append(np.ascontiguousarray(a, dtype=np.uint32))
-            sizes[i] = a.shape[0]
-        words = np.concatenate(arrs) if sizes.sum() else np.zeros(1, dtype=np.uint32)
+        sizes = np.fromiter(map(len, arrs), np.int32, self.N)
+        words = np.ascontiguousarray(np.concatenate(arrs), np.uint32) if sizes.any() else np.zeros(1, dtype=np.uint32)
         _nat.check(self._lib.rcb_load(self._h, _nat.ptr(words), _nat.ptr(sizes)))
 
     # gpu_range_coder.py:509-527
@@ -79,19 +79,21 @@ class _RangeCoderBatch:
     def finalize(self):
         _nat.check(self._lib.rcb_finalize(self._h))
 
-    def get_sizes_list(self):
+    def _sizes(self) -> np.ndarray:
         sizes = np.zeros(self.N, dtype=np.int32)
         _nat.check(self._lib.rcb_get_sizes(self._h, _nat.ptr(sizes)))
-        return [int(s) for s in sizes]
+        return sizes
+
+    def get_sizes_list(self):
+        return self._sizes().tolist()
 
     def get_compressed_list(self):
-        sizes = np.asarray(self.get_sizes_list(), dtype=np.int64)
-        total = int(sizes.sum())
+        ends = np.cumsum(self._sizes(), dtype=np.int64).tolist()
+        total = ends[-1]
         words = np.zeros(max(total, 1), dtype=np.uint32)
         got = ctypes.c_int64(0)
         _nat.check(self._lib.rcb_get_words(self._h, _nat.ptr(words), words.size, ctypes.byref(got)))
-        offs = np.concatenate([[0], np.cumsum(sizes)])
-        return [words[offs[i]:offs[i + 1]].copy() for i in range(self.N)]
+        return [words[a:b].copy() for a, b in zip([0] + ends, ends)]
 
     def init_decoder(self):
         _nat.check(self._lib.rcb_init_decoder(self._h))
