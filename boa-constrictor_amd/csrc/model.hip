@@ -3824,7 +3824,8 @@ extern "C" int boa_model_step(boa_ctx* x, const int32_t* d_tokens, int32_t lanes
 //
 // Within a step, a kernel with too few workgroups is cut finer: the mixer input over groups of in_proj chunks (its
 // x_proj partials then folded by the scan), the scan over four threads per channel, the feed-forward and the head over
-// 16 rows instead of 64.  finish(t0, Tc, xin) handles a tile that has passed the last layer.
+// 16 rows instead of 64, the feed-forward with the fewest rows over four workgroups per 16 (two launches).  finish(t0, Tc,
+// xin) handles a tile that has passed the last layer.
 // Where the lines lie (compress, ms; d 256 x 8 layers over 704 positions, d 512 x 16 layers bf16w over 320):
 //   PIPE_LANES: against tile after tile on two streams, which from 512 lanes on fills the GPU by itself.  fp32 64 lanes
 //     29.0 -> 8.4, 256: 30.6 -> 26.3, 375: 50.2 -> 39.4, 512: 50.1 -> 50.5; bf16x3 375: 23.6 -> 21.1, 512: 26.4 -> 28.4;
