@@ -570,9 +570,9 @@ __global__ void __launch_bounds__(256) k_embed_bytes(const uint8_t* __restrict__
 }
 
 // Layer 0 of a full compress tile reads its input rows straight from the embedding table in the LN1 prologue of
-// the mixer-input kernel (k_mixin, k_mixin512: template parameter EMB), which also writes them to x, the residual
+// the mixer-input kernel (k_mixin, k_mixin512: MixinOne<true>), which also writes them to x, the residual
 // stream the feed-forward kernel adds to; the separate embedding pass (k_embed_bytes) and its HBM round trip are
-// skipped.  Without EMB the kernels read x as written by an embedding pass or the previous layer, and ignore this.
+// skipped.  Otherwise the kernels read x as written by an embedding pass or the previous layer, and ignore this.
 struct EmbedIn {
     const uint8_t* bytes = nullptr;  // the group's bytes [lanes][stride]
     int64_t stride = 0;
@@ -838,13 +838,17 @@ __device__ __forceinline__ int h_off(int r, int k) { return r * HC + (((k >> 3) 
 // accumulating its 16 K steps in ascending order through mfma_split_step (as the out_proj GEMM does); mm then
 // stays on chip (fp32 in the operand buffer) for LN2, instead of a round trip through HBM.  Wave w owns
 // out_proj outputs 32 w .. + 31 of all 64 rows; its 32 W_out blocks stream through a 4-slot ring.
-template <int NT, bool OUTP>
-__device__ __forceinline__ void ffn_rows(const float* __restrict__ mm, const float* __restrict__ ln_w,
-                                         const float* __restrict__ ln_b, const uint16_t* __restrict__ W1p,
-                                         const float* __restrict__ b1, const uint16_t* __restrict__ W2p,
-                                         const float* __restrict__ b2, float* __restrict__ x, int64_t M,
-                                         const uint16_t* __restrict__ yh, const uint16_t* __restrict__ yl,
-                                         const uint16_t* __restrict__ Wop, const float* __restrict__ bo) {
+// A: FfnTile, or FfnTiles for several tiles in one launch (blockIdx.y picks the tile; rows past a tile's M read 0 and
+// store nothing).  One kernel template for both, its body in the kernel itself: as a device function called from two
+// kernels the same body took 128 registers and spilled 53 (fp32) and 40 (bf16x3) in either kernel.
+template <int NT, bool OUTP, class A>
+__global__ void __launch_bounds__(512, 4) k_ffn(A a) {
+    const FfnTile& tile = ffn_tile(a);
+    const int64_t M = tile.M;
+    if ((int64_t)blockIdx.x * ffn::BM >= M) return;
+    const float *mm = tile.mm, *ln_w = tile.ln_w, *ln_b = tile.ln_b, *b1 = tile.ff1_b, *b2 = tile.ff2_b, *bo = tile.out_b;
+    const uint16_t *W1p = tile.ff1_p, *W2p = tile.ff2_p, *yh = tile.yh, *yl = tile.yl, *Wop = tile.out_p;
+    float* x = tile.x;
     using namespace ffn;
     __shared__ __attribute__((aligned(16))) uint16_t sA[2][BM * D];
     __shared__ __attribute__((aligned(16))) uint16_t sH[2][BM * HC];
@@ -1093,24 +1097,6 @@ __device__ __forceinline__ void ffn_rows(const float* __restrict__ mm, const flo
     }
 }
 
-template <int NT, bool OUTP>
-__global__ void __launch_bounds__(512, 4) k_ffn(const float* __restrict__ mm, const float* __restrict__ ln_w,
-                                                const float* __restrict__ ln_b, const uint16_t* __restrict__ W1p,
-                                                const float* __restrict__ b1, const uint16_t* __restrict__ W2p,
-                                                const float* __restrict__ b2, float* __restrict__ x, int64_t M,
-                                                const uint16_t* __restrict__ yh, const uint16_t* __restrict__ yl,
-                                                const uint16_t* __restrict__ Wop, const float* __restrict__ bo) {
-    ffn_rows<NT, OUTP>(mm, ln_w, ln_b, W1p, b1, W2p, b2, x, M, yh, yl, Wop, bo);
-}
-
-// The same over several tiles in one launch: blockIdx.y picks the tile (rows past a tile's M read 0, store nothing).
-template <int NT>
-__global__ void __launch_bounds__(512, 4) k_ffn_gen(FfnTiles a) {
-    const FfnTile& t = a.t[blockIdx.y];
-    if ((int64_t)blockIdx.x * ffn::BM >= t.M) return;
-    ffn_rows<NT, true>(nullptr, t.ln_w, t.ln_b, t.ff1_p, t.ff1_b, t.ff2_p, t.ff2_b, t.x, t.M, t.yh, t.yl, t.out_p, t.out_b);
-}
-
 // ================================================================================================
 // The same feed-forward half for d_model 512 (d_ff 2048; configs[4]'s shape):
 //   x <- x + FF2(GELU(FF1(LN2(mm))))
@@ -1151,13 +1137,15 @@ constexpr int ffn_groups() { return NT == 2 ? 2 : 1; }
 // through the LDS operand buffer, each output accumulating its 32 K steps in ascending order through
 // mfma_split_step (as the out_proj GEMM does); mm then stays on chip (fp32 in the operand buffer) for LN2.
 // Wave w owns out_proj outputs 64 w .. + 63 of all 64 rows; its W_out blocks stream through an 8-slot ring.
-template <int NT, bool OUTP>
-__device__ __forceinline__ void ffn512_rows(const float* __restrict__ mm, const float* __restrict__ ln_w,
-                                            const float* __restrict__ ln_b, const uint16_t* __restrict__ W1p,
-                                            const float* __restrict__ b1, const uint16_t* __restrict__ W2p,
-                                            const float* __restrict__ b2, float* __restrict__ x, int64_t M,
-                                            const uint16_t* __restrict__ yh, const uint16_t* __restrict__ yl,
-                                            const uint16_t* __restrict__ Wop, const float* __restrict__ bo) {
+// A: as k_ffn's.
+template <int NT, bool OUTP, class A>
+__global__ void __launch_bounds__(512, 2) k_ffn512(A a) {
+    const FfnTile& tile = ffn_tile(a);
+    const int64_t M = tile.M;
+    if ((int64_t)blockIdx.x * ffn5::BM >= M) return;
+    const float *mm = tile.mm, *ln_w = tile.ln_w, *ln_b = tile.ln_b, *b1 = tile.ff1_b, *b2 = tile.ff2_b, *bo = tile.out_b;
+    const uint16_t *W1p = tile.ff1_p, *W2p = tile.ff2_p, *yh = tile.yh, *yl = tile.yl, *Wop = tile.out_p;
+    float* x = tile.x;
     using namespace ffn5;
     __shared__ __attribute__((aligned(16))) uint16_t sA[2][BM * D];
     __shared__ __attribute__((aligned(16))) uint16_t sH[2][BM * HC * ffn_groups<NT>()];
@@ -1421,25 +1409,6 @@ __device__ __forceinline__ void ffn512_rows(const float* __restrict__ mm, const 
     }
 }
 
-template <int NT, bool OUTP>
-__global__ void __launch_bounds__(512, 2) k_ffn512(const float* __restrict__ mm, const float* __restrict__ ln_w,
-                                                   const float* __restrict__ ln_b, const uint16_t* __restrict__ W1p,
-                                                   const float* __restrict__ b1, const uint16_t* __restrict__ W2p,
-                                                   const float* __restrict__ b2, float* __restrict__ x, int64_t M,
-                                                   const uint16_t* __restrict__ yh, const uint16_t* __restrict__ yl,
-                                                   const uint16_t* __restrict__ Wop, const float* __restrict__ bo) {
-    ffn512_rows<NT, OUTP>(mm, ln_w, ln_b, W1p, b1, W2p, b2, x, M, yh, yl, Wop, bo);
-}
-
-// The same over several tiles in one launch, as k_ffn_gen.
-template <int NT>
-__global__ void __launch_bounds__(512, 2) k_ffn512_gen(FfnTiles a) {
-    const FfnTile& t = a.t[blockIdx.y];
-    if ((int64_t)blockIdx.x * ffn5::BM >= t.M) return;
-    ffn512_rows<NT, true>(nullptr, t.ln_w, t.ln_b, t.ff1_p, t.ff1_b, t.ff2_p, t.ff2_b, t.x, t.M, t.yh, t.yl, t.out_p,
-                          t.out_b);
-}
-
 // ================================================================================================
 // Input half of the mixer in one kernel (split modes, d_model 256, compress tiles of 64 positions):
 //   LN1 -> in_proj (+bias) -> z to HBM; x -> causal conv + SiLU over the 64 positions -> xs to HBM ->
@@ -1468,25 +1437,44 @@ struct MixinTile {
     int p0m3, Tc;
 };
 struct MixinTiles {
+    static constexpr bool GEN = true;
     MixinTile t[PIPE_MAX];
     EmbedIn e;       // the embedding source of tile `emb` (its layer is the model's first), if any
     int emb;         // -1: no tile gathers embedding rows
     int per;         // in_proj chunks per workgroup (blockIdx.z takes chunks per * z ..)
+    __device__ __forceinline__ const MixinTile& tile() const { return t[blockIdx.y]; }
+    __device__ __forceinline__ bool gather() const { return (int)blockIdx.y == emb; }
+    __device__ __forceinline__ int first_chunk() const { return (int)blockIdx.z * per; }
+    __device__ __forceinline__ int chunks() const { return per; }
+};
+// A full tile (64 positions) of one layer, all its chunks; EMB: it gathers embedding rows.
+template <bool EMB>
+struct MixinOne {
+    static constexpr bool GEN = false;
+    MixinTile t;
+    EmbedIn e;
+    __device__ __forceinline__ const MixinTile& tile() const { return t; }
+    __device__ __forceinline__ bool gather() const { return EMB; }
+    __device__ __forceinline__ int first_chunk() const { return 0; }
+    __device__ __forceinline__ int chunks() const { return 0; }
 };
 
-// GEN: the general form, for tiles of Tc <= 64 positions and for launches with few tiles.  Rows past Tc repeat the
-// tile's last row and are not stored.  A workgroup may own only the in_proj chunks [c0, c1) of its tile: the x
-// chunks' channels are independent of each other up to x_proj, whose partial of each 64-channel K block is then
-// stored (part: [rows][8][48], row stride ldp) for the scan to fold in the same order.  Workgroup `first` also
-// copies the embedding rows out.
-template <int NT, bool EMB, bool GEN>
-__device__ __forceinline__ void mixin_tile(const float* __restrict__ x, const float* __restrict__ ln_w,
-                                           const float* __restrict__ ln_b, const uint16_t* __restrict__ Wip,
-                                           const float* __restrict__ bin, const float* __restrict__ conv_w,
-                                           const float* __restrict__ conv_b, const uint16_t* __restrict__ Wxp,
-                                           float* __restrict__ xz, float* __restrict__ xs,
-                                           float* __restrict__ dbc, float* __restrict__ hist, int p0m3, EmbedIn e,
-                                           bool gather, int tc, int c0, int c1) {
+// A: MixinOne, or MixinTiles: the general form (GEN), for tiles of Tc <= 64 positions and for launches with few tiles.
+// There blockIdx.y picks the tile, and rows past Tc repeat the tile's last row and are not stored.  A workgroup may own
+// only the in_proj chunks [c0, c1) of its tile (blockIdx.z): the x chunks' channels are independent of each other up to
+// x_proj, whose partial of each 64-channel K block (48 values) then goes to the x half of the row's xz, for the scan to
+// fold in the same order.  The workgroup of the first chunks also copies the embedding rows out.
+// One template with the body in the kernel: as a device function called from two kernels the body took 9 registers more
+// (fp32 239 instead of 230) in the full-tile kernels and 10 more in the general ones.
+template <int NT, class A>
+__global__ void __launch_bounds__(256, 2) k_mixin(A a) {
+    constexpr bool GEN = A::GEN;
+    const MixinTile& tile = a.tile();
+    const float *x = tile.x, *ln_w = tile.ln_w, *ln_b = tile.ln_b, *bin = tile.in_b, *conv_w = tile.conv_w, *conv_b = tile.conv_b;
+    const uint16_t *Wip = tile.in_p, *Wxp = tile.x_p;
+    float *xz = tile.xz, *xs = tile.xs, *dbc = tile.dbc, *hist = tile.hist;
+    const int p0m3 = tile.p0m3, tc = tile.Tc, c0 = a.first_chunk(), c1 = c0 + a.chunks();
+    const EmbedIn& e = a.e;
     using namespace mixin;
     constexpr int BLK = two_part_blocks<NT>() ? 1024 : 512;
     __shared__ __attribute__((aligned(16))) uint16_t sA[2][BM * D];  // LN1 output (hi, lo)
@@ -1497,14 +1485,14 @@ __device__ __forceinline__ void mixin_tile(const float* __restrict__ x, const fl
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int Tc = GEN ? tc : BM;
     const int64_t b = blockIdx.x, m0 = b * Tc;
-    const bool emb = GEN ? gather : EMB;  // compile-time without GEN
+    const bool emb = a.gather();  // compile-time without GEN
     const bool split = GEN && c1 - c0 < 2 * DI / CH;
     // ---- LN1 (layer 0 of a compress tile: of the embedding rows, which are also written to x at the end; lane q
     //      of a wave reads the token of its row q, handed to every lane by readlane)
     int tokv = 0;
     if constexpr (GEN) {
         if (emb) tokv = embed_token(e, b, 16 * wave + (lane & 15), Tc);
-    } else if constexpr (EMB) {
+    } else if (emb) {
         tokv = byte_token(e.bytes, e.stride, e.lens, b, e.t0 + 16 * wave + (lane & 15), e.V);
     }
     {
@@ -1710,26 +1698,6 @@ __device__ __forceinline__ void mixin_tile(const float* __restrict__ x, const fl
     }
 }
 
-template <int NT, bool EMB>
-__global__ void __launch_bounds__(256, 2) k_mixin(const float* __restrict__ x, const float* __restrict__ ln_w,
-                                                 const float* __restrict__ ln_b, const uint16_t* __restrict__ Wip,
-                                                 const float* __restrict__ bin, const float* __restrict__ conv_w,
-                                                 const float* __restrict__ conv_b, const uint16_t* __restrict__ Wxp,
-                                                 float* __restrict__ xz, float* __restrict__ xs,
-                                                 float* __restrict__ dbc, float* __restrict__ hist, int p0m3,
-                                                 EmbedIn e) {
-    mixin_tile<NT, EMB, false>(x, ln_w, ln_b, Wip, bin, conv_w, conv_b, Wxp, xz, xs, dbc, hist, p0m3, e, EMB, 0, 0, 0);
-}
-
-// The general form: blockIdx.y picks the tile, blockIdx.z the in_proj chunks.
-template <int NT>
-__global__ void __launch_bounds__(256, 2) k_mixin_gen(MixinTiles a) {
-    const MixinTile& t = a.t[blockIdx.y];
-    const int c0 = (int)blockIdx.z * a.per;
-    mixin_tile<NT, false, true>(t.x, t.ln_w, t.ln_b, t.in_p, t.in_b, t.conv_w, t.conv_b, t.x_p, t.xz, t.xs, t.dbc,
-                                t.hist, t.p0m3, a.e, (int)blockIdx.y == a.emb, t.Tc, c0, c0 + a.per);
-}
-
 // The mixer's input half for d_model 512 (d_inner 1024, dt_rank 32, x_proj width 64; configs[4]'s shape), one
 // lane's tile of 64 positions per workgroup: LN1 -> in_proj (+bias) -> z to HBM; x -> causal conv + SiLU over the
 // tile -> xs to HBM -> x_proj, folded over 64-channel K blocks (XPROJ_KB) in registers -> dbc to HBM; the conv
@@ -1746,15 +1714,16 @@ namespace mixin5 {
 constexpr int BM = 64, D = 512, DI = 1024, CH = 64, FW = 64;
 }  // namespace mixin5
 
-// GEN: as in mixin_tile (part: [rows][16][64]).
-template <int NT, bool EMB, bool GEN>
-__device__ __forceinline__ void mixin512_tile(const float* __restrict__ x, const float* __restrict__ ln_w,
-                                              const float* __restrict__ ln_b, const uint16_t* __restrict__ Wip,
-                                              const float* __restrict__ bin, const float* __restrict__ conv_w,
-                                              const float* __restrict__ conv_b, const uint16_t* __restrict__ Wxp,
-                                              float* __restrict__ xz, float* __restrict__ xs,
-                                              float* __restrict__ dbc, float* __restrict__ hist, int p0m3, EmbedIn e,
-                                              bool gather, int tc, int c0, int c1) {
+// A: as k_mixin's (x_proj partials of 64 values).
+template <int NT, class A>
+__global__ void __launch_bounds__(512, 2) k_mixin512(A a) {
+    constexpr bool GEN = A::GEN;
+    const MixinTile& tile = a.tile();
+    const float *x = tile.x, *ln_w = tile.ln_w, *ln_b = tile.ln_b, *bin = tile.in_b, *conv_w = tile.conv_w, *conv_b = tile.conv_b;
+    const uint16_t *Wip = tile.in_p, *Wxp = tile.x_p;
+    float *xz = tile.xz, *xs = tile.xs, *dbc = tile.dbc, *hist = tile.hist;
+    const int p0m3 = tile.p0m3, tc = tile.Tc, c0 = a.first_chunk(), c1 = c0 + a.chunks();
+    const EmbedIn& e = a.e;
     using namespace mixin5;
     using mixin::sx_off;
     using mixin::x_off;
@@ -1767,14 +1736,14 @@ __device__ __forceinline__ void mixin512_tile(const float* __restrict__ x, const
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int Tc = GEN ? tc : BM;
     const int64_t b = blockIdx.x, m0 = b * Tc;
-    const bool emb = GEN ? gather : EMB;  // compile-time without GEN
+    const bool emb = a.gather();  // compile-time without GEN
     const bool split = GEN && c1 - c0 < 2 * DI / CH;
     // ---- LN1: 8 rows per wave (layer 0 of a compress tile: of the embedding rows, which are also written to x at
     //      the end; lane q of a wave reads the token of its row q, handed to every lane by readlane)
     int tokv = 0;
     if constexpr (GEN) {
         if (emb) tokv = embed_token(e, b, 8 * wave + (lane & 7), Tc);
-    } else if constexpr (EMB) {
+    } else if (emb) {
         tokv = byte_token(e.bytes, e.stride, e.lens, b, e.t0 + 8 * wave + (lane & 7), e.V);
     }
     {
@@ -1924,7 +1893,7 @@ __device__ __forceinline__ void mixin512_tile(const float* __restrict__ x, const
                 sXl[x_off(r, cl)] = (uint16_t)lo;
             }
             // history ring: inputs of positions p0 + Tc - 3, - 2, - 1 in slots (p0 + Tc) mod 3, + 1, + 2 (wave 7), as
-            // in mixin_tile
+            // in k_mixin
             const int e0 = (p0m3 + Tc) % 3, e1 = (e0 + 1) % 3, e2 = (e0 + 2) % 3;
             const __amdgpu_buffer_rsrc_t hw = buf_rsrc(hist + b * 3 * DI, g == BM / 8 - 1 ? 3 * DI * 4 : 0);
             const uint32_t none = 0xFFFFFFF0u;
@@ -1975,26 +1944,6 @@ __device__ __forceinline__ void mixin512_tile(const float* __restrict__ x, const
             *reinterpret_cast<float4*>(xr_ + 256) = ldg_f4(er + 256);
         }
     }
-}
-
-template <int NT, bool EMB>
-__global__ void __launch_bounds__(512, 2) k_mixin512(const float* __restrict__ x, const float* __restrict__ ln_w,
-                                                     const float* __restrict__ ln_b, const uint16_t* __restrict__ Wip,
-                                                     const float* __restrict__ bin, const float* __restrict__ conv_w,
-                                                     const float* __restrict__ conv_b, const uint16_t* __restrict__ Wxp,
-                                                     float* __restrict__ xz, float* __restrict__ xs,
-                                                     float* __restrict__ dbc, float* __restrict__ hist, int p0m3,
-                                                     EmbedIn e) {
-    mixin512_tile<NT, EMB, false>(x, ln_w, ln_b, Wip, bin, conv_w, conv_b, Wxp, xz, xs, dbc, hist, p0m3, e, EMB, 0, 0, 0);
-}
-
-// The general form: blockIdx.y picks the tile, blockIdx.z the in_proj chunks.
-template <int NT>
-__global__ void __launch_bounds__(512, 2) k_mixin512_gen(MixinTiles a) {
-    const MixinTile& t = a.t[blockIdx.y];
-    const int c0 = (int)blockIdx.z * a.per;
-    mixin512_tile<NT, false, true>(t.x, t.ln_w, t.ln_b, t.in_p, t.in_b, t.conv_w, t.conv_b, t.x_p, t.xz, t.xs, t.dbc,
-                                   t.hist, t.p0m3, a.e, (int)blockIdx.y == a.emb, t.Tc, c0, c0 + a.per);
 }
 
 // fp32 mode: the K-block fold over the fp32 weight matrix (k_xproj_f32)
@@ -3356,18 +3305,33 @@ static MixinTile mixin_tile_args(const boa_ctx* x, int l, int64_t row_off, int64
     t.p0m3 = (int)(pos % 3); t.Tc = Tc;
     return t;
 }
+// The feed-forward half of M rows from row_off on.
+static FfnTile ffn_tile_args(const boa_ctx* x, const LayerW& w, int64_t row_off, int64_t M) {
+    const int64_t d = x->d, di = x->di;
+    FfnTile t;
+    t.out_b = w.out_b; t.ln_w = w.ln2_w; t.ln_b = w.ln2_b; t.ff1_b = w.ff1_b; t.ff2_b = w.ff2_b;
+    t.out_p = w.out_w.p; t.ff1_p = w.ff1_w.p; t.ff2_p = w.ff2_w.p;
+    t.x = x->x + row_off * d;
+    t.mm = nullptr;
+    const bool split = x->prec != BOA_PREC_F32;
+    t.yh = split ? x->ah + row_off * di : reinterpret_cast<const uint16_t*>(x->xs + row_off * di);
+    t.yl = split ? x->al + row_off * di : nullptr;
+    t.hid = x->xz + row_off * 2 * di;  // the scan has read z; a row holds the 4 d hidden units
+    t.M = M;
+    return t;
+}
 // blockIdx.z workgroups per tile, each with an equal share of its in_proj chunks (per chunks)
 static void launch_mixin_gen(const boa_ctx* x, const MixinTiles& a, int lanes, int tiles, int z, hipStream_t s) {
     const dim3 grid((unsigned)lanes, (unsigned)tiles, (unsigned)z);
     if (x->d == mixin5::D) {
-        if (x->prec == BOA_PREC_BF16X3) hipLaunchKernelGGL((k_mixin512_gen<3>), grid, dim3(512), 0, s, a);
-        else hipLaunchKernelGGL((k_mixin512_gen<2>), grid, dim3(512), 0, s, a);
+        if (x->prec == BOA_PREC_BF16X3) hipLaunchKernelGGL((k_mixin512<3, MixinTiles>), grid, dim3(512), 0, s, a);
+        else hipLaunchKernelGGL((k_mixin512<2, MixinTiles>), grid, dim3(512), 0, s, a);
     } else if (x->prec == BOA_PREC_F32) {
-        hipLaunchKernelGGL((k_mixin_gen<1>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_mixin<1, MixinTiles>), grid, dim3(256), 0, s, a);
     } else if (x->prec == BOA_PREC_BF16X3) {
-        hipLaunchKernelGGL((k_mixin_gen<3>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_mixin<3, MixinTiles>), grid, dim3(256), 0, s, a);
     } else {
-        hipLaunchKernelGGL((k_mixin_gen<2>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_mixin<2, MixinTiles>), grid, dim3(256), 0, s, a);
     }
 }
 static int mixin_chunks(const boa_ctx* x) { return 2 * x->di / 64; }
@@ -3417,9 +3381,10 @@ static int run_layer(boa_ctx* x, int l, int B, int Tc, int part = 7) {
     float* hist = x->conv_hist + ((int64_t)l * x->max_lanes + x->lane0) * 3 * di;
     const bool mix5 = mixin512_layer(x, w, Tc);
     const bool shorter = Tc < mixin::BM && (mix5 || mixin_layer(x, w, Tc));
+    const MixinTile mt = mixin_tile_args(x, l, 0, x->pos, Tc);
     if (shorter && (part & 1)) {
         MixinTiles a;
-        a.t[0] = mixin_tile_args(x, l, 0, x->pos, Tc);
+        a.t[0] = mt;
         a.e = ein; a.emb = emb ? 0 : -1; a.per = mixin_chunks(x);
         PROF(PC_MIXIN, gemm_flops(M, 2 * di, d) + gemm_flops(M, R + 2 * NS, di) + 8.0 * M * di,
              4.0 * M * (d + di + di + R + 2 * NS) + 4.0 * 6 * B * di, launch_mixin_gen(x, a, B, 1, 1, s));
@@ -3429,20 +3394,12 @@ static int run_layer(boa_ctx* x, int l, int B, int Tc, int part = 7) {
         const double bytes = 4.0 * M * (d + di + di + R + 2 * NS) + 4.0 * 6 * B * di;
         if (w.in_w.l)
             PROF(PC_MIXIN, flops, bytes,
-                 if (emb) hipLaunchKernelGGL((k_mixin512<3, true>), dim3((unsigned)B), dim3(512), 0, s, x->x, w.ln1_w,
-                                           w.ln1_b, w.in_w.p, w.in_b, w.conv_w, w.conv_b, w.x_w.p, x->xz, x->xs,
-                                           x->dbc, hist, (int)(x->pos % 3), ein);
-                 else hipLaunchKernelGGL((k_mixin512<3, false>), dim3((unsigned)B), dim3(512), 0, s, x->x, w.ln1_w,
-                                           w.ln1_b, w.in_w.p, w.in_b, w.conv_w, w.conv_b, w.x_w.p, x->xz, x->xs,
-                                           x->dbc, hist, (int)(x->pos % 3), ein));
+                 if (emb) hipLaunchKernelGGL((k_mixin512<3, MixinOne<true>>), dim3((unsigned)B), dim3(512), 0, s, MixinOne<true>{mt, ein});
+                 else hipLaunchKernelGGL((k_mixin512<3, MixinOne<false>>), dim3((unsigned)B), dim3(512), 0, s, MixinOne<false>{mt, ein}));
         else
             PROF(PC_MIXIN, flops, bytes,
-                 if (emb) hipLaunchKernelGGL((k_mixin512<2, true>), dim3((unsigned)B), dim3(512), 0, s, x->x, w.ln1_w,
-                                           w.ln1_b, w.in_w.p, w.in_b, w.conv_w, w.conv_b, w.x_w.p, x->xz, x->xs,
-                                           x->dbc, hist, (int)(x->pos % 3), ein);
-                 else hipLaunchKernelGGL((k_mixin512<2, false>), dim3((unsigned)B), dim3(512), 0, s, x->x, w.ln1_w,
-                                           w.ln1_b, w.in_w.p, w.in_b, w.conv_w, w.conv_b, w.x_w.p, x->xz, x->xs,
-                                           x->dbc, hist, (int)(x->pos % 3), ein));
+                 if (emb) hipLaunchKernelGGL((k_mixin512<2, MixinOne<true>>), dim3((unsigned)B), dim3(512), 0, s, MixinOne<true>{mt, ein});
+                 else hipLaunchKernelGGL((k_mixin512<2, MixinOne<false>>), dim3((unsigned)B), dim3(512), 0, s, MixinOne<false>{mt, ein}));
     }
     // (fp32 mode included: its fragment-packed weights exist at d_model 256)
     const bool mix = mixin_layer(x, w, Tc);
@@ -3454,28 +3411,16 @@ static int run_layer(boa_ctx* x, int l, int B, int Tc, int part = 7) {
         const double bytes = 4.0 * M * (d + di + di + R + 2 * NS) + 4.0 * 6 * B * di;
         if (x->prec == BOA_PREC_F32)
             PROF(PC_MIXIN, flops, bytes,
-                 if (emb) hipLaunchKernelGGL((k_mixin<1, true>), dim3((unsigned)B), dim3(256), 0, s, x->x, w.ln1_w,
-                                           w.ln1_b, w.in_w.p, w.in_b, w.conv_w, w.conv_b, w.x_w.p, x->xz, x->xs,
-                                           x->dbc, hist, (int)(x->pos % 3), ein);
-                 else hipLaunchKernelGGL((k_mixin<1, false>), dim3((unsigned)B), dim3(256), 0, s, x->x, w.ln1_w,
-                                           w.ln1_b, w.in_w.p, w.in_b, w.conv_w, w.conv_b, w.x_w.p, x->xz, x->xs,
-                                           x->dbc, hist, (int)(x->pos % 3), ein));
+                 if (emb) hipLaunchKernelGGL((k_mixin<1, MixinOne<true>>), dim3((unsigned)B), dim3(256), 0, s, MixinOne<true>{mt, ein});
+                 else hipLaunchKernelGGL((k_mixin<1, MixinOne<false>>), dim3((unsigned)B), dim3(256), 0, s, MixinOne<false>{mt, ein}));
         else if (w.in_w.l)
             PROF(PC_MIXIN, flops, bytes,
-                 if (emb) hipLaunchKernelGGL((k_mixin<3, true>), dim3((unsigned)B), dim3(256), 0, s, x->x, w.ln1_w,
-                                           w.ln1_b, w.in_w.p, w.in_b, w.conv_w, w.conv_b, w.x_w.p, x->xz, x->xs,
-                                           x->dbc, hist, (int)(x->pos % 3), ein);
-                 else hipLaunchKernelGGL((k_mixin<3, false>), dim3((unsigned)B), dim3(256), 0, s, x->x, w.ln1_w,
-                                           w.ln1_b, w.in_w.p, w.in_b, w.conv_w, w.conv_b, w.x_w.p, x->xz, x->xs,
-                                           x->dbc, hist, (int)(x->pos % 3), ein));
+                 if (emb) hipLaunchKernelGGL((k_mixin<3, MixinOne<true>>), dim3((unsigned)B), dim3(256), 0, s, MixinOne<true>{mt, ein});
+                 else hipLaunchKernelGGL((k_mixin<3, MixinOne<false>>), dim3((unsigned)B), dim3(256), 0, s, MixinOne<false>{mt, ein}));
         else
             PROF(PC_MIXIN, flops, bytes,
-                 if (emb) hipLaunchKernelGGL((k_mixin<2, true>), dim3((unsigned)B), dim3(256), 0, s, x->x, w.ln1_w,
-                                           w.ln1_b, w.in_w.p, w.in_b, w.conv_w, w.conv_b, w.x_w.p, x->xz, x->xs,
-                                           x->dbc, hist, (int)(x->pos % 3), ein);
-                 else hipLaunchKernelGGL((k_mixin<2, false>), dim3((unsigned)B), dim3(256), 0, s, x->x, w.ln1_w,
-                                           w.ln1_b, w.in_w.p, w.in_b, w.conv_w, w.conv_b, w.x_w.p, x->xz, x->xs,
-                                           x->dbc, hist, (int)(x->pos % 3), ein));
+                 if (emb) hipLaunchKernelGGL((k_mixin<2, MixinOne<true>>), dim3((unsigned)B), dim3(256), 0, s, MixinOne<true>{mt, ein});
+                 else hipLaunchKernelGGL((k_mixin<2, MixinOne<false>>), dim3((unsigned)B), dim3(256), 0, s, MixinOne<false>{mt, ein}));
     } else if (!mix5 && !mix) {
     // LN1 + in_proj -> xz [M][2di]
     if (part & 1) {
@@ -3538,6 +3483,8 @@ static int run_layer(boa_ctx* x, int l, int B, int Tc, int part = 7) {
         }
     }
     if (!(part & 4)) return BOA_OK;
+    FfnTile f = ffn_tile_args(x, w, 0, M);
+    f.mm = x->mm;
     const bool ffn512 = split && d == ffn5::D && 4 * d == ffn5::DF && w.ff1_w.p && w.ff2_w.p;
     if (ffn512 && x->ffn_outp && w.out_w.p) {
         // out_proj + LN2 + FF1 + GELU + FF2 + residual in one kernel, d_model 512 (mm and the hidden layer kept
@@ -3547,12 +3494,10 @@ static int run_layer(boa_ctx* x, int l, int B, int Tc, int part = 7) {
         const unsigned grid = (unsigned)((M + ffn5::BM - 1) / ffn5::BM);
         if (w.ff1_w.l)
             PROF(PC_FFN, flops, bytes,
-                 hipLaunchKernelGGL((k_ffn512<3, true>), dim3(grid), dim3(512), 0, s, nullptr, w.ln2_w, w.ln2_b,
-                                    w.ff1_w.p, w.ff1_b, w.ff2_w.p, w.ff2_b, x->x, M, x->ah, x->al, w.out_w.p, w.out_b));
+                 hipLaunchKernelGGL((k_ffn512<3, true, FfnTile>), dim3(grid), dim3(512), 0, s, f));
         else
             PROF(PC_FFN, flops, bytes,
-                 hipLaunchKernelGGL((k_ffn512<2, true>), dim3(grid), dim3(512), 0, s, nullptr, w.ln2_w, w.ln2_b,
-                                    w.ff1_w.p, w.ff1_b, w.ff2_w.p, w.ff2_b, x->x, M, x->ah, x->al, w.out_w.p, w.out_b));
+                 hipLaunchKernelGGL((k_ffn512<2, true, FfnTile>), dim3(grid), dim3(512), 0, s, f));
         return BOA_OK;
     }
     // (fp32 mode included: its fragment-packed weights exist at d_model 256; its y is fp32 in place of xs)
@@ -3564,17 +3509,13 @@ static int run_layer(boa_ctx* x, int l, int B, int Tc, int part = 7) {
         const unsigned grid = (unsigned)((M + ffn::BM - 1) / ffn::BM);
         if (!split)
             PROF(PC_FFN, flops, bytes,
-                 hipLaunchKernelGGL((k_ffn<1, true>), dim3(grid), dim3(512), 0, s, nullptr, w.ln2_w, w.ln2_b, w.ff1_w.p,
-                                    w.ff1_b, w.ff2_w.p, w.ff2_b, x->x, M, reinterpret_cast<const uint16_t*>(x->xs),
-                                    nullptr, w.out_w.p, w.out_b));
+                 hipLaunchKernelGGL((k_ffn<1, true, FfnTile>), dim3(grid), dim3(512), 0, s, f));
         else if (w.ff1_w.l)
             PROF(PC_FFN, flops, bytes,
-                 hipLaunchKernelGGL((k_ffn<3, true>), dim3(grid), dim3(512), 0, s, nullptr, w.ln2_w, w.ln2_b, w.ff1_w.p,
-                                    w.ff1_b, w.ff2_w.p, w.ff2_b, x->x, M, x->ah, x->al, w.out_w.p, w.out_b));
+                 hipLaunchKernelGGL((k_ffn<3, true, FfnTile>), dim3(grid), dim3(512), 0, s, f));
         else
             PROF(PC_FFN, flops, bytes,
-                 hipLaunchKernelGGL((k_ffn<2, true>), dim3(grid), dim3(512), 0, s, nullptr, w.ln2_w, w.ln2_b, w.ff1_w.p,
-                                    w.ff1_b, w.ff2_w.p, w.ff2_b, x->x, M, x->ah, x->al, w.out_w.p, w.out_b));
+                 hipLaunchKernelGGL((k_ffn<2, true, FfnTile>), dim3(grid), dim3(512), 0, s, f));
         return BOA_OK;
     }
     // out_proj -> mm [M][d]
@@ -3595,12 +3536,10 @@ static int run_layer(boa_ctx* x, int l, int B, int Tc, int part = 7) {
         const unsigned grid = (unsigned)((M + ffn5::BM - 1) / ffn5::BM);
         if (w.ff1_w.l)
             PROF(PC_FFN, flops, bytes,
-                 hipLaunchKernelGGL((k_ffn512<3, false>), dim3(grid), dim3(512), 0, s, x->mm, w.ln2_w, w.ln2_b,
-                                    w.ff1_w.p, w.ff1_b, w.ff2_w.p, w.ff2_b, x->x, M, nullptr, nullptr, nullptr, nullptr));
+                 hipLaunchKernelGGL((k_ffn512<3, false, FfnTile>), dim3(grid), dim3(512), 0, s, f));
         else
             PROF(PC_FFN, flops, bytes,
-                 hipLaunchKernelGGL((k_ffn512<2, false>), dim3(grid), dim3(512), 0, s, x->mm, w.ln2_w, w.ln2_b,
-                                    w.ff1_w.p, w.ff1_b, w.ff2_w.p, w.ff2_b, x->x, M, nullptr, nullptr, nullptr, nullptr));
+                 hipLaunchKernelGGL((k_ffn512<2, false, FfnTile>), dim3(grid), dim3(512), 0, s, f));
         return BOA_OK;
     }
     if (ffn256) {
@@ -3610,16 +3549,13 @@ static int run_layer(boa_ctx* x, int l, int B, int Tc, int part = 7) {
         const unsigned grid = (unsigned)((M + ffn::BM - 1) / ffn::BM);
         if (!split)
             PROF(PC_FFN, flops, bytes,
-                 hipLaunchKernelGGL((k_ffn<1, false>), dim3(grid), dim3(512), 0, s, x->mm, w.ln2_w, w.ln2_b, w.ff1_w.p,
-                                    w.ff1_b, w.ff2_w.p, w.ff2_b, x->x, M, nullptr, nullptr, nullptr, nullptr));
+                 hipLaunchKernelGGL((k_ffn<1, false, FfnTile>), dim3(grid), dim3(512), 0, s, f));
         else if (w.ff1_w.l)
             PROF(PC_FFN, flops, bytes,
-                 hipLaunchKernelGGL((k_ffn<3, false>), dim3(grid), dim3(512), 0, s, x->mm, w.ln2_w, w.ln2_b, w.ff1_w.p,
-                                    w.ff1_b, w.ff2_w.p, w.ff2_b, x->x, M, nullptr, nullptr, nullptr, nullptr));
+                 hipLaunchKernelGGL((k_ffn<3, false, FfnTile>), dim3(grid), dim3(512), 0, s, f));
         else
             PROF(PC_FFN, flops, bytes,
-                 hipLaunchKernelGGL((k_ffn<2, false>), dim3(grid), dim3(512), 0, s, x->mm, w.ln2_w, w.ln2_b, w.ff1_w.p,
-                                    w.ff1_b, w.ff2_w.p, w.ff2_b, x->x, M, nullptr, nullptr, nullptr, nullptr));
+                 hipLaunchKernelGGL((k_ffn<2, false, FfnTile>), dim3(grid), dim3(512), 0, s, f));
         return BOA_OK;
     }
     // LN2 + FF1 + GELU -> g [M][4d]
@@ -3907,14 +3843,7 @@ int PipeRun::advance(Finish&& finish) {
             st.ssm = x->ssm + ((int64_t)l * x->max_lanes + lane0) * di * NS;
             st.yh = split ? x->ah + ro * di : nullptr; st.yl = split ? x->al + ro * di : nullptr;
             st.Tc = Tc;
-            FfnTile& ft = fa.t[ne];
-            ft.out_b = w.out_b; ft.ln_w = w.ln2_w; ft.ln_b = w.ln2_b; ft.ff1_b = w.ff1_b; ft.ff2_b = w.ff2_b;
-            ft.out_p = w.out_w.p; ft.ff1_p = w.ff1_w.p; ft.ff2_p = w.ff2_w.p;
-            ft.x = x->x + ro * d;
-            ft.yh = split ? st.yh : reinterpret_cast<const uint16_t*>(st.xs);
-            ft.yl = st.yl;
-            ft.hid = x->xz + ro * 2 * di;  // the scan has read z; a row holds the 4 d hidden units
-            ft.M = M;
+            fa.t[ne] = ffn_tile_args(x, w, ro, M);
             rows += M;
             groups64 += (M + 63) / 64;
             max_m = std::max(max_m, M);
@@ -3952,17 +3881,17 @@ int PipeRun::advance(Finish&& finish) {
         hipError_t e = hipSuccess;
         if (d == ffn5::D) {
             PROF(PC_FFN, fflops, fbytes,
-                 if (nt == 3) hipLaunchKernelGGL((k_ffn512_gen<3>), g64, dim3(512), 0, s, fa);
-                 else hipLaunchKernelGGL((k_ffn512_gen<2>), g64, dim3(512), 0, s, fa));
+                 if (nt == 3) hipLaunchKernelGGL((k_ffn512<3, true, FfnTiles>), g64, dim3(512), 0, s, fa);
+                 else hipLaunchKernelGGL((k_ffn512<2, true, FfnTiles>), g64, dim3(512), 0, s, fa));
         } else if (groups64 <= PIPE_ROWS16) {
             const int64_t groups16 = (int64_t)ne * ((max_m + 15) / 16);
             const int fsplit = groups16 * 4 <= x->cus ? 4 : (nt == 1 && groups16 * 2 <= x->cus ? 2 : 1);  // while CUs idle
             PROF(PC_FFN, fflops, fbytes, e = launch_ffn16(fa, ne, max_m, fsplit, nt, s));
         } else {
             PROF(PC_FFN, fflops, fbytes,
-                 if (nt == 1) hipLaunchKernelGGL((k_ffn_gen<1>), g64, dim3(512), 0, s, fa);
-                 else if (nt == 3) hipLaunchKernelGGL((k_ffn_gen<3>), g64, dim3(512), 0, s, fa);
-                 else hipLaunchKernelGGL((k_ffn_gen<2>), g64, dim3(512), 0, s, fa));
+                 if (nt == 1) hipLaunchKernelGGL((k_ffn<1, true, FfnTiles>), g64, dim3(512), 0, s, fa);
+                 else if (nt == 3) hipLaunchKernelGGL((k_ffn<3, true, FfnTiles>), g64, dim3(512), 0, s, fa);
+                 else hipLaunchKernelGGL((k_ffn<2, true, FfnTiles>), g64, dim3(512), 0, s, fa));
         }
         if (e == hipSuccess) e = hipGetLastError();
         if (e != hipSuccess) return boa_fail_hip(e, "run_pipe", __FILE__, __LINE__);

@@ -85,6 +85,7 @@ struct FfnTile {
     const float *out_b, *ln_w, *ln_b, *ff1_b, *ff2_b;
     const uint16_t *out_p, *ff1_p, *ff2_p;
     float* x;
+    const float* mm;          // out_proj's output where it ran on its own (k_ffn and k_ffn512 without OUTP)
     const uint16_t *yh, *yl;  // the scan's output: split parts, or fp32 at yh (fp32 mode)
     float* hid;               // [M][4 d], for k_ffn16 in two launches
     int64_t M;
@@ -92,6 +93,8 @@ struct FfnTile {
 struct FfnTiles {
     FfnTile t[PIPE_MAX];
 };
+__device__ __forceinline__ const FfnTile& ffn_tile(const FfnTile& a) { return a; }
+__device__ __forceinline__ const FfnTile& ffn_tile(const FfnTiles& a) { return a.t[blockIdx.y]; }
 // d_model 256, 16 rows per workgroup (fused_step.hip): for launches whose tiles are too few for k_ffn's 64-row workgroups
 // split: workgroups per 16 rows (1, 4, in the fp32 mode also 2).
 hipError_t launch_ffn16(const FfnTiles& a, int tiles, int64_t max_rows, int split, int nt, hipStream_t s);
