@@ -840,12 +840,15 @@ __device__ __forceinline__ int h_off(int r, int k) { return r * HC + (((k >> 3) 
 // out_proj outputs 32 w .. + 31 of all 64 rows; its 32 W_out blocks stream through a 4-slot ring.
 // A: FfnTile, or FfnTiles for several tiles in one launch (blockIdx.y picks the tile; rows past a tile's M read 0 and
 // store nothing).  One kernel template for both, its body in the kernel itself: as a device function called from two
-// kernels the same body took 128 registers and spilled 53 (fp32) and 40 (bf16x3) in either kernel.
+// kernels the same body took 128 registers and spilled 53 (fp32) and 40 (bf16x3) in either kernel.  (The one-tile form's
+// grid covers its rows exactly; with the other's early return it took 122 registers instead of 118.)
 template <int NT, bool OUTP, class A>
 __global__ void __launch_bounds__(512, 4) k_ffn(A a) {
     const FfnTile& tile = ffn_tile(a);
     const int64_t M = tile.M;
-    if ((int64_t)blockIdx.x * ffn::BM >= M) return;
+    if constexpr (std::is_same_v<A, FfnTiles>) {
+        if ((int64_t)blockIdx.x * ffn::BM >= M) return;
+    }
     const float *mm = tile.mm, *ln_w = tile.ln_w, *ln_b = tile.ln_b, *b1 = tile.ff1_b, *b2 = tile.ff2_b, *bo = tile.out_b;
     const uint16_t *W1p = tile.ff1_p, *W2p = tile.ff2_p, *yh = tile.yh, *yl = tile.yl, *Wop = tile.out_p;
     float* x = tile.x;
@@ -1142,7 +1145,9 @@ template <int NT, bool OUTP, class A>
 __global__ void __launch_bounds__(512, 2) k_ffn512(A a) {
     const FfnTile& tile = ffn_tile(a);
     const int64_t M = tile.M;
-    if ((int64_t)blockIdx.x * ffn5::BM >= M) return;
+    if constexpr (std::is_same_v<A, FfnTiles>) {
+        if ((int64_t)blockIdx.x * ffn5::BM >= M) return;
+    }
     const float *mm = tile.mm, *ln_w = tile.ln_w, *ln_b = tile.ln_b, *b1 = tile.ff1_b, *b2 = tile.ff2_b, *bo = tile.out_b;
     const uint16_t *W1p = tile.ff1_p, *W2p = tile.ff2_p, *yh = tile.yh, *yl = tile.yl, *Wop = tile.out_p;
     float* x = tile.x;
