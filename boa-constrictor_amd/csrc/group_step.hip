@@ -358,7 +358,8 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
         // the first to decide for this launch: `was` holds an earlier launch's decision
         auto decide = [&](uint64_t was, uint64_t how) {
             if (was != open && was != shut)
-                __hip_atomic_compare_exchange_strong(gate, &was, how, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                return __hip_atomic_compare_exchange_strong(gate, &was, how, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return false;
         };
         const uint64_t n = __hip_atomic_fetch_add(gate + 1, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         uint64_t st = state();
@@ -366,7 +367,8 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
         const uint64_t t0 = wall_clock64();
         while (st != open && st != shut) {
             st = state();
-            if (wall_clock64() - t0 > a0.gate_ticks) decide(st, shut);
+            if (wall_clock64() - t0 > a0.gate_ticks && decide(st, shut))
+                __hip_atomic_fetch_add(gate + 2, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         sGo = st == open ? 1 : 0;
     }

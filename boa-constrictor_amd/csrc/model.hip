@@ -2719,7 +2719,7 @@ struct boa_ctx {
     // decode steps with several workgroups per 16 lanes (BOA_GROUP_STEP=0: the fused kernels only)
     uint64_t* xch = nullptr;
     int32_t* xbad = nullptr;
-    uint64_t* xgate = nullptr;         // where a group launch's workgroups meet: [decisions, arrivals]
+    uint64_t* xgate = nullptr;         // where a group launch's workgroups meet: [decisions, arrivals, shut out]
     uint64_t xarrived = 0;             // arrivals so far
     bool group_shut = false;           // BOA_GROUP_STEP=shut: the gate never opens (tests of the launch that then follows)
     uint32_t xseq = 1;                 // the next sequence number of an exchange packet
@@ -2794,6 +2794,17 @@ extern "C" int boa_profile_read(boa_ctx* x, boa_prof_entry* out, int32_t cap, in
             e.ms = ms;
             e.flops = p.flops;
             e.bytes = p.bytes;
+        }
+        ++k;
+    }
+    // group launches of the context that did not all get onto the GPU in time (the fused kernel did their work)
+    uint64_t shut = 0;
+    if (x->xgate) BOA_HIP_TRY(hipMemcpy(&shut, x->xgate + 2, sizeof(shut), hipMemcpyDeviceToHost));
+    if (shut) {
+        if (k < cap) {
+            memset(&out[k], 0, sizeof(out[k]));
+            snprintf(out[k].name, sizeof(out[k].name), "group_shut_out");
+            out[k].launches = (int64_t)shut;
         }
         ++k;
     }
@@ -3701,7 +3712,7 @@ static hipError_t launch_fused(boa_ctx* x, FusedArgs& a, hipStream_t s) {
             cap = hipStreamCaptureStatusActive;
         }
         if (cap == hipStreamCaptureStatusNone) {
-            a.xch = x->xch; a.bad = x->xbad; a.seq0 = x->xseq; a.gate = x->xgate; a.arrived = x->group_shut ? ~0ull : x->xarrived;
+            a.xch = x->xch; a.bad = x->xbad; a.seq0 = x->xseq; a.gate = x->xgate; a.arrived = x->group_shut ? GATE_NEVER : x->xarrived;
             a.gate_ticks = 50000u + 5000u * (uint32_t)a.nsteps;  // 0.5 ms and 50 us per step
             const hipError_t e = launch_group_step(a, x->d, nt, g, s);
             if (e != hipSuccess) return e;

@@ -64,7 +64,8 @@ struct FusedArgs {
     float* scr;
     // group_step.hip: the exchange packets, the first sequence number of this launch, and where an expired wait is
     // reported; the gate its workgroups meet at (gate[0]: the launches' decisions, 2 seq0 + 1 for "not all here";
-    // gate[1]: arrivals, `arrived` before this launch) and how long they wait there, in 10 ns
+    // gate[1]: arrivals, `arrived` before this launch, or GATE_NEVER; gate[2]: launches that were shut out) and how long
+    // they wait there, in 10 ns
     uint64_t* xch;
     uint32_t seq0;
     int32_t* bad;
@@ -74,6 +75,7 @@ struct FusedArgs {
     // fused kernels: run only if the group launch with this decision word (2 seq0 + 1) did not start (0: always run)
     uint64_t only_if;
 };
+constexpr uint64_t GATE_NEVER = 1ull << 63;  // `arrived` of a launch whose gate no count of arrivals opens
 // Whether a fused launch is left out: it follows a group launch that did run.
 __device__ __forceinline__ bool left_out(const FusedArgs& a) { return a.only_if != 0 && a.gate[0] != a.only_if; }
 
@@ -131,7 +133,7 @@ hipError_t launch_fused_step512(const FusedArgs& a, int nt, hipStream_t s);
 constexpr int GROUP_MAX = 128;  // groups of 16 lanes at most
 int64_t group_step_bytes(int d_model, int64_t max_lanes);     // exchange packets, in bytes
 int group_step_width(int d_model, int lanes, int cus);         // workgroups per group on a GPU of that many CUs; 1: none
-constexpr int GROUP_GATE_WORDS = 2;
+constexpr int GROUP_GATE_WORDS = 3;
 // takes 1 + nsteps (L + 1) sequence numbers from a.seq0 on; adds group_step_blocks to the gate's arrivals.  Does nothing
 // (and says so at the gate) if its workgroups do not all get onto the GPU in time: a fused launch with only_if follows.
 int64_t group_step_blocks(int lanes, int g);

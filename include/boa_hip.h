@@ -110,7 +110,9 @@ typedef struct boa_prof_entry {
 } boa_prof_entry;
 /* enable != 0 starts a fresh window; 0 stops recording. */
 int boa_profile(boa_ctx* ctx, int enable);
-/* Synchronizes, resolves the recorded events and copies up to cap entries; *n receives the count.      */
+/* Synchronizes, resolves the recorded events and copies up to cap entries; *n receives the count.  An entry
+ * "group_shut_out" (launches alone) counts the context's few-lane step launches, since its creation, that did
+ * not get all their workgroups onto the GPU in time, so that the one-workgroup kernel did their work.        */
 int boa_profile_read(boa_ctx* ctx, boa_prof_entry* out, int32_t cap, int32_t* n);
 
 /* ------------------------------------------------------------------------------------------------ */

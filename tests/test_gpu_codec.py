@@ -622,6 +622,46 @@ def test_group_step_matches_fused_kernels(gpu, monkeypatch, d_model, precision, 
             assert np.array_equal(got["0"][1], got[other][1]), (n, other)
 
 
+def _shut_out(gpu, eng):
+    """How many of the context's group launches did not start (the fused kernel did their work)."""
+    import ctypes
+
+    from boa_amd import _native as N
+
+    ents, n = (N.ProfEntry * 32)(), ctypes.c_int32(0)
+    N.check(gpu.boa_profile_read(eng.h, ents, 32, ctypes.byref(n)))
+    return sum(e.launches for e in ents[:n.value] if e.name == b"group_shut_out")
+
+
+@pytest.mark.parametrize("d_model,precision,n", [(256, "f32", 1), (256, "f32", 20), (256, "bf16x3", 300), (512, "bf16w", 17)])
+def test_shut_gate_leaves_the_work_to_the_fused_kernel(gpu, monkeypatch, d_model, precision, n):
+    """A group launch whose workgroups do not meet does nothing at all, from a context's first launch on: steps and a
+    decode over several launches give the fused kernels' values, and every group launch counts as shut out."""
+    import codec
+    import model as M
+    from boa_amd import weights as W
+
+    monkeypatch.setenv("BOA_FUSED_STEPS_PER_LAUNCH", "4")
+    blob = W.seeded_blob(W.Cfg(d_model=d_model, n_layers=2), 7)
+    got = {}
+    for group in ("0", "shut", "1"):
+        monkeypatch.setenv("BOA_GROUP_STEP", group)
+        rng = np.random.default_rng(n)
+        m = M.BoaConstrictor(d_model, 2, 256).load_blob(blob)
+        m.precision = precision
+        inf = m.init_stream(max_len=8, batch_size=n)
+        logits = [m.step(torch.from_numpy(rng.integers(0, 256, n).astype(np.int32)).cuda(), inf).cpu() for _ in range(3)]
+        nw = rng.integers(0, 9, n)
+        payload = rng.integers(0, 1 << 32, int(nw.sum()), dtype=np.uint64).astype(np.uint32)
+        out = codec.decompress_payload(m, payload, nw, [14] * n, rng.integers(0, 256, n).tolist())
+        got[group] = (logits, out)
+        want = {"0": (0, 0), "shut": (3, 4), "1": (0, 0)}[group]
+        assert (_shut_out(gpu, inf.engine), _shut_out(gpu, m._engines["codec"][1])) == want
+    for group in ("shut", "1"):
+        assert all(torch.equal(a, b) for a, b in zip(got["0"][0], got[group][0]))
+        assert np.array_equal(got["0"][1], got[group][1])
+
+
 def test_step_under_capture(gpu):
     """A step recorded into a graph (which cannot hold the group kernel's sequence numbers) replays as the eager step
     from the same state."""
