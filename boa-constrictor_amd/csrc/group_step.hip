@@ -32,9 +32,11 @@
 // written: the last to arrive opens it; the first to find its time up (another kernel holds the CUs) closes it for this
 // launch, all of them leave, and the fused launch that follows does the work (left_out).  Beyond the gate every wait ends
 // because its partners run.  (A cooperative launch gives the same guarantee but took 80 us longer per launch, of a step's
-// 187.)  The waits are bounded all the same (WAIT_TICKS): if one expires, the workgroup stops waiting for good, reports it
-// in *bad, and gives NaN logits.  With more groups than CUs / 2 the fused kernels, one workgroup per group, fill the GPU
-// and have no exchange.
+// 187.)  The waits are bounded all the same (wait_ticks): if one expires (the process was taken off the GPU for seconds),
+// the workgroup stops waiting for good, goes through the rest of the launch on whatever it holds, and notes the launch in
+// CTL_EXPIRED and for the host.  What the others make of its packets is as void as its own results: the launch that
+// follows sees the note and sets all logits to NaN, as do all steps until the state is reset, and the host refuses the
+// next call.  With more groups than CUs / 2 the fused kernels, one workgroup per group, fill the GPU and have no exchange.
 //
 // Arithmetic: every GEMM output accumulates its K steps in ascending order through mfma_split_step_t, x_proj is the left
 // fold of 64-channel partials, and every elementwise step is the shared function of model_dev.h, as in the fused and
@@ -53,9 +55,15 @@ namespace boa {
 namespace {
 
 constexpr int ROWS = 16, NTHR = 512, NWAVE = 8, NS = 16, VV = 256;
-constexpr uint64_t WAIT_TICKS = 300000000ull;  // of the 100 MHz wall clock
-
 typedef uint64_t Packet;
+
+typedef __attribute__((address_space(4))) const FusedArgs KArgs;
+// kernel arguments through an opaque pointer (kept out of SGPRs across the step loop and the waits)
+__device__ __forceinline__ KArgs& kargs() {
+    auto kp = (__attribute__((address_space(4))) const char*)__builtin_amdgcn_kernarg_segment_ptr();
+    __asm__ volatile("" : "+s"(kp));
+    return *reinterpret_cast<KArgs*>(kp);
+}
 
 // exchange regions of one group, in packets
 template <int D>
@@ -80,8 +88,7 @@ typedef uint32_t bufv2 __attribute__((vector_size(8)));
 struct Link {
     __amdgpu_buffer_rsrc_t x;
     bool near;
-    volatile int* dead;
-    int32_t* bad;
+    volatile uint32_t* limit;  // of a wait, in ticks of the 100 MHz wall clock; 0: the workgroup waits no more
 };
 __device__ __forceinline__ void send(const Link& k, uint32_t at, uint32_t seq, uint32_t v) {
     if (k.near) __builtin_amdgcn_raw_buffer_store_b64(bufv2{v, seq}, k.x, at * 8, 0, CPOL_GROUP);
@@ -114,12 +121,16 @@ __device__ __forceinline__ void receive(const Link& k, const uint32_t (&at)[N], 
             v[2 * i] = w[i].x;
             v[2 * i + 1] = w[i].z;
         }
-        if (off == 0u || *k.dead) return;
+        const uint32_t limit = *k.limit;
+        if (off == 0u || limit == 0u) return;
         const uint64_t now = wall_clock64();
         if (t0 == 0) t0 = now;
-        if (now - t0 > WAIT_TICKS) {
-            *k.dead = 1;
-            *k.bad = 1;
+        if (now - t0 >= limit) {
+            KArgs& a = kargs();
+            const uint64_t launch = 2ull * a.seq0 + 1ull;
+            *k.limit = 0u;
+            __hip_atomic_store(a.ctl + CTL_EXPIRED, launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(a.host_expired, launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             return;
         }
     }
@@ -306,7 +317,6 @@ __device__ __forceinline__ Ids ids() {
     const int tid = id_.tid, lane = id_.lane, lane16 = id_.lane16, row = id_.row, cq = id_.cq;          \
     const bool live = row < nb;                                                                         \
     (void)tid; (void)lane; (void)lane16; (void)row; (void)cq; (void)live;
-typedef __attribute__((address_space(4))) const FusedArgs KArgs;
 // the layer's parameter table entry from opaque copies of its index (its pointers are loaded again where they are used)
 #define LAYER                                 \
     int l_ = l;                               \
@@ -338,7 +348,8 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
     __shared__ __attribute__((aligned(16))) float sDbc[ROWS * FW];
     __shared__ floatx4 sAcc[NWAVE * 64 / 2];
     __shared__ int sTok[ROWS];
-    __shared__ int sDead, sMaxLen, sGo;
+    __shared__ int sMaxLen, sGo;
+    __shared__ uint32_t sLimit;
     float* sXZ = reinterpret_cast<float*>(op + OFF_XZ);
     unsigned char* sCv = op + OFF_CV;
 
@@ -348,12 +359,12 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
     const int64_t b0 = (int64_t)group * ROWS;
     if (b0 >= a0.B) return;
     const int nb = (int)((a0.B - b0) < ROWS ? (a0.B - b0) : ROWS);
-    volatile int* dead = &sDead;
+    volatile uint32_t* limit = &sLimit;
     // ---- the gate
     if (threadIdx.x == 0) {
         const uint64_t open = 2ull * a0.seq0, shut = open + 1ull;
         const uint64_t total = (uint64_t)((a0.B + ROWS - 1) / ROWS) * G;
-        uint64_t* const gate = a0.gate;
+        uint64_t* const gate = a0.ctl + CTL_GATE;
         auto state = [&]() { return __hip_atomic_load(gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
         // the first to decide for this launch: `was` holds an earlier launch's decision
         auto decide = [&](uint64_t was, uint64_t how) {
@@ -361,16 +372,18 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
                 return __hip_atomic_compare_exchange_strong(gate, &was, how, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return false;
         };
-        const uint64_t n = __hip_atomic_fetch_add(gate + 1, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // an earlier launch spoilt the state (this one's own waits come after every arrival): all leave
+        const bool spoilt = a0.ctl[CTL_EXPIRED] >= a0.valid_from;
+        const uint64_t n = __hip_atomic_fetch_add(a0.ctl + CTL_ARRIVED, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         uint64_t st = state();
         if (n - a0.arrived == total - 1) decide(st, open);
         const uint64_t t0 = wall_clock64();
-        while (st != open && st != shut) {
+        while (!spoilt && st != open && st != shut) {
             st = state();
             if (wall_clock64() - t0 > a0.gate_ticks && decide(st, shut))
-                __hip_atomic_fetch_add(gate + 2, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_fetch_add(a0.ctl + CTL_SHUT_OUT, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        sGo = st == open ? 1 : 0;
+        sGo = !spoilt && st == open ? 1 : 0;
     }
     __syncthreads();
     if (!sGo) return;
@@ -382,7 +395,7 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
             if (a0.decode)
                 for (int r = 0; r < nb; ++r) ml = a0.lens[b0 + r] > ml ? a0.lens[b0 + r] : ml;
             sMaxLen = ml;
-            sDead = 0;
+            sLimit = a0.wait_ticks;
         }
     }
     // coder state of this wave's rows 2 wave, 2 wave + 1 (every member keeps its own copy)
@@ -396,9 +409,9 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
     // whether every member found itself on the same XCD (HW_REG_XCC_ID)
     bool near;
     {
-        const Link far = {buf_rsrc(reinterpret_cast<Packet*>(a0.xch) + (int64_t)group * XC::SIZE, XC::SIZE * 8), false, dead, a0.bad};
+        const Link far = {buf_rsrc(reinterpret_cast<Packet*>(a0.xch) + (int64_t)group * XC::SIZE, XC::SIZE * 8), false, limit};
         const uint32_t xcc = __builtin_amdgcn_s_getreg(20 | (3 << 11));
-        if (threadIdx.x == 0) send(far, XC::W + member, a0.seq0, xcc);
+        if (threadIdx.x == 0) send(far, XC::W + member, a0.seq_first, xcc);
         uint32_t at[G / 2], v[G], differ = 0;
 #pragma unroll
         for (int i = 0; i < G / 2; ++i) at[i] = XC::W + 2 * i;
@@ -424,13 +437,10 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
     int p0m3 = a0.p0m3;
 #pragma unroll 1
     for (int step = 0; step < a0.nsteps; ++step) {
-        // kernel arguments through an opaque pointer (kept out of SGPRs across the step loop)
-        auto kp = (__attribute__((address_space(4))) const char*)__builtin_amdgcn_kernarg_segment_ptr();
-        __asm__ volatile("" : "+s"(kp));
-        KArgs& a = *reinterpret_cast<KArgs*>(kp);
+        KArgs& a = kargs();
         const int t = a.t + step;
         if (a.decode && t >= sMaxLen) break;  // every lane of the group is complete (the same for every member)
-        const Link xc = {buf_rsrc(reinterpret_cast<Packet*>(a.xch) + (int64_t)group * XC::SIZE, XC::SIZE * 8), near, dead, a.bad};
+        const Link xc = {buf_rsrc(reinterpret_cast<Packet*>(a.xch) + (int64_t)group * XC::SIZE, XC::SIZE * 8), near, limit};
         const uint32_t seq0 = a.seq0 + 1u + (uint32_t)step * (uint32_t)(a.L + 1);
         const int s1 = p0m3 == 2 ? 0 : p0m3 + 1, s2 = p0m3 == 0 ? 2 : p0m3 - 1;
         const int V = a.V;
@@ -818,12 +828,11 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
             IDS
             float v[2][4];
             receive_rows(XC::LG, WV{}, seqh, v, lane);
-            const float nan = __builtin_nanf("");
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
                 const int r = 2 * wave + q;
                 if (r >= nb) continue;
-                const float4 l4 = *dead ? make_float4(nan, nan, nan, nan) : make_float4(v[q][0], v[q][1], v[q][2], v[q][3]);
+                const float4 l4 = make_float4(v[q][0], v[q][1], v[q][2], v[q][3]);
                 if (a.logits && member == r % G) stg_f4(boa::GM(a.logits) + (b0 + r) * VV + 4 * lane, l4);
                 if (a.decode && t < a.lens[b0 + r]) {
                     const LaneWords words = lane_words(a.payload, a.payload_words, a.off, a.nwords, b0 + r);

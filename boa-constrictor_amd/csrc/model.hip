@@ -2563,6 +2563,12 @@ __global__ void __launch_bounds__(256) k_state_zero(float* __restrict__ hist, in
     for (int64_t i = i0; i < lanes * ns; i += stride) *reinterpret_cast<float4*>(ssm + l * max_lanes * ns + i) = z;
 }
 
+// Logits of a forward that continued a state which an expired wait had spoilt (left_out's test): NaN.
+__global__ void __launch_bounds__(256) k_void_logits(float* __restrict__ logits, int64_t n, const uint64_t* __restrict__ expired,
+                                                    uint64_t valid_from) {
+    if (*expired >= valid_from) void_logits(logits, n);
+}
+
 __global__ void k_enc_finish(EncState* states, uint32_t* words, int64_t pitch, int32_t* nwords, int32_t* overflow,
                              int n) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2718,11 +2724,18 @@ struct boa_ctx {
     int64_t ws_rows = 0;
     // decode steps with several workgroups per 16 lanes (BOA_GROUP_STEP=0: the fused kernels only)
     uint64_t* xch = nullptr;
-    int32_t* xbad = nullptr;
-    uint64_t* xgate = nullptr;         // where a group launch's workgroups meet: [decisions, arrivals, shut out]
-    uint64_t xarrived = 0;             // arrivals so far
-    bool group_shut = false;           // BOA_GROUP_STEP=shut: the gate never opens (tests of the launch that then follows)
+    uint64_t* xctl = nullptr;          // control words (CTL_*)
+    uint64_t xarrived = 0;             // arrivals at the gate so far
     uint32_t xseq = 1;                 // the next sequence number of an exchange packet
+    // an expired wait: the launch it was in (pinned host memory, 0: none), the first launch since the state was reset,
+    // whether the state has gone through a group launch since then, and whether group launches are given up
+    uint64_t* xexpired = nullptr;
+    uint64_t valid_from = 2;
+    bool grouped = false;
+    bool group_off = false;
+    // tests, by BOA_GROUP_STEP: the gate never opens (shut); a launch's first packets carry a number that nobody waits
+    // for, and the wait is short (expire)
+    bool group_shut = false, group_expire = false;
     int cus = 0;
     hipStream_t stream2 = nullptr;
     hipStream_t stream3 = nullptr;     // the third compress group's
@@ -2799,7 +2812,7 @@ extern "C" int boa_profile_read(boa_ctx* x, boa_prof_entry* out, int32_t cap, in
     }
     // group launches of the context that did not all get onto the GPU in time (the fused kernel did their work)
     uint64_t shut = 0;
-    if (x->xgate) BOA_HIP_TRY(hipMemcpy(&shut, x->xgate + 2, sizeof(shut), hipMemcpyDeviceToHost));
+    if (x->xctl) BOA_HIP_TRY(hipMemcpy(&shut, x->xctl + CTL_SHUT_OUT, sizeof(shut), hipMemcpyDeviceToHost));
     if (shut) {
         if (k < cap) {
             memset(&out[k], 0, sizeof(out[k]));
@@ -2914,7 +2927,7 @@ static int64_t ctx_plan_bytes(const boa_model_cfg& c, int R, int precision, int6
         b += 2 * std::max<int64_t>(2 * mats, 1);  // fp32 fragment-packed weights, in 16-bit units
     }
     if (want_fused(c, R, precision)) b += (int64_t)sizeof(FusedLayer) * L;
-    if (want_group(c, R, precision)) b += group_step_bytes(c.d_model, max_lanes) + (int64_t)sizeof(int32_t) + 8 * GROUP_GATE_WORDS;
+    if (want_group(c, R, precision)) b += group_step_bytes(c.d_model, max_lanes) + 8 * CTL_WORDS;
     return b;
 }
 
@@ -2937,9 +2950,10 @@ extern "C" int boa_ctx_destroy(boa_ctx* ctx) {
     else (void)hipDeviceSynchronize();
     void* ptrs[] = {ctx->wblob, ctx->aneg, ctx->conv_hist, ctx->ssm, ctx->x, ctx->xz, ctx->xs, ctx->dbc,
                     ctx->mm, ctx->logits, ctx->stats, ctx->tokens, ctx->enc, ctx->dec, ctx->flag, ctx->wsplit,
-                    ctx->ah, ctx->al, ctx->wfrag, ctx->d_layers, ctx->xch, ctx->xbad, ctx->xgate};
+                    ctx->ah, ctx->al, ctx->wfrag, ctx->d_layers, ctx->xch, ctx->xctl};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
+    if (ctx->xexpired) (void)hipHostFree(ctx->xexpired);
     for (auto& p : ctx->prof)
         for (hipEvent_t e : p.ev) (void)hipEventDestroy(e);
     for (hipEvent_t e : ctx->half_ev) (void)hipEventDestroy(e);
@@ -3165,11 +3179,11 @@ extern "C" int boa_ctx_create(const boa_model_cfg* cfg, const void* h_weights, i
         const int64_t n = group_step_bytes(c.d_model, max_lanes) / 8;
         int dev = 0;
         e = dmalloc(x, &x->xch, n);
-        if (e == hipSuccess) e = dmalloc(x, &x->xbad, 1);
-        if (e == hipSuccess) e = dmalloc(x, &x->xgate, GROUP_GATE_WORDS);
-        if (e == hipSuccess) e = hipMemsetAsync(x->xgate, 0, 8 * GROUP_GATE_WORDS, x->stream);
+        if (e == hipSuccess) e = dmalloc(x, &x->xctl, CTL_WORDS);
+        if (e == hipSuccess) e = hipMemsetAsync(x->xctl, 0, 8 * CTL_WORDS, x->stream);
         if (e == hipSuccess) e = hipMemsetAsync(x->xch, 0, (size_t)n * 8, x->stream);  // sequence number 0: none
-        if (e == hipSuccess) e = hipMemsetAsync(x->xbad, 0, sizeof(int32_t), x->stream);
+        if (e == hipSuccess) e = hipHostMalloc((void**)&x->xexpired, sizeof(uint64_t), hipHostMallocDefault);
+        if (e == hipSuccess) *x->xexpired = 0;
         if (e == hipSuccess) e = hipGetDevice(&dev);
         if (e == hipSuccess) e = hipDeviceGetAttribute(&x->cus, hipDeviceAttributeMultiprocessorCount, dev);
     }
@@ -3203,7 +3217,10 @@ extern "C" int boa_ctx_create(const boa_model_cfg* cfg, const void* h_weights, i
         boa_ctx_destroy(x);
         return boa_fail_hip(e, "boa_ctx_create upload", __FILE__, __LINE__);
     }
-    if (const char* v = getenv("BOA_GROUP_STEP")) x->group_shut = strcmp(v, "shut") == 0;
+    if (const char* v = getenv("BOA_GROUP_STEP")) {
+        x->group_shut = strcmp(v, "shut") == 0;
+        x->group_expire = strcmp(v, "expire") == 0;
+    }
     if (const char* v = getenv("BOA_DECODE_HALVES")) x->decode_halves = atoi(v) == 1 ? 1 : 2;
     if (const char* v = getenv("BOA_FFN_OUTP")) x->ffn_outp = atoi(v) != 0;
     if (const char* v = getenv("BOA_HEAD_XQ")) x->head_xq = atoi(v) != 0;
@@ -3234,9 +3251,29 @@ extern "C" int boa_ctx_create(const boa_model_cfg* cfg, const void* h_weights, i
     return BOA_OK;
 }
 
+// Whether a wait between workgroups expired since the state was reset, as far as the host has heard of it.  The fused
+// kernels then take all later steps: what took the process off the GPU may do it again.
+static bool wait_expired(boa_ctx* x) {
+    if (!x->xexpired || __atomic_load_n(x->xexpired, __ATOMIC_RELAXED) < x->valid_from) return false;
+    x->group_off = true;
+    return true;
+}
+static int fail_expired(const char* who) {
+    return boa_fail(BOA_ERR_HIP, "%s: a wait between workgroups expired; the state has to be reset", who);
+}
+static bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 extern "C" int boa_state_reset(boa_ctx* x, int32_t lanes) {
     if (!x || lanes < 0 || lanes > x->max_lanes) return boa_fail(BOA_ERR_ARG, "boa_state_reset: bad lanes");
     x->pos = 0;
+    (void)wait_expired(x);
+    x->valid_from = 2ull * x->xseq;
+    x->grouped = false;
     if (lanes == 0) return BOA_OK;
     // one launch for all layers (two memsets per layer took 2 us each plus their gaps: 60 us at 8 layers)
     const int64_t ns = (int64_t)x->di * x->NS;
@@ -3702,22 +3739,21 @@ static FusedArgs fused_args(boa_ctx* x, int32_t lanes, const int32_t* tokens_in)
 
 static hipError_t launch_fused(boa_ctx* x, FusedArgs& a, hipStream_t s) {
     const int nt = x->prec == BOA_PREC_BF16X3 ? 3 : (x->prec == BOA_PREC_BF16W ? 2 : 1);
-    const int g = x->xch ? group_step_width(x->d, a.B, x->cus) : 1;
-    a.only_if = 0;
-    if (g > 1) {
-        // a stream that is being captured takes the fused kernel: replays would repeat the sequence numbers
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
-            (void)hipGetLastError();
-            cap = hipStreamCaptureStatusActive;
-        }
-        if (cap == hipStreamCaptureStatusNone) {
-            a.xch = x->xch; a.bad = x->xbad; a.seq0 = x->xseq; a.gate = x->xgate; a.arrived = x->group_shut ? GATE_NEVER : x->xarrived;
+    // a stream that is being captured takes the fused kernel: replays would repeat the sequence numbers
+    if (x->xch && !x->group_off && !capturing(s)) {
+        a.ctl = x->xctl; a.valid_from = x->valid_from;
+        const int g = group_step_width(x->d, a.B, x->cus);
+        if (g > 1) {
+            a.xch = x->xch; a.seq0 = x->xseq; a.arrived = x->group_shut ? GATE_NEVER : x->xarrived;
             a.gate_ticks = 50000u + 5000u * (uint32_t)a.nsteps;  // 0.5 ms and 50 us per step
+            a.seq_first = x->group_expire ? 0u : a.seq0;     // (0: the number of a packet never written)
+            a.wait_ticks = x->group_expire ? 1000u : 300000000u;  // 10 us, 3 s
+            a.host_expired = x->xexpired;
             const hipError_t e = launch_group_step(a, x->d, nt, g, s);
             if (e != hipSuccess) return e;
             x->xseq += 1u + (uint32_t)a.nsteps * (uint32_t)(x->L + 1);
             x->xarrived += (uint64_t)group_step_blocks(a.B, g);
+            x->grouped = true;
             a.only_if = 2ull * a.seq0 + 1ull;  // then the fused launch, which leaves if the group launch ran
         }
     }
@@ -3749,6 +3785,7 @@ static double fused_flops(const boa_ctx* x, int32_t lanes) {
 extern "C" int boa_model_step(boa_ctx* x, const int32_t* d_tokens, int32_t lanes, float* d_logits) {
     if (!x || !d_tokens || !d_logits || lanes < 1 || lanes > x->max_lanes)
         return boa_fail(BOA_ERR_ARG, "boa_model_step: bad arguments");
+    if (wait_expired(x)) return fail_expired("boa_model_step");
     if (x->fused) {
         FusedArgs a = fused_args(x, lanes, d_tokens);
         a.logits = d_logits;
@@ -3986,10 +4023,7 @@ static bool head_xq_any(const boa_ctx* x);
 static int launch_head_xq(boa_ctx* x, const float* xin, int lanes, int Tc, int t0, const uint8_t* bytes, int64_t stride,
                           const int32_t* lens, uint2* lf, float* logits, int64_t len);
 
-extern "C" int boa_model_forward(boa_ctx* x, const int32_t* d_tokens, int64_t tok_stride, int32_t lanes, int32_t len,
-                                 float* d_logits) {
-    if (!x || !d_tokens || !d_logits || lanes < 1 || lanes > x->max_lanes || len < 0 || tok_stride < len)
-        return boa_fail(BOA_ERR_ARG, "boa_model_forward: bad arguments");
+static int forward(boa_ctx* x, const int32_t* d_tokens, int64_t tok_stride, int32_t lanes, int32_t len, float* d_logits) {
     if (len > 0 && pipe_ok(x, lanes)) {
         EmbedIn src;
         src.tokens = d_tokens; src.stride = tok_stride; src.emb = x->emb; src.V = x->V;
@@ -4020,6 +4054,20 @@ extern "C" int boa_model_forward(boa_ctx* x, const int32_t* d_tokens, int64_t to
         hipLaunchKernelGGL(k_scatter_logits, dim3(row_blocks(rows)), dim3(256), 0, x->stream, x->logits, x->V, Tc, t0,
                            len, rows, d_logits);
     }
+    BOA_HIP_TRY(hipGetLastError());
+    return BOA_OK;
+}
+
+extern "C" int boa_model_forward(boa_ctx* x, const int32_t* d_tokens, int64_t tok_stride, int32_t lanes, int32_t len,
+                                 float* d_logits) {
+    if (!x || !d_tokens || !d_logits || lanes < 1 || lanes > x->max_lanes || len < 0 || tok_stride < len)
+        return boa_fail(BOA_ERR_ARG, "boa_model_forward: bad arguments");
+    if (wait_expired(x)) return fail_expired("boa_model_forward");
+    const int rc = forward(x, d_tokens, tok_stride, lanes, len, d_logits);
+    if (rc || len == 0 || !x->grouped || capturing(x->stream)) return rc;
+    // the state came through group launches that the host has not heard from yet
+    hipLaunchKernelGGL(k_void_logits, dim3(256), dim3(256), 0, x->stream, d_logits, (int64_t)lanes * len * x->V,
+                       x->xctl + CTL_EXPIRED, x->valid_from);
     BOA_HIP_TRY(hipGetLastError());
     return BOA_OK;
 }
@@ -4234,10 +4282,8 @@ extern "C" int boa_decompress(boa_ctx* x, const uint32_t* d_payload, int64_t pay
             if (e != hipSuccess) return boa_fail_hip(e, "k_fused_step", __FILE__, __LINE__);
             x->pos += a.nsteps;
         }
-        int32_t bad = 0;
-        if (x->xbad) BOA_HIP_TRY(hipMemcpyAsync(&bad, x->xbad, sizeof(int32_t), hipMemcpyDeviceToHost, s));
         BOA_HIP_TRY(hipStreamSynchronize(s));
-        if (bad) return boa_fail(BOA_ERR_HIP, "boa_decompress: a wait between workgroups expired");
+        if (wait_expired(x)) return fail_expired("boa_decompress");
         return BOA_OK;
     }
     if (x->stream2 && lanes >= 512) {

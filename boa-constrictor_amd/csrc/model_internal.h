@@ -62,22 +62,42 @@ struct FusedArgs {
     // d_model 512 kernel only: per-lane scratch in device memory (the context's workspace rows, row = lane): the
     // mixer's z | conv output [lanes][2 d_inner]
     float* scr;
-    // group_step.hip: the exchange packets, the first sequence number of this launch, and where an expired wait is
-    // reported; the gate its workgroups meet at (gate[0]: the launches' decisions, 2 seq0 + 1 for "not all here";
-    // gate[1]: arrivals, `arrived` before this launch, or GATE_NEVER; gate[2]: launches that were shut out) and how long
-    // they wait there, in 10 ns
+    // group_step.hip: the exchange packets, the first sequence number of this launch, its control words (below; arrivals
+    // before this launch: `arrived`, or GATE_NEVER), how long its workgroups wait at the gate and for a packet, in 10 ns,
+    // and where an expired wait is reported to the host
     uint64_t* xch;
     uint32_t seq0;
-    int32_t* bad;
-    uint64_t* gate;
+    uint32_t seq_first;        // what the first exchange's packets carry: seq0 (another number: that wait expires)
+    uint64_t* ctl;
     uint64_t arrived;
     uint32_t gate_ticks;
+    uint32_t wait_ticks;
+    uint64_t* host_expired;
+    // an expired wait of a launch from this one on (a decision word) has spoilt the state that this launch continues
+    uint64_t valid_from;
     // fused kernels: run only if the group launch with this decision word (2 seq0 + 1) did not start (0: always run)
     uint64_t only_if;
 };
+// Control words of a context's group launches: the last decision at the gate (2 seq0: open, 2 seq0 + 1: not all here),
+// arrivals there, launches that were shut out, and the (shut) decision word of the last launch in which a wait expired.
+enum { CTL_GATE, CTL_ARRIVED, CTL_SHUT_OUT, CTL_EXPIRED, CTL_WORDS };
 constexpr uint64_t GATE_NEVER = 1ull << 63;  // `arrived` of a launch whose gate no count of arrivals opens
-// Whether a fused launch is left out: it follows a group launch that did run.
-__device__ __forceinline__ bool left_out(const FusedArgs& a) { return a.only_if != 0 && a.gate[0] != a.only_if; }
+
+// Logits of a step that cannot be formed: NaN for every lane (all threads of the grid).
+__device__ __forceinline__ void void_logits(float* logits, int64_t n) {
+    const float nan = __builtin_nanf("");
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) logits[i] = nan;
+}
+// Whether a fused launch is left out: it follows a group launch that did run, or a wait between workgroups expired in it
+// or in an earlier launch since the state was reset (ctl is null where no group launch can have run).
+__device__ __forceinline__ bool left_out(const FusedArgs& a) {
+    if (a.ctl == nullptr) return false;
+    if (a.ctl[CTL_EXPIRED] >= a.valid_from) {
+        if (a.logits) void_logits(a.logits, (int64_t)a.B * a.V);
+        return true;
+    }
+    return a.only_if != 0 && a.ctl[CTL_GATE] != a.only_if;
+}
 
 // Launches over several tiles at once (a tile: all lanes of a group at Tc consecutive positions, at one layer).
 constexpr int PIPE_MAX = 16;  // tiles per launch at most
@@ -133,7 +153,6 @@ hipError_t launch_fused_step512(const FusedArgs& a, int nt, hipStream_t s);
 constexpr int GROUP_MAX = 128;  // groups of 16 lanes at most
 int64_t group_step_bytes(int d_model, int64_t max_lanes);     // exchange packets, in bytes
 int group_step_width(int d_model, int lanes, int cus);         // workgroups per group on a GPU of that many CUs; 1: none
-constexpr int GROUP_GATE_WORDS = 3;
 // takes 1 + nsteps (L + 1) sequence numbers from a.seq0 on; adds group_step_blocks to the gate's arrivals.  Does nothing
 // (and says so at the gate) if its workgroups do not all get onto the GPU in time: a fused launch with only_if follows.
 int64_t group_step_blocks(int lanes, int g);

@@ -662,6 +662,69 @@ def test_shut_gate_leaves_the_work_to_the_fused_kernel(gpu, monkeypatch, d_model
         assert np.array_equal(got["0"][1], got[group][1])
 
 
+@pytest.mark.parametrize("d_model,precision,n", [(256, "f32", 1), (256, "bf16x3", 600), (512, "bf16w", 40)])
+def test_expired_wait_is_reported(gpu, monkeypatch, d_model, precision, n):
+    """A wait between workgroups that expires (here the first of every launch; all workgroups leave normally) never gives
+    finite logits: the step's are NaN, calls made once the host knows are refused, a forward enqueued before that gives
+    NaN, and a decode fails.  A reset gives a working context again."""
+    import codec
+    import model as M
+    from boa_amd import _native as N
+    from boa_amd import weights as W
+    from model import _Engine
+
+    cfg = W.Cfg(d_model=d_model, n_layers=2)
+    blob = W.seeded_blob(cfg, 5)
+    tok = torch.from_numpy(np.random.default_rng(6).integers(0, 256, (n, 20)).astype(np.int32)).cuda()
+    first = tok[:, 0].contiguous()
+    ref, out = (torch.zeros((n, 256), device="cuda") for _ in range(2))
+    monkeypatch.setenv("BOA_GROUP_STEP", "0")
+    eng = _Engine(blob, cfg, n, 20, precision)
+    eng.reset(n)
+    eng.step(first, ref)
+    monkeypatch.setenv("BOA_GROUP_STEP", "expire")
+    eng = _Engine(blob, cfg, n, 20, precision)
+    eng.reset(n)
+    eng.step(first, out)
+    long = torch.zeros((n, 20, 256), device="cuda")
+    try:
+        eng.forward(tok, long)  # most likely before the step has run
+    except N.BoaError:
+        long.fill_(float("nan"))
+    torch.cuda.synchronize()
+    assert out.isnan().all() and long.isnan().all()
+    with pytest.raises(N.BoaError):
+        eng.step(first, out)
+    with pytest.raises(N.BoaError):
+        eng.forward(tok, long)
+    eng.reset(n)
+    for _ in range(2):
+        eng.reset(n)
+        eng.step(first, out)
+        assert torch.equal(out, ref)
+    # steps enqueued behind the expired one, and a reset before the host knows
+    eng = _Engine(blob, cfg, n, 20, precision)
+    eng.reset(n)
+    eng.step(first, out)
+    later = torch.zeros_like(out)
+    try:
+        eng.step(first, later)
+    except N.BoaError:
+        later.fill_(float("nan"))
+    eng.reset(n)
+    torch.cuda.synchronize()
+    assert out.isnan().all() and later.isnan().all()
+
+    m = M.BoaConstrictor(d_model, 2, 256).load_blob(blob)
+    m.precision = precision
+    chunks = [np.random.default_rng(i).integers(0, 256, 9).astype(np.uint8) for i in range(n)]
+    payload, nw, fb, Ls = codec.compress_payload(m, chunks)
+    with pytest.raises(N.BoaError):
+        codec.decompress_payload(m, payload, nw, Ls, fb)
+    out = codec.decompress_payload(m, payload, nw, Ls, fb)
+    assert all((out[i, :9] == c).all() for i, c in enumerate(chunks))
+
+
 def test_step_under_capture(gpu):
     """A step recorded into a graph (which cannot hold the group kernel's sequence numbers) replays as the eager step
     from the same state."""
