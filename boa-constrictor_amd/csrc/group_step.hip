@@ -25,8 +25,9 @@
 //
 // A packet is rewritten only by the same exchange of the next layer (or step), and its writer gets there only after
 // every member has sent its packets of a later exchange of this layer, which it does after reading this one (a barrier
-// between): no packet is overwritten before all have read it.  Sequence numbers grow over the context's life, so what
-// earlier launches left never matches.
+// between): no packet is overwritten before all have read it.  Sequence numbers grow from launch to launch, so what
+// earlier launches left never matches; a packet holds their low 32 bits, and before those wrap the host zeroes all packets
+// (launch_fused; 0 is never expected).
 //
 // All workgroups have to be resident at once (at most one per CU).  They meet at a gate first, before anything is read or
 // written: the last to arrive opens it; the first to find its time up (another kernel holds the CUs) closes it for this
@@ -415,7 +416,7 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
         uint32_t at[G / 2], v[G], differ = 0;
 #pragma unroll
         for (int i = 0; i < G / 2; ++i) at[i] = XC::W + 2 * i;
-        receive(far, at, a0.seq0, v);
+        receive(far, at, (uint32_t)a0.seq0, v);
 #pragma unroll
         for (int i = 0; i < G; ++i) differ |= v[i] ^ xcc;
         near = __builtin_amdgcn_readfirstlane(differ) == 0u;
@@ -441,7 +442,7 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
         const int t = a.t + step;
         if (a.decode && t >= sMaxLen) break;  // every lane of the group is complete (the same for every member)
         const Link xc = {buf_rsrc(reinterpret_cast<Packet*>(a.xch) + (int64_t)group * XC::SIZE, XC::SIZE * 8), near, limit};
-        const uint32_t seq0 = a.seq0 + 1u + (uint32_t)step * (uint32_t)(a.L + 1);
+        const uint32_t seq0 = (uint32_t)a.seq0 + 1u + (uint32_t)step * (uint32_t)(a.L + 1);
         const int s1 = p0m3 == 2 ? 0 : p0m3 + 1, s2 = p0m3 == 0 ? 2 : p0m3 - 1;
         const int V = a.V;
         auto tok_of = [&](int r) {

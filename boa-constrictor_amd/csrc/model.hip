@@ -2726,7 +2726,7 @@ struct boa_ctx {
     uint64_t* xch = nullptr;
     uint64_t* xctl = nullptr;          // control words (CTL_*)
     uint64_t xarrived = 0;             // arrivals at the gate so far
-    uint32_t xseq = 1;                 // the next sequence number of an exchange packet
+    uint64_t xseq = 1;                 // the next launch's first sequence number
     // an expired wait: the launch it was in (pinned host memory, 0: none), the first launch since the state was reset,
     // whether the state has gone through a group launch since then, and whether group launches are given up
     uint64_t* xexpired = nullptr;
@@ -2734,7 +2734,7 @@ struct boa_ctx {
     bool grouped = false;
     bool group_off = false;
     // tests, by BOA_GROUP_STEP: the gate never opens (shut); a launch's first packets carry a number that nobody waits
-    // for, and the wait is short (expire)
+    // for, and the wait is short (expire); the first launch's sequence numbers would wrap (wrap)
     bool group_shut = false, group_expire = false;
     int cus = 0;
     hipStream_t stream2 = nullptr;
@@ -3220,6 +3220,7 @@ extern "C" int boa_ctx_create(const boa_model_cfg* cfg, const void* h_weights, i
     if (const char* v = getenv("BOA_GROUP_STEP")) {
         x->group_shut = strcmp(v, "shut") == 0;
         x->group_expire = strcmp(v, "expire") == 0;
+        if (strcmp(v, "wrap") == 0) x->xseq = (1ull << 32) - 3;
     }
     if (const char* v = getenv("BOA_DECODE_HALVES")) x->decode_halves = atoi(v) == 1 ? 1 : 2;
     if (const char* v = getenv("BOA_FFN_OUTP")) x->ffn_outp = atoi(v) != 0;
@@ -3744,14 +3745,21 @@ static hipError_t launch_fused(boa_ctx* x, FusedArgs& a, hipStream_t s) {
         a.ctl = x->xctl; a.valid_from = x->valid_from;
         const int g = group_step_width(x->d, a.B, x->cus);
         if (g > 1) {
+            const uint32_t seqs = group_step_seqs(a.nsteps, x->L);
+            if ((x->xseq >> 32) != ((x->xseq + seqs) >> 32)) {
+                // the low 32 bits would wrap (after some 10^8 steps): no packet of theirs is left to match the new ones
+                x->xseq = ((x->xseq >> 32) + 1) << 32 | 1;
+                const hipError_t e = hipMemsetAsync(x->xch, 0, (size_t)group_step_bytes(x->d, x->max_lanes), s);
+                if (e != hipSuccess) return e;
+            }
             a.xch = x->xch; a.seq0 = x->xseq; a.arrived = x->group_shut ? GATE_NEVER : x->xarrived;
             a.gate_ticks = 50000u + 5000u * (uint32_t)a.nsteps;  // 0.5 ms and 50 us per step
-            a.seq_first = x->group_expire ? 0u : a.seq0;     // (0: the number of a packet never written)
+            a.seq_first = x->group_expire ? 0u : (uint32_t)a.seq0;     // (0: the number of a packet never written)
             a.wait_ticks = x->group_expire ? 1000u : 300000000u;  // 10 us, 3 s
             a.host_expired = x->xexpired;
             const hipError_t e = launch_group_step(a, x->d, nt, g, s);
             if (e != hipSuccess) return e;
-            x->xseq += 1u + (uint32_t)a.nsteps * (uint32_t)(x->L + 1);
+            x->xseq += seqs;
             x->xarrived += (uint64_t)group_step_blocks(a.B, g);
             x->grouped = true;
             a.only_if = 2ull * a.seq0 + 1ull;  // then the fused launch, which leaves if the group launch ran

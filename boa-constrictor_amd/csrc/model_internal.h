@@ -62,11 +62,12 @@ struct FusedArgs {
     // d_model 512 kernel only: per-lane scratch in device memory (the context's workspace rows, row = lane): the
     // mixer's z | conv output [lanes][2 d_inner]
     float* scr;
-    // group_step.hip: the exchange packets, the first sequence number of this launch, its control words (below; arrivals
-    // before this launch: `arrived`, or GATE_NEVER), how long its workgroups wait at the gate and for a packet, in 10 ns,
-    // and where an expired wait is reported to the host
+    // group_step.hip: the exchange packets, the first sequence number of this launch (a packet carries its low 32 bits,
+    // which a launch does not let wrap), its control words (below; arrivals before this launch: `arrived`, or GATE_NEVER),
+    // how long its workgroups wait at the gate and for a packet, in 10 ns, and where an expired wait is reported to the
+    // host
     uint64_t* xch;
-    uint32_t seq0;
+    uint64_t seq0;
     uint32_t seq_first;        // what the first exchange's packets carry: seq0 (another number: that wait expires)
     uint64_t* ctl;
     uint64_t arrived;
@@ -153,9 +154,10 @@ hipError_t launch_fused_step512(const FusedArgs& a, int nt, hipStream_t s);
 constexpr int GROUP_MAX = 128;  // groups of 16 lanes at most
 int64_t group_step_bytes(int d_model, int64_t max_lanes);     // exchange packets, in bytes
 int group_step_width(int d_model, int lanes, int cus);         // workgroups per group on a GPU of that many CUs; 1: none
-// takes 1 + nsteps (L + 1) sequence numbers from a.seq0 on; adds group_step_blocks to the gate's arrivals.  Does nothing
+// takes group_step_seqs sequence numbers from a.seq0 on; adds group_step_blocks to the gate's arrivals.  Does nothing
 // (and says so at the gate) if its workgroups do not all get onto the GPU in time: a fused launch with only_if follows.
 int64_t group_step_blocks(int lanes, int g);
+inline uint32_t group_step_seqs(int nsteps, int L) { return 1u + (uint32_t)nsteps * (uint32_t)(L + 1); }
 hipError_t launch_group_step(const FusedArgs& a, int d_model, int nt, int g, hipStream_t s);
 
 }  // namespace boa

@@ -725,6 +725,32 @@ def test_expired_wait_is_reported(gpu, monkeypatch, d_model, precision, n):
     assert all((out[i, :9] == c).all() for i, c in enumerate(chunks))
 
 
+@pytest.mark.parametrize("d_model,precision", [(256, "f32"), (512, "bf16w")])
+def test_sequence_numbers_wrap(gpu, monkeypatch, d_model, precision):
+    """Steps and decodes whose packets' 32-bit sequence numbers run out (contexts that start just before) give the fused
+    kernels' values: 0 marks a packet that was never written and is never expected."""
+    import codec
+    import model as M
+    from boa_amd import weights as W
+
+    monkeypatch.setenv("BOA_FUSED_STEPS_PER_LAUNCH", "3")
+    blob = W.seeded_blob(W.Cfg(d_model=d_model, n_layers=2), 7)
+    n, got = 20, {}
+    for group in ("0", "wrap"):
+        monkeypatch.setenv("BOA_GROUP_STEP", group)
+        rng = np.random.default_rng(n)
+        m = M.BoaConstrictor(d_model, 2, 256).load_blob(blob)
+        m.precision = precision
+        inf = m.init_stream(max_len=8, batch_size=n)
+        logits = [m.step(torch.from_numpy(rng.integers(0, 256, n).astype(np.int32)).cuda(), inf).cpu() for _ in range(4)]
+        nw = rng.integers(0, 9, n)
+        payload = rng.integers(0, 1 << 32, int(nw.sum()), dtype=np.uint64).astype(np.uint32)
+        out = codec.decompress_payload(m, payload, nw, [14] * n, rng.integers(0, 256, n).tolist())
+        got[group] = (logits, out)
+    assert all(torch.equal(a, b) for a, b in zip(got["0"][0], got["wrap"][0]))
+    assert np.array_equal(got["0"][1], got["wrap"][1])
+
+
 def test_step_under_capture(gpu):
     """A step recorded into a graph (which cannot hold the group kernel's sequence numbers) replays as the eager step
     from the same state."""
