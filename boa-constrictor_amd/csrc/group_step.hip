@@ -56,6 +56,10 @@ namespace boa {
 namespace {
 
 constexpr int ROWS = 16, NTHR = 512, NWAVE = 8, NS = 16, VV = 256;
+// Wait at the gate, in 10 ns, of a launch behind one that was shut out.  With room, the last of a launch's workgroups is
+// there about 3 us after the first (up to 256 workgroups, 1200 launches: 5 us passed in 3%, 10 us in none).  With the whole
+// wait (0.5 ms and more) every step of a context beside other work paid it.
+constexpr uint32_t SHUT_TICKS = 2000;
 typedef uint64_t Packet;
 
 typedef __attribute__((address_space(4))) const FusedArgs KArgs;
@@ -378,10 +382,12 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
         const uint64_t n = __hip_atomic_fetch_add(a0.ctl + CTL_ARRIVED, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         uint64_t st = state();
         if (n - a0.arrived == total - 1) decide(st, open);
+        // if the launch before found no room, other work most likely still has the CUs: a short wait (SHUT_TICKS)
+        const uint32_t ticks = (st & 1ull) != 0 && st != shut && a0.gate_ticks > SHUT_TICKS ? SHUT_TICKS : a0.gate_ticks;
         const uint64_t t0 = wall_clock64();
         while (!spoilt && st != open && st != shut) {
             st = state();
-            if (wall_clock64() - t0 > a0.gate_ticks && decide(st, shut))
+            if (wall_clock64() - t0 > ticks && decide(st, shut))
                 __hip_atomic_fetch_add(a0.ctl + CTL_SHUT_OUT, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         sGo = !spoilt && st == open ? 1 : 0;

@@ -751,6 +751,84 @@ def test_sequence_numbers_wrap(gpu, monkeypatch, d_model, precision):
     assert np.array_equal(got["0"][1], got["wrap"][1])
 
 
+def test_steps_beside_other_work(gpu):
+    """Two contexts stepping at the same time on their own streams, and one beside matrix products that hold all CUs:
+    whichever launches find room, every step gives the logits of a context on its own, bit for bit, and once the GPU is
+    free again the group kernel runs again."""
+    from boa_amd import weights as W
+    from model import _Engine
+
+    cfg = W.Cfg(n_layers=3)
+    blob = W.seeded_blob(cfg, 3)
+    B, T = 300, 12
+    tok = torch.from_numpy(np.random.default_rng(1).integers(0, 256, (T, B)).astype(np.int32)).cuda()
+
+    def steps(eng, out):
+        for t in range(T):
+            eng.step(tok[t], out[t])
+
+    ref = torch.zeros((T, B, 256), device="cuda")
+    eng = _Engine(blob, cfg, B, 1, "f32")
+    eng.reset(B)
+    steps(eng, ref)
+    a = torch.randn((8192, 8192), device="cuda", dtype=torch.bfloat16)
+    c = torch.empty_like(a)
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    outs = [torch.zeros_like(ref) for _ in range(2)]
+    torch.cuda.synchronize()
+    engs = []
+    for s in streams[:2]:
+        with torch.cuda.stream(s):
+            engs.append(_Engine(blob, cfg, B, 1, "f32"))
+    for load in (False, True):
+        if load:
+            with torch.cuda.stream(streams[2]):
+                for _ in range(40):
+                    torch.mm(a, a, out=c)
+        for o in outs:
+            o.zero_()
+        torch.cuda.synchronize() if not load else torch.cuda.current_stream().synchronize()
+        for e in engs:
+            e.reset(B)
+        for t in range(T):
+            for e, o in zip(engs, outs):
+                e.step(tok[t], o[t])
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, ref) for o in outs), load
+    before = [_shut_out(gpu, e) for e in engs]
+    for e, o in zip(engs, outs):
+        e.reset(B)
+        for t in range(T):
+            e.step(tok[t], o[t])
+        torch.cuda.synchronize()
+        assert torch.equal(o, ref)
+    assert [_shut_out(gpu, e) for e in engs] == before
+
+
+def test_shut_out_steps_wait_once(gpu, monkeypatch):
+    """A context whose group launches keep finding no room waits its 0.5 ms at the gate for the first of them only."""
+    import time
+
+    from boa_amd import weights as W
+    from model import _Engine
+
+    cfg = W.Cfg(n_layers=2)
+    blob = W.seeded_blob(cfg, 3)
+    tok, out, took = torch.zeros(1, dtype=torch.int32, device="cuda"), torch.zeros((1, 256), device="cuda"), {}
+    for group in ("0", "shut"):
+        monkeypatch.setenv("BOA_GROUP_STEP", group)
+        eng = _Engine(blob, cfg, 1, 1, "f32")
+        eng.reset(1)
+        for n in (20, 200):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            for _ in range(n):
+                eng.step(tok, out)
+            torch.cuda.synchronize()
+            took[group] = (time.perf_counter() - t) / n
+    assert took["shut"] < took["0"] + 250e-6, took
+
+
 def test_step_under_capture(gpu):
     """A step recorded into a graph (which cannot hold the group kernel's sequence numbers) replays as the eager step
     from the same state."""
