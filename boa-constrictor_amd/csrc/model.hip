@@ -2736,7 +2736,7 @@ struct boa_ctx {
     // tests, by BOA_GROUP_STEP: the gate never opens (shut); a launch's first packets carry a number that nobody waits
     // for, and the wait is short (expire); the first launch's sequence numbers would wrap (wrap)
     bool group_shut = false, group_expire = false;
-    int cus = 0;
+    int cus = 0;                       // of the GPU: what decode steps, compress and forward size their launches by
     hipStream_t stream2 = nullptr;
     hipStream_t stream3 = nullptr;     // the third compress group's
     std::vector<hipEvent_t> half_ev;   // [2][L]: state group of layer l done, per half; [2L], [2L + 1]: stream joins
@@ -3175,17 +3175,17 @@ extern "C" int boa_ctx_create(const boa_model_cfg* cfg, const void* h_weights, i
         }
     }
     if (e == hipSuccess && x->fused) e = dmalloc(x, &x->d_layers, (int64_t)L);
+    int dev = 0;
+    if (e == hipSuccess) e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&x->cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e == hipSuccess && want_group(c, R, x->prec)) {
         const int64_t n = group_step_bytes(c.d_model, max_lanes) / 8;
-        int dev = 0;
         e = dmalloc(x, &x->xch, n);
         if (e == hipSuccess) e = dmalloc(x, &x->xctl, CTL_WORDS);
         if (e == hipSuccess) e = hipMemsetAsync(x->xctl, 0, 8 * CTL_WORDS, x->stream);
         if (e == hipSuccess) e = hipMemsetAsync(x->xch, 0, (size_t)n * 8, x->stream);  // sequence number 0: none
         if (e == hipSuccess) e = hipHostMalloc((void**)&x->xexpired, sizeof(uint64_t), hipHostMallocDefault);
         if (e == hipSuccess) *x->xexpired = 0;
-        if (e == hipSuccess) e = hipGetDevice(&dev);
-        if (e == hipSuccess) e = hipDeviceGetAttribute(&x->cus, hipDeviceAttributeMultiprocessorCount, dev);
     }
     if (e != hipSuccess) {
         boa_ctx_destroy(x);

@@ -563,6 +563,34 @@ def test_feed_forward_in_shares(gpu, monkeypatch, precision, n, length):
     assert torch.equal(got[0][2], got[1][2])
 
 
+@pytest.mark.parametrize("switch", ["BOA_GROUP_STEP", "BOA_FUSED_STEP"])
+def test_decode_switches_leave_compress_alone(gpu, monkeypatch, switch):
+    """The switches of the decode kernels change neither the words of a compress of few lanes nor the kernels it takes
+    (shared feed-forward, heads beside the next step): the same time, where without those it takes 1.3 times as long."""
+    import time
+
+    import codec
+    import model as M
+    from boa_amd import weights as W
+
+    blob = W.seeded_blob(W.Cfg(n_layers=8), 3)
+    chunks = [np.random.default_rng(1).integers(0, 256, 1000).astype(np.uint8)]
+    best, words = {}, {}
+    models = {}
+    for v in ("1", "0"):
+        monkeypatch.setenv(switch, v)
+        models[v] = M.BoaConstrictor(256, 8, 256).load_blob(blob)
+        words[v] = codec.compress_payload(models[v], chunks)[0]
+    for _ in range(8):
+        for v, m in models.items():
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            codec.compress_payload(m, chunks)
+            best[v] = min(best.get(v, 1e9), time.perf_counter() - t)
+    assert np.array_equal(words["0"], words["1"])
+    assert best["0"] < 1.12 * best["1"], best
+
+
 @pytest.mark.parametrize("d_model,precision", [(256, "f32"), (256, "bf16x3"), (512, "bf16w")])
 @pytest.mark.parametrize("split", [1, 2, 3, 64, 65, 130])
 def test_forward_in_pieces_and_steps(gpu, d_model, precision, split):
