@@ -2727,11 +2727,11 @@ struct boa_ctx {
     uint64_t* xctl = nullptr;          // control words (CTL_*)
     uint64_t xarrived = 0;             // arrivals at the gate so far
     uint64_t xseq = 1;                 // the next launch's first sequence number
-    // an expired wait: the launch it was in (pinned host memory, 0: none), the first launch since the state was reset,
-    // whether the state has gone through a group launch since then, and whether group launches are given up
+    // an expired wait: the launch it was in (pinned host memory, 0: none), the first launch since the state was reset, the
+    // lanes whose state has gone through group launches since then, and whether group launches are given up
     uint64_t* xexpired = nullptr;
     uint64_t valid_from = 2;
-    bool grouped = false;
+    int grouped = 0;
     bool group_off = false;
     // tests, by BOA_GROUP_STEP: the gate never opens (shut); a launch's first packets carry a number that nobody waits
     // for, and the wait is short (expire); the first launch's sequence numbers would wrap (wrap)
@@ -3273,8 +3273,10 @@ extern "C" int boa_state_reset(boa_ctx* x, int32_t lanes) {
     if (!x || lanes < 0 || lanes > x->max_lanes) return boa_fail(BOA_ERR_ARG, "boa_state_reset: bad lanes");
     x->pos = 0;
     (void)wait_expired(x);
-    x->valid_from = 2ull * x->xseq;
-    x->grouped = false;
+    if (lanes >= x->grouped) {
+        x->valid_from = 2ull * x->xseq;
+        x->grouped = 0;
+    }
     if (lanes == 0) return BOA_OK;
     // one launch for all layers (two memsets per layer took 2 us each plus their gaps: 60 us at 8 layers)
     const int64_t ns = (int64_t)x->di * x->NS;
@@ -3761,7 +3763,7 @@ static hipError_t launch_fused(boa_ctx* x, FusedArgs& a, hipStream_t s) {
             if (e != hipSuccess) return e;
             x->xseq += seqs;
             x->xarrived += (uint64_t)group_step_blocks(a.B, g);
-            x->grouped = true;
+            x->grouped = std::max(x->grouped, (int)a.B);
             a.only_if = 2ull * a.seq0 + 1ull;  // then the fused launch, which leaves if the group launch ran
         }
     }

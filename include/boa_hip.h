@@ -90,7 +90,7 @@ int boa_state_reset(boa_ctx* ctx, int32_t lanes);
  * BoaPredictorGPU::step_batch (boa_gpu.hpp:560-578).
  * Steps of few lanes run on workgroups that wait for each other; should such a wait expire (3 s: the process
  * was taken off the GPU), that step's logits and those of everything that continues its state are NaN, and
- * calls made after the host has heard of it return BOA_ERR_HIP, until boa_state_reset.                     */
+ * calls made after the host has heard of it return BOA_ERR_HIP, until boa_state_reset of all those lanes.                   */
 int boa_model_step(boa_ctx* ctx, const int32_t* d_tokens, int32_t lanes, float* d_logits);
 
 /* Teacher-forced forward from the current state: d_tokens int32 [lanes][len] (row stride tok_stride)
