@@ -2744,6 +2744,7 @@ struct boa_ctx {
     uint16_t* wfrag = nullptr;         // fragment-packed GEMM weights (fused)
     FusedLayer* d_layers = nullptr;    // per-layer pointer table (fused)
     int64_t device_bytes = 0;
+    int64_t bytes_limit = INT64_MAX;   // BOA_CTX_MAX_BYTES
     bool prof_on = false;
     ProfClassState prof[PC_COUNT];
 };
@@ -2893,7 +2894,8 @@ static bool tile_kernels(const boa_model_cfg& c, int R, int precision) {
 // Positions per tile of run_pipe, and the workspace rows of a context: max_lanes tiles as every path needs, and for
 // contexts of few lanes room for run_pipe's other tiles in flight: one per layer, but at most PIPE_TILES (lane, tile)
 // pairs in all, which is enough 64-row workgroups for every CU with room to even out the last round.  Sized for the
-// lanes rounded up to a power of two (16 at least).
+// lanes rounded up to a power of two (16 at least), and for no fewer rows than any context of fewer lanes: up to PIPE_LANES,
+// and beyond, the rows never shrink as the lanes grow; from one to the other (no tiles in flight) they do.
 constexpr int PIPE_TILES = 2048, PIPE_MIN_TILE = 16, PIPE_LANES = 511;
 static int pipe_tile(int64_t tile_len) { return (int)std::min<int64_t>(tile_len, 64); }
 static int64_t workspace_rows(const boa_model_cfg& c, int R, int precision, int64_t max_lanes, int64_t tile_len) {
@@ -2901,18 +2903,20 @@ static int64_t workspace_rows(const boa_model_cfg& c, int R, int precision, int6
     const char* env = getenv("BOA_PIPE");
     if (!tile_kernels(c, R, precision) || pipe_tile(tile_len) < PIPE_MIN_TILE || max_lanes > PIPE_LANES || (env && env[0] == '0'))
         return rows;
-    int64_t up = 16;
-    while (up < max_lanes) up *= 2;
-    int64_t p = std::max<int64_t>(1, std::min<int64_t>(PIPE_TILES / up, std::min(c.n_layers, PIPE_MAX)));
-    if (up == 16) ++p;  // for the tile whose head runs beside the next step (run_pipe)
-    return rows + (p - 1) * up * pipe_tile(tile_len);
+    int64_t ws = 0;
+    for (int64_t up = 16; up < 2 * std::max<int64_t>(max_lanes, 9); up *= 2) {
+        int64_t p = std::max<int64_t>(1, std::min<int64_t>(PIPE_TILES / up, std::min(c.n_layers, PIPE_MAX)));
+        if (up == 16) ++p;  // for the tile whose head runs beside the next step (run_pipe)
+        ws = std::max(ws, std::min(max_lanes, up) * tile_len + (p - 1) * up * pipe_tile(tile_len));
+    }
+    return ws;
 }
 
 // Device bytes boa_ctx_create allocates for this shape: the same list of buffers, in the same order, each
 // rounded as dmalloc rounds it.  boa_ctx_create checks its own total against this after allocating.
-static int64_t ctx_plan_bytes(const boa_model_cfg& c, int R, int precision, int64_t max_lanes, int64_t tile_len) {
+static int64_t ctx_plan_bytes(const boa_model_cfg& c, int R, int precision, int64_t max_lanes, int64_t tile_len, int64_t ws) {
     const int64_t d = c.d_model, di = (int64_t)c.expand * c.d_model, NS = c.d_state, V = c.vocab, L = c.n_layers;
-    const int64_t rows = max_lanes * tile_len, ws = workspace_rows(c, R, precision, max_lanes, tile_len);
+    const int64_t rows = max_lanes * tile_len;
     auto f4 = [](int64_t n) { return 4 * std::max<int64_t>(n, 1); };
     int64_t b = f4(weights_floats(c, R)) + f4(L * di * NS) + f4(L * max_lanes * 3 * di) + f4(L * max_lanes * di * NS) +
                 f4(ws * d) + f4(ws * std::max(2 * di, 4 * d)) + f4(ws * di) + f4(ws * (R + 2 * NS)) +
@@ -2940,7 +2944,7 @@ extern "C" int boa_ctx_plan_bytes(const boa_model_cfg* cfg, int precision, int32
     if (rc != BOA_OK) return rc;
     if (max_lanes < 1 || tile_len < 1 || tile_len > 256)
         return boa_fail(BOA_ERR_ARG, "need max_lanes >= 1 and 1 <= tile_len <= 256 (got %d, %d)", max_lanes, tile_len);
-    *out_bytes = ctx_plan_bytes(c, R, precision, max_lanes, tile_len);
+    *out_bytes = ctx_plan_bytes(c, R, precision, max_lanes, tile_len, workspace_rows(c, R, precision, max_lanes, tile_len));
     return BOA_OK;
 }
 
@@ -2967,6 +2971,7 @@ template <typename T>
 static hipError_t dmalloc(boa_ctx* c, T** p, int64_t count) {
     const int64_t bytes = std::max<int64_t>(count, 1) * (int64_t)sizeof(T);
     c->device_bytes += bytes;
+    if (c->device_bytes > c->bytes_limit) return hipErrorOutOfMemory;
     return hipMalloc((void**)p, (size_t)bytes);
 }
 
@@ -3013,24 +3018,10 @@ static void pack_fragments(const uint16_t* hi, const uint16_t* lo, int N, int K,
         }
 }
 
-extern "C" int boa_ctx_create(const boa_model_cfg* cfg, const void* h_weights, int64_t nbytes, int precision,
-                              int32_t max_lanes, int32_t tile_len, void* stream, boa_ctx** out) {
-    if (!out) return boa_fail(BOA_ERR_ARG, "boa_ctx_create: null output");
-    *out = nullptr;
-    boa_model_cfg c;
-    int R;
-    int rc = resolve_cfg(cfg, c, R);
-    if (rc != BOA_OK) return rc;
-    if (precision != BOA_PREC_F32 && precision != BOA_PREC_BF16X3 && precision != BOA_PREC_BF16W)
-        return boa_fail(BOA_ERR_ARG, "boa_ctx_create: unknown precision mode %d", precision);
-    const int64_t nf = weights_floats(c, R);
-    if (!h_weights || nbytes != nf * 4)
-        return boa_fail(BOA_ERR_ARG, "weight blob must be %lld bytes (got %lld)", (long long)(nf * 4), (long long)nbytes);
-    if (max_lanes < 1 || tile_len < 1 || tile_len > 256)
-        return boa_fail(BOA_ERR_ARG, "need max_lanes >= 1 and 1 <= tile_len <= 256 (got %d, %d)", max_lanes, tile_len);
-    const int64_t max_rows = (int64_t)max_lanes * tile_len;
-    if (max_rows > (int64_t)1 << 31) return boa_fail(BOA_ERR_ARG, "max_lanes * tile_len too large");
-
+// A context with a workspace of ws rows; e: the HIP error, if that is why it failed.
+static int ctx_create(const boa_model_cfg& c, int R, const void* h_weights, int64_t nbytes, int precision, int32_t max_lanes,
+                      int32_t tile_len, int64_t ws, void* stream, hipError_t& e, boa_ctx** out) {
+    const int64_t nf = weights_floats(c, R), max_rows = (int64_t)max_lanes * tile_len;
     boa_ctx* x = new boa_ctx();
     x->cfg = c;
     x->d = c.d_model; x->di = c.expand * c.d_model; x->NS = c.d_state; x->R = R; x->V = c.vocab;
@@ -3039,11 +3030,12 @@ extern "C" int boa_ctx_create(const boa_model_cfg* cfg, const void* h_weights, i
     x->prec = precision;
     x->max_lanes = max_lanes; x->tile_len = tile_len; x->max_rows = max_rows;
     const int d = x->d, di = x->di, NS = x->NS, V = x->V, L = x->L;
-    x->ws_rows = workspace_rows(c, R, precision, max_lanes, tile_len);
+    x->ws_rows = ws;
+    if (const char* v = getenv("BOA_CTX_MAX_BYTES")) x->bytes_limit = atoll(v);
     if (const char* v = getenv("BOA_PIPE")) x->pipe = v[0] != '0';
     x->pipe = x->pipe && tile_kernels(c, R, precision);
 
-    hipError_t e = hipSuccess;
+    e = hipSuccess;
 #define TRY_ALLOC(p, n) do { if (e == hipSuccess) e = dmalloc(x, &(p), (n)); } while (0)
     TRY_ALLOC(x->wblob, nf);
     TRY_ALLOC(x->aneg, (int64_t)L * di * NS);
@@ -3243,13 +3235,42 @@ extern "C" int boa_ctx_create(const boa_model_cfg* cfg, const void* h_weights, i
             return boa_fail_hip(e, "boa_ctx_create streams", __FILE__, __LINE__);
         }
     }
-    if (x->device_bytes != ctx_plan_bytes(c, R, precision, max_lanes, tile_len)) {
-        const long long got = (long long)x->device_bytes, plan = (long long)ctx_plan_bytes(c, R, precision, max_lanes, tile_len);
+    if (x->device_bytes != ctx_plan_bytes(c, R, precision, max_lanes, tile_len, ws)) {
+        const long long got = (long long)x->device_bytes, plan = (long long)ctx_plan_bytes(c, R, precision, max_lanes, tile_len, ws);
         boa_ctx_destroy(x);
         return boa_fail(BOA_ERR_STATE, "internal: context holds %lld bytes, plan says %lld", got, plan);
     }
     *out = x;
     return BOA_OK;
+}
+
+extern "C" int boa_ctx_create(const boa_model_cfg* cfg, const void* h_weights, int64_t nbytes, int precision,
+                              int32_t max_lanes, int32_t tile_len, void* stream, boa_ctx** out) {
+    if (!out) return boa_fail(BOA_ERR_ARG, "boa_ctx_create: null output");
+    *out = nullptr;
+    boa_model_cfg c;
+    int R;
+    int rc = resolve_cfg(cfg, c, R);
+    if (rc != BOA_OK) return rc;
+    if (precision != BOA_PREC_F32 && precision != BOA_PREC_BF16X3 && precision != BOA_PREC_BF16W)
+        return boa_fail(BOA_ERR_ARG, "boa_ctx_create: unknown precision mode %d", precision);
+    const int64_t nf = weights_floats(c, R);
+    if (!h_weights || nbytes != nf * 4)
+        return boa_fail(BOA_ERR_ARG, "weight blob must be %lld bytes (got %lld)", (long long)(nf * 4), (long long)nbytes);
+    if (max_lanes < 1 || tile_len < 1 || tile_len > 256)
+        return boa_fail(BOA_ERR_ARG, "need max_lanes >= 1 and 1 <= tile_len <= 256 (got %d, %d)", max_lanes, tile_len);
+    const int64_t max_rows = (int64_t)max_lanes * tile_len;
+    if (max_rows > (int64_t)1 << 31) return boa_fail(BOA_ERR_ARG, "max_lanes * tile_len too large");
+
+    const int64_t ws = workspace_rows(c, R, precision, max_lanes, tile_len);
+    hipError_t e = hipSuccess;
+    rc = ctx_create(c, R, h_weights, nbytes, precision, max_lanes, tile_len, ws, stream, e, out);
+    if (rc != BOA_OK && e == hipErrorOutOfMemory && ws > max_rows) {
+        // without room for tiles in flight the context still does everything, slower with few lanes
+        (void)hipGetLastError();
+        rc = ctx_create(c, R, h_weights, nbytes, precision, max_lanes, tile_len, max_rows, stream, e, out);
+    }
+    return rc;
 }
 
 // Whether a wait between workgroups expired since the state was reset, as far as the host has heard of it.  The fused

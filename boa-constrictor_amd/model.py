@@ -72,6 +72,26 @@ class MambaBlock(nn.Module):
         self.ff = nn.Sequential(nn.Linear(d_model, 4 * d_model), nn.GELU(), nn.Linear(4 * d_model, d_model))
 
 
+# Contexts of up to this many lanes hold extra workspace for tiles in flight (PIPE_LANES, model.hip): their memory grows
+# with the lanes on either side of it, but falls from here to the next.
+_PIPE_LANES = 511
+
+
+def _most_lanes(need, most: int, budget: float) -> int:
+    """The largest number of lanes in [1, most] whose need(lanes) is within the budget (at least 1)."""
+    for lo, hi in ((_PIPE_LANES + 1, most), (1, min(most, _PIPE_LANES))):
+        if lo > hi or (need(lo) > budget and lo > 1):
+            continue
+        while lo < hi:
+            mid = (lo + hi + 1) // 2
+            if need(mid) <= budget:
+                lo = mid
+            else:
+                hi = mid - 1
+        return lo
+    return 1
+
+
 class _Engine:
     """One libboa_hip model context: device copy of the weights + recurrent state + workspace."""
 
@@ -198,16 +218,7 @@ class BoaBytePredictor(nn.Module):
             _nat.check(lib.boa_ctx_plan_bytes(ctypes.byref(c), prec, lanes, tile, ctypes.byref(b)))
             return float(b.value) + lanes * (9.0 * chunk_len + 80.0)
 
-        lo, hi = 1, max(1, min(int(n_chunks), int(cap)))
-        if need(hi) <= budget:
-            return hi
-        while lo < hi:  # largest lanes with need(lanes) <= budget (at least 1)
-            mid = (lo + hi + 1) // 2
-            if need(mid) <= budget:
-                lo = mid
-            else:
-                hi = mid - 1
-        return lo
+        return _most_lanes(need, max(1, min(int(n_chunks), int(cap))), budget)
 
     # ---- reference API ----------------------------------------------------------------------------
     @torch.inference_mode()

@@ -75,7 +75,9 @@ int boa_ctx_destroy(boa_ctx* ctx);
 /* Bytes of device memory the context holds. */
 int64_t boa_ctx_device_bytes(const boa_ctx* ctx);
 /* Bytes of device memory boa_ctx_create would allocate for this shape (exact: creation checks its total
- * against it).  For sizing waves of chunks from free device memory.  Replaces
+ * against it).  For sizing waves of chunks from free device memory.  They grow with max_lanes up to 511 lanes
+ * and from 512 on; up to 511 they include workspace that few lanes run faster with, and a context that only
+ * fits without it is created without it.  Replaces
  * BoaPredictorGPU::estimate_memory_static (boa_gpu.hpp:625-662) as used by auto_size_params
  * (boa.cpp:103-150).                                                                                  */
 int boa_ctx_plan_bytes(const boa_model_cfg* cfg, int precision, int32_t max_lanes, int32_t tile_len,

@@ -4,6 +4,8 @@ import os
 import re
 import subprocess
 
+import pytest
+
 from conftest import REPO
 
 
@@ -72,3 +74,28 @@ def test_ctx_plan_bytes_host_only():
     per_lane = 8 * 4 * (3 * 512 + 512 * 16) + 64 * per_row + 4 + 32 + 32
     assert vals[1] - vals[0] == per_lane
     assert lib.boa_ctx_plan_bytes(ctypes.byref(c), 1, 0, 64, ctypes.byref(out)) == _native.BOA_ERR_ARG
+
+
+@pytest.mark.parametrize("d,L,prec,tile", [(256, 8, 0, 64), (256, 1, 1, 64), (256, 16, 2, 33), (512, 16, 2, 64),
+                                           (512, 40, 1, 200), (512, 4, 0, 64), (256, 3, 0, 15)])
+def test_ctx_plan_grows_and_wave_sizing_finds_the_most_lanes(d, L, prec, tile):
+    """Planned bytes never shrink as the lanes grow, but for the step from 511 to 512 lanes, and the wave sizing's search
+    finds the largest number of lanes within a budget, as trying all of them does."""
+    import random
+
+    import model
+    from boa_amd import _native
+
+    lib = _native.load_cdll()
+    c = _native.ModelCfg(d, L, 256, 16, 4, 2, 0)
+    out = ctypes.c_int64(0)
+    need = [0]
+    for lanes in range(1, 1500):
+        assert lib.boa_ctx_plan_bytes(ctypes.byref(c), prec, lanes, tile, ctypes.byref(out)) == 0
+        need.append(out.value)
+    assert all(a < b for i, (a, b) in enumerate(zip(need, need[1:])) if i != 511)
+    rng = random.Random(d + L)
+    for _ in range(300):
+        most, budget = rng.randrange(1, 1500), rng.randrange(need[1], max(need) + 1)
+        assert model._most_lanes(need.__getitem__, most, budget) == max(n for n in range(1, most + 1) if need[n] <= budget)
+    assert model._most_lanes(need.__getitem__, 1400, need[1] - 1) == 1

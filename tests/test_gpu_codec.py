@@ -563,6 +563,39 @@ def test_feed_forward_in_shares(gpu, monkeypatch, precision, n, length):
     assert torch.equal(got[0][2], got[1][2])
 
 
+@pytest.mark.parametrize("d_model,precision,n", [(256, "f32", 3), (512, "bf16w", 20)])
+def test_context_without_room_for_tiles_in_flight(gpu, monkeypatch, d_model, precision, n):
+    """Where a context only fits without the workspace of tiles in flight, it is created without it and gives the same
+    words, bytes and logits; where even that does not fit, creation fails."""
+    import codec
+    import model as M
+    from boa_amd import _native as N
+    from boa_amd import weights as W
+
+    blob = W.seeded_blob(W.Cfg(d_model=d_model, n_layers=4), 3)
+    rng = np.random.default_rng(2)
+    chunks = [rng.integers(0, 256, 300 - i).astype(np.uint8) for i in range(n)]
+    tok = torch.from_numpy(rng.integers(0, 256, (n, 200))).cuda()
+    got = []
+    for short in (0, 1):
+        m = M.BoaConstrictor(d_model, 4, 256).load_blob(blob)
+        m.precision = precision
+        payload, nw, fb, Ls = codec.compress_payload(m, chunks)
+        out = codec.decompress_payload(m, payload, nw, Ls, fb)
+        assert all((out[i, :Ls[i]] == c).all() for i, c in enumerate(chunks))
+        got.append((payload, nw, m.forward(tok).cpu(), m._engines["codec"][1].device_bytes))
+        monkeypatch.setenv("BOA_CTX_MAX_BYTES", str(got[0][3] - 1))
+    assert got[1][3] < got[0][3]
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]) and torch.equal(got[0][2], got[1][2])
+    m = M.BoaConstrictor(d_model, 4, 256).load_blob(blob)
+    m.precision = precision
+    monkeypatch.setenv("BOA_CTX_MAX_BYTES", str(got[1][3] - 1))
+    with pytest.raises(N.BoaError):
+        codec.compress_payload(m, chunks)
+    monkeypatch.setenv("BOA_CTX_MAX_BYTES", str(got[1][3]))
+    assert np.array_equal(codec.compress_payload(m, chunks)[0], got[0][0])
+
+
 @pytest.mark.parametrize("switch", ["BOA_GROUP_STEP", "BOA_FUSED_STEP"])
 def test_decode_switches_leave_compress_alone(gpu, monkeypatch, switch):
     """The switches of the decode kernels change neither the words of a compress of few lanes nor the kernels it takes
