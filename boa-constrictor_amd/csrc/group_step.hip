@@ -377,20 +377,18 @@ __global__ void __launch_bounds__(NTHR, 1) k_group_step(FusedArgs a0) {
                 return __hip_atomic_compare_exchange_strong(gate, &was, how, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return false;
         };
-        // an earlier launch spoilt the state (this one's own waits come after every arrival): all leave
-        const bool spoilt = a0.ctl[CTL_EXPIRED] >= a0.valid_from;
         const uint64_t n = __hip_atomic_fetch_add(a0.ctl + CTL_ARRIVED, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         uint64_t st = state();
         if (n - a0.arrived == total - 1) decide(st, open);
         // if the launch before found no room, other work most likely still has the CUs: a short wait (SHUT_TICKS)
         const uint32_t ticks = (st & 1ull) != 0 && st != shut && a0.gate_ticks > SHUT_TICKS ? SHUT_TICKS : a0.gate_ticks;
         const uint64_t t0 = wall_clock64();
-        while (!spoilt && st != open && st != shut) {
+        while (st != open && st != shut) {
             st = state();
             if (wall_clock64() - t0 > ticks && decide(st, shut))
                 __hip_atomic_fetch_add(a0.ctl + CTL_SHUT_OUT, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        sGo = !spoilt && st == open ? 1 : 0;
+        sGo = st == open ? 1 : 0;
     }
     __syncthreads();
     if (!sGo) return;

@@ -79,9 +79,9 @@ struct FusedArgs {
     // fused kernels: run only if the group launch with this decision word (2 seq0 + 1) did not start (0: always run)
     uint64_t only_if;
 };
-// Control words of a context's group launches: the last decision at the gate (2 seq0: open, 2 seq0 + 1: not all here),
-// arrivals there, launches that were shut out, and the (shut) decision word of the last launch in which a wait expired.
-enum { CTL_GATE, CTL_ARRIVED, CTL_SHUT_OUT, CTL_EXPIRED, CTL_WORDS };
+// Control words of a context's group launches: the last decision at the gate (2 seq0: open, 2 seq0 + 1: not all here), the
+// (shut) decision word of the last launch in which a wait expired, arrivals at the gate, launches that were shut out.
+enum { CTL_GATE, CTL_EXPIRED, CTL_ARRIVED, CTL_SHUT_OUT, CTL_WORDS };
 constexpr uint64_t GATE_NEVER = 1ull << 63;  // `arrived` of a launch whose gate no count of arrivals opens
 
 // Logits of a step that cannot be formed: NaN for every lane (all threads of the grid).
@@ -93,11 +93,13 @@ __device__ __forceinline__ void void_logits(float* logits, int64_t n) {
 // or in an earlier launch since the state was reset (ctl is null where no group launch can have run).
 __device__ __forceinline__ bool left_out(const FusedArgs& a) {
     if (a.ctl == nullptr) return false;
-    if (a.ctl[CTL_EXPIRED] >= a.valid_from) {
+    typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+    const u64x2 ctl = *reinterpret_cast<const u64x2*>(a.ctl);  // both words in one access
+    if (ctl[CTL_EXPIRED] >= a.valid_from) {
         if (a.logits) void_logits(a.logits, (int64_t)a.B * a.V);
         return true;
     }
-    return a.only_if != 0 && a.ctl[CTL_GATE] != a.only_if;
+    return a.only_if != 0 && ctl[CTL_GATE] != a.only_if;
 }
 
 // Launches over several tiles at once (a tile: all lanes of a group at Tc consecutive positions, at one layer).
