@@ -126,8 +126,9 @@ __device__ __forceinline__ void receive(const Link& k, const uint32_t (&at)[N], 
             v[2 * i] = w[i].x;
             v[2 * i + 1] = w[i].z;
         }
+        if (off == 0u) return;
         const uint32_t limit = *k.limit;
-        if (off == 0u || limit == 0u) return;
+        if (limit == 0u) return;
         const uint64_t now = wall_clock64();
         if (t0 == 0) t0 = now;
         if (now - t0 >= limit) {
