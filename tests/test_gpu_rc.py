@@ -167,6 +167,48 @@ def test_decode_tables_arbitrary_words_many_streams(gpu, ora, T, zero):
         assert (out[s] == ora.decode_tables(P, cdf[s], words[s, :nw[s]])).all(), s
 
 
+@pytest.mark.parametrize("T,shift", [(128, 0), (128, 4), (131, 0)])
+@pytest.mark.parametrize("zero", [False, True])
+def test_decode_tables_long_many_streams(gpu, ora, T, shift, zero):
+    """The eight-streams decoder (more than 4096 streams) over many moves of its window of words, whole passes of 8 with
+    word stores (symbols 8-byte aligned) and byte stores (not, or a last pass of 3): encoder words of symbols that cost
+    about 10 bits each, and words that no encoder wrote, of lengths from 0 to 2 T that end before, in and behind the
+    window.  61 tables, each shared by every 61st stream, against the oracle."""
+    from boa_amd import _native as N
+
+    rng = np.random.default_rng(70 + T + shift + zero)
+    S, K, P, U = 4099, 256, 16, 61
+    cdf = ora.xq_cdf(rng.normal(0, 1.5, (U, T, K)).astype(np.float32), P)
+    if zero:
+        cdf = _zero_runs(cdf, rng, P)
+    which = np.arange(S) % U
+    d_cdf = _dev(cdf[..., :K].astype(np.uint16).view(np.int16))[torch.from_numpy(which).cuda()].contiguous()
+    pitch = 2 * T + 8
+    syms = rng.integers(0, K, (U, T))
+    if zero:
+        syms = _sample(cdf, rng, P)
+    enc = [ora.encode_tables(P, cdf[u], syms[u]) for u in range(U)]
+    assert zero or min(len(e) for e in enc) > T // 4  # more than eight bits a symbol
+    coded = np.zeros((S, pitch), dtype=np.uint32)
+    n_coded = np.array([len(enc[u]) for u in which], dtype=np.int32)
+    for s in range(S):
+        coded[s, :n_coded[s]] = enc[which[s]]
+    words = rng.integers(0, 1 << 32, (S, pitch), dtype=np.uint64).astype(np.uint32)
+    nw = rng.integers(0, 2 * T + 1, S).astype(np.int32)
+    nw[::3] = rng.integers(0, T // 4, len(nw[::3]))  # ends inside the stream
+    for w, n, want in ((coded, n_coded, lambda s: syms[which[s]]),
+                       (words, nw, lambda s: ora.decode_tables(P, cdf[which[s]], words[s, :nw[s]]))):
+        d_out = torch.full((S * T + 32,), 171, dtype=torch.uint8, device="cuda")
+        d_w, d_n = _dev(w.view(np.int32)), _dev(n)
+        N.check(gpu.rc_decode_tables(P, 2, N.ptr(d_cdf), K, N.ptr(d_w), pitch, N.ptr(d_n), S, T, d_out.data_ptr() + shift,
+                                     N.stream_ptr()))
+        out = d_out.cpu().numpy()
+        assert (out[:shift] == 171).all() and (out[shift + S * T:] == 171).all()
+        out = out[shift:shift + S * T].reshape(S, T)
+        for s in range(S):
+            assert (out[s] == want(s)).all(), s
+
+
 @pytest.mark.parametrize("S,T", [(1, 8), (7, 16), (33, 8), (1, 4), (9, 12), (65, 4)])
 def test_decode_tables_short_streams(gpu, ora, S, T):
     """The throughput decoder at its smallest shapes: one stream, fewer streams than a wavefront holds, and lengths of
