@@ -916,3 +916,38 @@ def test_step_under_capture(gpu):
             g.replay()
             s.synchronize()
             assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("lanes,length", [(1, 150), (3, 700), (100, 150)])
+def test_forward_under_capture(gpu, lanes, length):
+    """A forward recorded into a graph, with finished tiles' heads on the second stream and with the lanes in two halves
+    on two, replays as the eager forward from the same state, as often as it is replayed, and eager calls go on working
+    between the replays."""
+    from boa_amd import weights as W
+    from model import _Engine
+
+    cfg = W.Cfg(n_layers=8)
+    tok = torch.from_numpy(np.random.default_rng(length).integers(0, 256, (lanes, length)).astype(np.int32)).cuda()
+    out, ref, again = (torch.zeros((lanes, length, 256), device="cuda") for _ in range(3))
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        eng = _Engine(W.seeded_blob(cfg, 1), cfg, lanes, 64, "f32")
+        eng.reset(lanes)
+        eng.forward(tok, ref)
+        eng.reset(lanes)
+        s.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            eng.forward(tok, out)
+        for _ in range(3):
+            eng.reset(lanes)
+            out.zero_()
+            g.replay()
+            s.synchronize()
+            assert torch.equal(out, ref)
+            eng.reset(lanes)
+            again.zero_()
+            eng.forward(tok, again)
+            s.synchronize()
+            assert torch.equal(again, ref)
