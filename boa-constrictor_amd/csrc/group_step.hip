@@ -34,8 +34,8 @@
 // launch, all of them leave, and the fused launch that follows does the work (left_out).  Beyond the gate every wait ends
 // because its partners run.  (A cooperative launch gives the same guarantee but took 80 us longer per launch, of a step's
 // 187.)  The waits are bounded all the same (wait_ticks): if one expires (the process was taken off the GPU for seconds),
-// the workgroup stops waiting for good, goes through the rest of the launch on whatever it holds, and notes the launch in
-// CTL_EXPIRED and for the host.  What the others make of its packets is as void as its own results: the launch that
+// the workgroup stops waiting for good, goes through the rest of the launch on whatever it holds, and notes it in
+// CTL_EXPIRED and, with the launch, for the host.  What the others make of its packets is as void as its own results: the launch that
 // follows sees the note and sets all logits to NaN, as do all steps until the state is reset, and the host refuses the
 // next call.  With more groups than CUs / 2 the fused kernels, one workgroup per group, fill the GPU and have no exchange.
 //
@@ -133,10 +133,9 @@ __device__ __forceinline__ void receive(const Link& k, const uint32_t (&at)[N], 
         if (t0 == 0) t0 = now;
         if (now - t0 >= limit) {
             KArgs& a = kargs();
-            const uint64_t launch = 2ull * a.seq0 + 1ull;
             *k.limit = 0u;
-            __hip_atomic_store(a.ctl + CTL_EXPIRED, launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(a.host_expired, launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(a.ctl + CTL_EXPIRED, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(a.host_expired, 2ull * a.seq0 + 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             return;
         }
     }

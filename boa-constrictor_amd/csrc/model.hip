@@ -2553,9 +2553,10 @@ __global__ void __launch_bounds__(256) k_encode_lf(const uint2* __restrict__ lf,
 }
 
 // Zeroes the recurrent state of lanes [0, lanes) of every layer (blockIdx.y: conv history rows of nh floats, state rows
-// of ns floats per lane), in one launch and without memset nodes.
+// of ns floats per lane) and the note of an expired wait (expired; null: it stays), in one launch and without memset nodes.
 __global__ void __launch_bounds__(256) k_state_zero(float* __restrict__ hist, int64_t nh, float* __restrict__ ssm,
-                                                   int64_t ns, int lanes, int64_t max_lanes) {
+                                                   int64_t ns, int lanes, int64_t max_lanes, uint64_t* expired) {
+    if (expired && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *expired = 0;
     const int64_t l = blockIdx.y, stride = (int64_t)gridDim.x * blockDim.x * 4;
     const int64_t i0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -2564,9 +2565,8 @@ __global__ void __launch_bounds__(256) k_state_zero(float* __restrict__ hist, in
 }
 
 // Logits of a forward that continued a state which an expired wait had spoilt (left_out's test): NaN.
-__global__ void __launch_bounds__(256) k_void_logits(float* __restrict__ logits, int64_t n, const uint64_t* __restrict__ expired,
-                                                    uint64_t valid_from) {
-    if (*expired >= valid_from) void_logits(logits, n);
+__global__ void __launch_bounds__(256) k_void_logits(float* __restrict__ logits, int64_t n, const uint64_t* __restrict__ expired) {
+    if (*expired != 0) void_logits(logits, n);
 }
 
 __global__ void k_enc_finish(EncState* states, uint32_t* words, int64_t pitch, int32_t* nwords, int32_t* overflow,
@@ -2727,8 +2727,8 @@ struct boa_ctx {
     uint64_t* xctl = nullptr;          // control words (CTL_*)
     uint64_t xarrived = 0;             // arrivals at the gate so far
     uint64_t xseq = 1;                 // the next launch's first sequence number
-    // an expired wait: the launch it was in (pinned host memory, 0: none), the first launch since the state was reset, the
-    // lanes whose state has gone through group launches since then, and whether group launches are given up
+    // an expired wait: the launch it was in (pinned host memory, 0: none), the first launch since the state was reset (as
+    // decision words), the lanes whose state has gone through group launches since then, and whether those are given up
     uint64_t* xexpired = nullptr;
     uint64_t valid_from = 2;
     int grouped = 0;
@@ -3294,7 +3294,8 @@ extern "C" int boa_state_reset(boa_ctx* x, int32_t lanes) {
     if (!x || lanes < 0 || lanes > x->max_lanes) return boa_fail(BOA_ERR_ARG, "boa_state_reset: bad lanes");
     x->pos = 0;
     (void)wait_expired(x);
-    if (lanes >= x->grouped) {
+    const bool all = lanes >= x->grouped;
+    if (all) {
         x->valid_from = 2ull * x->xseq;
         x->grouped = 0;
     }
@@ -3303,7 +3304,8 @@ extern "C" int boa_state_reset(boa_ctx* x, int32_t lanes) {
     const int64_t ns = (int64_t)x->di * x->NS;
     const unsigned blocks = (unsigned)std::min<int64_t>((lanes * ns / 4 + 255) / 256, 1024);
     hipLaunchKernelGGL(k_state_zero, dim3(blocks, (unsigned)x->L), dim3(256), 0, x->stream, x->conv_hist,
-                       (int64_t)3 * x->di, x->ssm, ns, lanes, (int64_t)x->max_lanes);
+                       (int64_t)3 * x->di, x->ssm, ns, lanes, (int64_t)x->max_lanes,
+                       all && x->xctl ? x->xctl + CTL_EXPIRED : nullptr);
     BOA_HIP_TRY(hipGetLastError());
     return BOA_OK;
 }
@@ -3763,9 +3765,9 @@ static FusedArgs fused_args(boa_ctx* x, int32_t lanes, const int32_t* tokens_in)
 
 static hipError_t launch_fused(boa_ctx* x, FusedArgs& a, hipStream_t s) {
     const int nt = x->prec == BOA_PREC_BF16X3 ? 3 : (x->prec == BOA_PREC_BF16W ? 2 : 1);
+    a.ctl = x->xctl;
     // a stream that is being captured takes the fused kernel: replays would repeat the sequence numbers
     if (x->xch && !x->group_off && !capturing(s)) {
-        a.ctl = x->xctl; a.valid_from = x->valid_from;
         const int g = group_step_width(x->d, a.B, x->cus);
         if (g > 1) {
             const uint32_t seqs = group_step_seqs(a.nsteps, x->L);
@@ -4095,10 +4097,10 @@ extern "C" int boa_model_forward(boa_ctx* x, const int32_t* d_tokens, int64_t to
         return boa_fail(BOA_ERR_ARG, "boa_model_forward: bad arguments");
     if (wait_expired(x)) return fail_expired("boa_model_forward");
     const int rc = forward(x, d_tokens, tok_stride, lanes, len, d_logits);
-    if (rc || len == 0 || !x->grouped || capturing(x->stream)) return rc;
+    if (rc || len == 0 || !x->grouped) return rc;
     // the state came through group launches that the host has not heard from yet
     hipLaunchKernelGGL(k_void_logits, dim3(256), dim3(256), 0, x->stream, d_logits, (int64_t)lanes * len * x->V,
-                       x->xctl + CTL_EXPIRED, x->valid_from);
+                       x->xctl + CTL_EXPIRED);
     BOA_HIP_TRY(hipGetLastError());
     return BOA_OK;
 }

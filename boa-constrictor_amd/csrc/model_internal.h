@@ -74,13 +74,11 @@ struct FusedArgs {
     uint32_t gate_ticks;
     uint32_t wait_ticks;
     uint64_t* host_expired;
-    // an expired wait of a launch from this one on (a decision word) has spoilt the state that this launch continues
-    uint64_t valid_from;
     // fused kernels: run only if the group launch with this decision word (2 seq0 + 1) did not start (0: always run)
     uint64_t only_if;
 };
-// Control words of a context's group launches: the last decision at the gate (2 seq0: open, 2 seq0 + 1: not all here), the
-// (shut) decision word of the last launch in which a wait expired, arrivals at the gate, launches that were shut out.
+// Control words of a context's group launches: the last decision at the gate (2 seq0: open, 2 seq0 + 1: not all here),
+// whether a wait expired since the state was reset (0: none did), arrivals at the gate, launches that were shut out.
 enum { CTL_GATE, CTL_EXPIRED, CTL_ARRIVED, CTL_SHUT_OUT, CTL_WORDS };
 constexpr uint64_t GATE_NEVER = 1ull << 63;  // `arrived` of a launch whose gate no count of arrivals opens
 
@@ -90,12 +88,12 @@ __device__ __forceinline__ void void_logits(float* logits, int64_t n) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) logits[i] = nan;
 }
 // Whether a fused launch is left out: it follows a group launch that did run, or a wait between workgroups expired in it
-// or in an earlier launch since the state was reset (ctl is null where no group launch can have run).
+// or in an earlier launch since the state was reset (ctl is null in contexts without group launches).
 __device__ __forceinline__ bool left_out(const FusedArgs& a) {
     if (a.ctl == nullptr) return false;
     typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
     const u64x2 ctl = *reinterpret_cast<const u64x2*>(a.ctl);  // both words in one access
-    if (ctl[CTL_EXPIRED] >= a.valid_from) {
+    if (ctl[CTL_EXPIRED] != 0) {
         if (a.logits) void_logits(a.logits, (int64_t)a.B * a.V);
         return true;
     }

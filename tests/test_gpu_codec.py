@@ -763,6 +763,24 @@ def test_expired_wait_is_reported(gpu, monkeypatch, d_model, precision, n):
         eng.reset(n)
         eng.step(first, out)
         assert torch.equal(out, ref)
+    # a step recorded into a graph, which no call of the host's is behind
+    st = torch.cuda.Stream()
+    with torch.cuda.stream(st):
+        eng = _Engine(blob, cfg, n, 20, precision)
+        eng.reset(n)
+        st.synchronize()
+        g, rec = torch.cuda.CUDAGraph(), torch.zeros_like(out)
+        with torch.cuda.graph(g, stream=st):
+            eng.step(first, rec)
+        eng.step(first, out)
+        g.replay()
+        st.synchronize()
+        assert out.isnan().all() and rec.isnan().all()
+        for _ in range(2):
+            eng.reset(n)
+            g.replay()
+            st.synchronize()
+            assert torch.equal(rec, ref)
     # steps enqueued behind the expired one, and a reset before the host knows
     eng = _Engine(blob, cfg, n, 20, precision)
     eng.reset(n)
