@@ -52,27 +52,27 @@ TRAFFIC_FILES = {p: os.path.join(REPO, "profiles", f"traffic_fused_step_{p}_d256
 CODER_TRAFFIC_FILE = os.path.join(REPO, "profiles", "traffic_rc_coder_configs1.json")
 
 # rocprof names of the kernel instances each profiled class launches at the benchmark's shapes, per precision
-# (k_gemm_bf<BM, BN, BK, EPI, NT, A split, C split>: EPI 0 none, 1 bias, 2 GELU, 4 residual; k_ffn<NT, true>:
-# out_proj + LN2 + FF1 + GELU + FF2 + residual in one kernel; k_mixin<NT>: LN1 + in_proj + conv + x_proj;
+# (k_gemm_bf<BM, BN, BK, EPI, NT, A split, C split>: EPI 0 none, 1 bias, 2 GELU, 4 residual; k_ffn<NT, true, ..>:
+# out_proj + LN2 + FF1 + GELU + FF2 + residual in one kernel; k_mixin<NT, ..>: LN1 + in_proj + conv + x_proj;
 # k_head_xq: head + quantiser; NT = 1 is the fp32 form, 3 the bf16x3 form)
 KERNEL_NAMES = {
     "f32": {
-        ("compress", "ffn"): "k_ffn<1, true>",
-        ("compress", "mixin"): "k_mixin<1>",
+        ("compress", "ffn"): "k_ffn<1, true, FfnTile>",
+        ("compress", "mixin"): "k_mixin<1, MixinOne<false>>",
         ("compress", "scan"): "k_scan<16, 16, false>",
-        ("compress", "head_xq"): "k_head_xq<1, 256>",
+        ("compress", "head_xq"): "k_head_xq<1, 256, false>",
         ("compress", "encode"): "k_encode_lf",
         ("decompress", "fused_step"): "k_fused_step<1, 512>",
     },
     "bf16x3": {
         ("compress", "gemm_in_proj"): "k_gemm_bf<128, 128, 32, 1, 3, true, false>",
-        ("compress", "ffn"): "k_ffn<3, true>",
-        ("compress", "mixin"): "k_mixin<3>",
+        ("compress", "ffn"): "k_ffn<3, true, FfnTile>",
+        ("compress", "mixin"): "k_mixin<3, MixinOne<false>>",
         ("compress", "gemm_out_proj"): "k_gemm_bf<128, 128, 32, 1, 3, true, false>",
         ("compress", "gemm_x_proj"): "k_xproj<3, 3>",
         ("compress", "scan"): "k_scan<16, 16, true>",
         ("compress", "conv"): "k_conv_silu",
-        ("compress", "head_xq"): "k_head_xq<3, 256>",
+        ("compress", "head_xq"): "k_head_xq<3, 256, false>",
         ("compress", "encode"): "k_encode_lf",
         ("decompress", "fused_step"): "k_fused_step<3, 512>",
     },

@@ -16,12 +16,16 @@
 // weights of the next GEMM (held in registers), conv history, SSM state and parameters; and with few rows per thread the
 // state is stored only after the next exchange has arrived.
 //
-// us per step, fused kernel -> this one (G):
-//   d 256 x 8, fp32:    1 lane 592 -> 186 (8), 64: 670 -> 223 (8), 512: 671 -> 238 (8), 1000: 675 -> 315 (4), 2048: 695 -> 514 (2)
-//   d 256 x 8, bf16x3:  64: 494 -> 174 (8), 1000: 483 -> 268 (4), 2048: 505 -> 430 (2)
-//   d 512 x 16, bf16w:  1: 2941 -> 346 (16), 256: 3730 -> 521 (16), 1000: 3785 -> 1016 (4), 2048: 4033 -> 1933 (2)
-// What remains at 64 lanes (fp32, of 228): the GEMMs' dependent MFMA chains 75 (FF2 32: 256 dependent MFMAs per output),
-// the five waits with LayerNorms and operand stores 117, the rest scan, conv and requests.
+// us per boa_model_step, fused kernel -> this one (G) and the fused launch behind it that leaves at once:
+//   d 256 x 8, fp32:    1 lane 597 -> 190 (8), 64: 668 -> 227 (8), 512: 684 -> 249 (8), 1000: 703 -> 332 (4), 2048: 731 -> 528 (2)
+//   d 256 x 8, bf16x3:  1: 429 -> 137 (8), 64: 493 -> 176 (8), 512: 497 -> 202 (8), 1000: 501 -> 276 (4), 2048: 526 -> 456 (2)
+//   d 512 x 16, bf16w:  1: 2924 -> 353 (16), 256: 3713 -> 526 (16), 1000: 3813 -> 990 (4), 2048: 4074 -> 1838 (2)
+//   d 512 x 16, bf16x3: 1: 3860 -> 411 (16), 256: 4633 -> 627 (16), 1000: 4590 -> 1548 (4), 2048: 5118 -> 3496 (2)
+// What remains at 64 lanes (fp32, 8 launches of 125 steps, hardware counters): the matrix cores of the 32 CUs are busy 50
+// of a step's 225 us, in chains of dependent MFMAs (256 per FF2 output), and the waves wait 48% of their cycles: for
+// packets, at barriers, for their own loads.
+// Registers: every form spills 70 to 113 scalar registers to vector lanes.  At d_model 512 with G = 2, where a member
+// holds most, vector registers go to scratch memory too: bf16w 67, bf16x3 188.
 //
 // A packet is rewritten only by the same exchange of the next layer (or step), and its writer gets there only after
 // every member has sent its packets of a later exchange of this layer, which it does after reading this one (a barrier
@@ -35,9 +39,10 @@
 // because its partners run.  (A cooperative launch gives the same guarantee but took 80 us longer per launch, of a step's
 // 187.)  The waits are bounded all the same (wait_ticks): if one expires (the process was taken off the GPU for seconds),
 // the workgroup stops waiting for good, goes through the rest of the launch on whatever it holds, and notes it in
-// CTL_EXPIRED and, with the launch, for the host.  What the others make of its packets is as void as its own results: the launch that
-// follows sees the note and sets all logits to NaN, as do all steps until the state is reset, and the host refuses the
-// next call.  With more groups than CUs / 2 the fused kernels, one workgroup per group, fill the GPU and have no exchange.
+// CTL_EXPIRED and, with the launch, for the host.  What the others make of its packets is as void as its own results: the
+// launch that follows sees the note and sets all logits to NaN, as do all steps until the state is reset, and the host
+// refuses the next call.  With more groups than CUs / 2 the fused kernels, one workgroup per group, fill the GPU and have
+// no exchange.
 //
 // Arithmetic: every GEMM output accumulates its K steps in ascending order through mfma_split_step_t, x_proj is the left
 // fold of 64-channel partials, and every elementwise step is the shared function of model_dev.h, as in the fused and
@@ -57,7 +62,7 @@ namespace {
 
 constexpr int ROWS = 16, NTHR = 512, NWAVE = 8, NS = 16, VV = 256;
 // Wait at the gate, in 10 ns, of a launch behind one that was shut out.  With room, the last of a launch's workgroups is
-// there about 3 us after the first (up to 256 workgroups, 1200 launches: 5 us passed in 3%, 10 us in none).  With the whole
+// there about 3 us after the first (up to 256 workgroups, 1200 launches: 5 us passed in 45, 10 us in none).  With the whole
 // wait (0.5 ms and more) every step of a context beside other work paid it.
 constexpr uint32_t SHUT_TICKS = 2000;
 typedef uint64_t Packet;
