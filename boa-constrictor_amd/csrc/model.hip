@@ -4297,7 +4297,8 @@ extern "C" int boa_decompress(boa_ctx* x, const uint32_t* d_payload, int64_t pay
         lanes < 1 || lanes > x->max_lanes || max_len < 1 || out_stride < max_len)
         return boa_fail(BOA_ERR_ARG, "boa_decompress: bad arguments");
     hipStream_t s = x->stream;
-    int rc = boa_state_reset(x, lanes);
+    // after an expired wait the state of all lanes concerned is void: one decode leaves none of it
+    int rc = boa_state_reset(x, wait_expired(x) ? std::max<int32_t>(lanes, x->grouped) : lanes);
     if (rc) return rc;
     hipLaunchKernelGGL(k_dec_init, dim3((lanes + 255) / 256), dim3(256), 0, s, x->dec, d_payload, payload_words,
                        d_word_off, d_nwords, d_first, d_lens, x->tokens, d_out, out_stride, lanes);
