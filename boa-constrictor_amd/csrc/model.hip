@@ -3850,15 +3850,15 @@ extern "C" int boa_model_step(boa_ctx* x, const int32_t* d_tokens, int32_t lanes
 // xin) handles a tile that has passed the last layer.
 // Where the lines lie (compress, ms; d 256 x 8 layers over 704 positions, d 512 x 16 layers bf16w over 320):
 //   PIPE_LANES: against tile after tile on two streams, which from 512 lanes on fills the GPU by itself.  fp32 64 lanes
-//     29.0 -> 8.4, 256: 30.6 -> 26.3, 375: 50.2 -> 39.4, 512: 50.1 -> 50.5; bf16x3 375: 23.6 -> 21.1, 512: 26.4 -> 28.4;
-//     d 512 64: 21.3 -> 8.6, 256: 29.5 -> 28.3, 375: 49.7 -> 40.1, 512: 54.0 -> 53.6.
+//     28.5 -> 8.3, 256: 30.2 -> 25.9, 375: 49.7 -> 38.8, 511: 51.4 -> 50.1; bf16x3 64: 14.4 -> 5.0, 256: 17.2 -> 14.3, 375:
+//     24.1 -> 20.2, 511: 27.2 -> 26.8; d 512 64: 21.1 -> 8.8, 256: 30.8 -> 28.6, 375: 51.4 -> 41.2, 511: 59.5 -> 55.4.
 //   PIPE_SPLIT: (lane, tile) pairs in a step up to which mixer input and scan are cut finer (1 lane fp32: 4.40 -> 1.96;
 //     16 lanes 5.12 -> 3.31; from 256 pairs on no difference), pipe_quad: up to which the scan is (at d 256 faster or
 //     the same up to 512 pairs; at d 512, whose dt_proj rows are twice as long, 10% slower at 512).
 //   PIPE_ROWS16: 64-row groups in a step up to which feed-forward and head run on 16-row workgroups (16 lanes fp32, 128
 //     groups: 4.02 -> 3.31; more 16-row workgroups than CUs stream the weights more often than they gain).
-//   pipe_two: pairs in flight from which the lanes run as two halves on two streams (fp32 100 lanes 13.2 -> 12.7, 180:
-//     22.3 -> 20.1; 8 lanes 2.37 -> 2.85; d 512 8 lanes 4.09 -> 3.88, 64: 10.2 -> 8.6).
+//   pipe_two: pairs in flight from which the lanes run as two halves on two streams (fp32 100 lanes 13.2 -> 12.5, 180:
+//     21.1 -> 19.6; 8 lanes, where it would begin otherwise, 2.37 -> 2.85; d 512 8 lanes 4.07 -> 3.89, 64: 10.6 -> 8.9).
 constexpr int PIPE_SPLIT = 128, PIPE_ROWS16 = 128;
 static int pipe_quad(const boa_ctx* x) { return x->d == ffn5::D ? 128 : 512; }
 static int pipe_two(const boa_ctx* x) { return x->d == ffn5::D ? 64 : 640; }
